@@ -175,7 +175,8 @@ struct pa_problem {
   double box_lo[3] = {0, 0, 0}, box_len[3] = {0, 0, 0};
   std::vector<int32_t> box_grid;  // (i, j, k) per node, host
   std::vector<std::unique_ptr<MgLevel>> mg;
-  DevArray<double> mg_Ainv;
+  DevArray<double> mg_Ainv, mg_T;
+  DevArray<double> mg_lz;  // spectral estimates: partials of each level, coefficients, pivot flag
   // Smoothing (measured at 128x64x64 and 256x128x128): on level 0 one damped block-Jacobi
   // step before and after the coarse correction (Chebyshev degree 1: 52-54 iterations at
   // 3 operator applications each beat degree 2's 48 at 5; unequal degrees break the
@@ -1740,6 +1741,8 @@ static int mg_build(pa_handle h) {
   if (h->mg.size() < 2) return fail(PA_ERR_UNSUPPORTED, "multigrid: the box has no coarser level");
   const size_t nc = 3 * (size_t)h->mg.back()->nn;
   PA_HIP(h->mg_Ainv.alloc(nc * nc));
+  PA_HIP(h->mg_T.alloc(nc * nc));
+  PA_HIP(h->mg_lz.alloc((h->mg.size() - 1) * (3 * (size_t)pa::kLzBlocks + 2 * pa::kLzSteps) + 1));
   return PA_OK;
 }
 
@@ -1906,49 +1909,6 @@ static bool mg_trace() {
   return on;
 }
 
-// Inverse of a symmetric positive definite n x n matrix (row major, in place in A;
-// U is n x n scratch): Cholesky A = L L^T into the lower triangle, U = L^-T (upper),
-// A^-1 = U U^T.  Every inner loop runs along contiguous rows.
-static int spd_inverse(std::vector<double>& A, std::vector<double>& U, int n) {
-  for (int j = 0; j < n; ++j) {
-    double* Aj = &A[(size_t)j * n];
-    double d = Aj[j];
-    for (int k = 0; k < j; ++k) d -= Aj[k] * Aj[k];
-    if (!(d > 0.0)) return fail(PA_ERR_NOT_CONVERGED, "multigrid: coarsest operator is not positive definite");
-    const double ljj = std::sqrt(d), inv = 1.0 / ljj;
-    Aj[j] = ljj;
-    for (int i = j + 1; i < n; ++i) {
-      double* Ai = &A[(size_t)i * n];
-      double t = Ai[j];
-      for (int k = 0; k < j; ++k) t -= Ai[k] * Aj[k];
-      Ai[j] = t * inv;
-    }
-  }
-  // row j of U holds column j of L^-1: U[j][i] = (L^-1)[i][j], i >= j
-  for (int j = 0; j < n; ++j) {
-    double* Uj = &U[(size_t)j * n];
-    Uj[j] = 1.0 / A[(size_t)j * n + j];
-    for (int i = j + 1; i < n; ++i) {
-      const double* Li = &A[(size_t)i * n];
-      double t = 0.0;
-      for (int k = j; k < i; ++k) t += Li[k] * Uj[k];
-      Uj[i] = -t / Li[i];
-    }
-  }
-  // A^-1[i][j] = sum_{k >= max(i, j)} (L^-1)[k][i] (L^-1)[k][j] = sum_k U[i][k] U[j][k]
-  for (int i = 0; i < n; ++i) {
-    const double* Ui = &U[(size_t)i * n];
-    for (int j = i; j < n; ++j) {
-      const double* Uj = &U[(size_t)j * n];
-      double t = 0.0;
-      for (int k = j; k < n; ++k) t += Ui[k] * Uj[k];
-      A[(size_t)i * n + j] = t;
-      A[(size_t)j * n + i] = t;
-    }
-  }
-  return PA_OK;
-}
-
 // Chebyshev coefficients of level L for the interval [lmax / ratio, lmax].
 static void mg_set_interval(pa_handle h, MgLevel& L, double lmax) {
   const double lmin = lmax / h->mg_ratio;
@@ -1989,49 +1949,25 @@ static double tridiag_max_eig(const std::vector<double>& a, const std::vector<do
   return hi;
 }
 
-// lambda_max(D^-1 K) of level l from below: the largest Ritz value of kLanczosSteps steps
+// lambda_max(D^-1 K) of a level from below: the largest Ritz value of kLzSteps steps
 // of block-Jacobi PCG on K x = v (v a fixed pseudo-random vector), whose coefficients give
 // the Lanczos tridiagonal T_jj = 1/alpha_j + beta_{j-1}/alpha_{j-1},
 // T_j,j+1 = sqrt(beta_j)/alpha_j (Saad, Iterative Methods for Sparse Linear Systems, 6.7.3).
 // Power iteration from the same start converges too slowly on high-contrast SIMP designs,
 // whose top eigenvectors sit on a few solid/void interfaces (a 12-step power estimate of
 // 2.13 against a true 2.63 made the smoother divergent there).
-static int mg_lambda_max(pa_handle h, size_t l, const double* vals0, bool mixed, double* lam) {
-  constexpr int kLanczosSteps = 16;
-  hipStream_t s = h->stream;
-  MgLevel& L = *h->mg[l];
-  const size_t nd = 3 * (size_t)L.nn;
-  const double* dinv = mg_dinv(h, l, mixed);
-  double *r = L.r.p, *z = L.y.p, *p = L.pw.p, *q = L.t.p;
-  std::vector<double> v0(nd);
-  for (size_t i = 0; i < nd; ++i) v0[i] = (double)((i * 2654435761ull >> 7) % 2001) / 1000.0 - 1.0;
-  PA_HIP(hipMemcpyAsync(r, v0.data(), nd * sizeof(double), hipMemcpyHostToDevice, s));
-  PA_HIP(pa::launch_dinv_apply(z, dinv, r, L.nn, s));
-  PA_HIP(hipMemcpyAsync(p, z, nd * sizeof(double), hipMemcpyDeviceToDevice, s));
-  double rz = 0.0;
-  if (int rc = mg_dot(h, r, z, nd, pa::kDot0, &rz)) return rc;
-  std::vector<double> alpha, beta, ta, tb;
-  const double rz0 = rz;
-  for (int j = 0; j < kLanczosSteps && rz > 1e-28 * rz0; ++j) {
-    if (int rc = mg_apply(h, l, p, q, vals0, mixed)) return rc;
-    double pq = 0.0;
-    if (int rc = mg_dot(h, p, q, nd, pa::kDot0, &pq)) return rc;
-    if (!(pq > 0.0) || !std::isfinite(pq)) break;
+// coef: rz_j = coef[2j], pq_j = coef[2j + 1]; the steps after a breakdown are ignored.
+static int mg_lambda_max(const double* coef, double* lam) {
+  std::vector<double> ta, tb;
+  double a_prev = 0.0, b_prev = 0.0;
+  for (int j = 0; j < pa::kLzSteps; ++j) {
+    const double rz = coef[2 * j], pq = coef[2 * j + 1];
+    if (!(rz > 1e-28 * coef[0]) || !(pq > 0.0) || !std::isfinite(pq)) break;
+    if (j > 0) b_prev = rz / coef[2 * j - 2];
     const double a = rz / pq;
-    const size_t g = grid_for(nd);
-    pa::k_axpy<<<g, 256, 0, s>>>(r, q, nd, -a);
-    PA_HIP(pa::launch_dinv_apply(z, dinv, r, L.nn, s));
-    double rz1 = 0.0;
-    if (int rc = mg_dot(h, r, z, nd, pa::kDot0, &rz1)) return rc;
-    const double b = rz1 / rz;
-    ta.push_back(1.0 / a + (j > 0 ? beta.back() / alpha.back() : 0.0));
-    if (j > 0) tb.push_back(std::sqrt(beta.back()) / alpha.back());
-    alpha.push_back(a);
-    beta.push_back(b);
-    pa::k_scale<<<g, 256, 0, s>>>(p, nd, b);
-    pa::k_axpy<<<g, 256, 0, s>>>(p, z, nd, 1.0);
-    PA_HIP(hipGetLastError());
-    rz = rz1;
+    ta.push_back(1.0 / a + (j > 0 ? b_prev / a_prev : 0.0));
+    if (j > 0) tb.push_back(std::sqrt(b_prev) / a_prev);
+    a_prev = a;
   }
   if (ta.empty()) return fail(PA_ERR_NOT_CONVERGED, "multigrid: bad spectral estimate");
   *lam = tridiag_max_eig(ta, tb);
@@ -2059,30 +1995,52 @@ static int mg_setup(pa_handle h, const double* z, const double* vals0, bool mixe
     }
   }
   // Chebyshev interval [lmax / ratio, lmax], lmax = 1.1 x the largest Ritz value of D^-1 K
-  // per smoothed level
-  for (size_t l = 0; l + 1 < nl; ++l) {
+  // per smoothed level, and the coarsest level's inverse; read back together
+  const size_t per = 2 * pa::kLzSteps, npart = 3 * (size_t)pa::kLzBlocks, ns = nl - 1;
+  double* coef = h->mg_lz.p + ns * npart;  // then the inverse's pivot flag
+  pa::LzArgs lz{};
+  for (size_t l = 0; l < ns; ++l) {
+    MgLevel& L = *h->mg[l];
+    pa::LzLevel& e = lz.L[l];
+    e.vals = l > 0 ? L.vals.p : (mixed ? nullptr : vals0);
+    e.rowmap = L.h->rowmap.p;
+    e.col = L.h->colidx.p;
+    e.dinv = mg_dinv(h, l, mixed);
+    e.r = L.r.p;
+    e.z = L.y.p;
+    e.p = L.pw.p;
+    e.q = L.t.p;
+    e.P = h->mg_lz.p + l * npart;
+    e.coef = coef + l * per;
+    e.nn = L.nn;
+    e.b0 = lz.blocks;
+    e.nb = std::min(pa::kLzBlocks, std::max(1, (L.nn + 15) / 16));
+    lz.blocks += e.nb;
+  }
+  lz.nlev = (int)ns;
+  PA_HIP(pa::launch_lz_init(lz, s));
+  for (int j = 0; j < pa::kLzSteps; ++j) {
+    if (mixed)
+      if (int rc = mg_apply(h, 0, lz.L[0].p, lz.L[0].q, vals0, true)) return rc;
+    PA_HIP(pa::launch_lz_spmv(lz, s));
+    PA_HIP(pa::launch_lz_update(lz, j, s));
+    if (j + 1 < pa::kLzSteps) PA_HIP(pa::launch_lz_dir(lz, j, s));
+  }
+  MgLevel& Lc = *h->mg.back();
+  PA_HIP(pa::launch_mg_dense_inverse(Lc.vals.p, Lc.h->rowmap.p, Lc.h->colidx.p, Lc.nn, h->mg_Ainv.p, h->mg_T.p,
+                                     coef + ns * per, s));
+  std::vector<double> hc(ns * per + 1);
+  PA_HIP(hipMemcpyAsync(hc.data(), coef, hc.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+  PA_HIP(hipStreamSynchronize(s));
+  if (hc.back() != 0.0) return fail(PA_ERR_NOT_CONVERGED, "multigrid: coarsest operator is not positive definite");
+  for (size_t l = 0; l < ns; ++l) {
     MgLevel& L = *h->mg[l];
     double lam = 0.0;
-    if (int rc = mg_lambda_max(h, l, vals0, mixed, &lam)) return rc;
+    if (int rc = mg_lambda_max(&hc[l * per], &lam)) return rc;
     L.lam = lam;
     if (mg_trace()) std::fprintf(stderr, "mg level %zu: %d nodes, lambda_max(D^-1 K) ~ %.6g\n", l, L.nn, lam);
     mg_set_interval(h, L, 1.1 * lam);
   }
-  // coarsest level: dense inverse on the host (a few hundred dofs)
-  MgLevel& Lc = *h->mg.back();
-  const int nc = 3 * Lc.nn;
-  const pa::Graph& g = Lc.h->graph;
-  std::vector<double> v(9 * (size_t)g.rowmap[Lc.nn]);
-  PA_HIP(hipMemcpyAsync(v.data(), Lc.vals.p, v.size() * sizeof(double), hipMemcpyDeviceToHost, s));
-  PA_HIP(hipStreamSynchronize(s));
-  std::vector<double> A((size_t)nc * nc, 0.0), U((size_t)nc * nc, 0.0);
-  for (int r = 0; r < Lc.nn; ++r)
-    for (int k = g.rowmap[r]; k < g.rowmap[r + 1]; ++k)
-      for (int i = 0; i < 3; ++i)
-        for (int j = 0; j < 3; ++j) A[(size_t)(3 * r + i) * nc + 3 * g.colidx[k] + j] = v[9 * (size_t)k + 3 * i + j];
-  if (int rc = spd_inverse(A, U, nc)) return rc;
-  PA_HIP(hipMemcpyAsync(h->mg_Ainv.p, A.data(), A.size() * sizeof(double), hipMemcpyHostToDevice, s));
-  PA_HIP(hipStreamSynchronize(s));
   return PA_OK;
 }
 

@@ -185,19 +185,6 @@ __global__ __launch_bounds__(kT) void k_add2(double* out, const double* a, const
   for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n; i += (size_t)gridDim.x * kT) out[i] = a[i] + b[i];
 }
 
-__global__ __launch_bounds__(kT) void k_dinv_apply(double* __restrict__ y, const double* __restrict__ dinv,
-                                                   const double* __restrict__ x, int nn) {
-  for (int n = blockIdx.x * kT + threadIdx.x; n < nn; n += gridDim.x * kT) {
-    const size_t o = 3 * (size_t)n;
-    const double xv[3] = {x[o], x[o + 1], x[o + 2]};
-    double zv[3];
-    dinv3(dinv + 9 * (size_t)n, xv, zv);
-    y[o] = zv[0];
-    y[o + 1] = zv[1];
-    y[o + 2] = zv[2];
-  }
-}
-
 // one wavefront per row, fixed-order lane sums
 __global__ __launch_bounds__(kT) void k_dense_gemv(const double* __restrict__ A, const double* __restrict__ x,
                                                    double* __restrict__ y, int n) {
@@ -292,10 +279,190 @@ __global__ __launch_bounds__(kT) void k_to_f32(const double* __restrict__ a, flo
   for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n; i += (size_t)gridDim.x * kT) b[i] = (float)a[i];
 }
 
-__global__ __launch_bounds__(kT) void k_scale_rsqrt(double* __restrict__ y, size_t n, const double* __restrict__ scal,
-                                                    int slot) {
-  const double f = 1.0 / sqrt(scal[slot]);
-  for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n; i += (size_t)gridDim.x * kT) y[i] *= f;
+// Spectral estimates (pa_mg.hpp).  What the host-driven form cost at 128x64x64 was the
+// host: 16 steps x 5 levels x 2 dot products read back (160 round trips of ~20 us), plus a
+// 13 MB start vector built and copied from the host; the kernels' own work is ~1 ms.
+// So the scalars stay on the device (each consumer sums the level's partials itself, as in
+// the PCG kernels) and one launch serves all levels: the coarse ones are a few work-groups
+// each and would be launch-bound alone.
+__device__ __forceinline__ int lz_level(const LzArgs& A) {
+  int l = 0;
+  while (l + 1 < A.nlev && (int)blockIdx.x >= A.L[l + 1].b0) ++l;
+  return l;
+}
+
+__global__ __launch_bounds__(kT) void k_lz_init(LzArgs A) {
+  __shared__ double sh[kT / 64];
+  const LzLevel& L = A.L[lz_level(A)];
+  const int b = blockIdx.x - L.b0;
+  double rz = 0.0;
+  for (int n = b * kT + threadIdx.x; n < L.nn; n += L.nb * kT) {
+    const size_t o = 3 * (size_t)n;
+    double v[3], z[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] = (double)(((unsigned long long)(o + i) * 2654435761ull >> 7) % 2001) / 1000.0 - 1.0;
+    dinv3(L.dinv + 9 * (size_t)n, v, z);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      L.r[o + i] = v[i];
+      L.z[o + i] = z[i];
+      L.p[o + i] = z[i];
+      rz += v[i] * z[i];
+    }
+  }
+  const double t = block_reduce_all<kT>(rz, sh);
+  if (threadIdx.x == 0) L.P[kLzBlocks + b] = t;
+}
+
+__global__ __launch_bounds__(kT) void k_lz_spmv(LzArgs A) {
+  __shared__ double sh[kT / 64];
+  const LzLevel& L = A.L[lz_level(A)];
+  const int b = blockIdx.x - L.b0;
+  double dot = 0.0;
+  if (L.vals) {
+    constexpr int kRows = kT / kLanesPerRow;
+    const int lane = threadIdx.x % kLanesPerRow;
+    const double* __restrict__ p = L.p;
+    auto X = [&](int c, int j) { return p[3 * (size_t)c + j]; };
+    for (int row = b * kRows + threadIdx.x / kLanesPerRow; row < L.nn; row += L.nb * kRows) {
+      double acc[3];
+      spmv_row(L.vals, L.rowmap, L.col, row, lane, X, acc);
+      if (lane < 3) {
+        const double a = lane == 0 ? acc[0] : (lane == 1 ? acc[1] : acc[2]);
+        const size_t d = 3 * (size_t)row + lane;
+        L.q[d] = a;
+        dot += p[d] * a;
+      }
+    }
+  } else {
+    for (size_t i = b * (size_t)kT + threadIdx.x; i < 3 * (size_t)L.nn; i += (size_t)L.nb * kT) dot += L.p[i] * L.q[i];
+  }
+  const double t = block_reduce_all<kT>(dot, sh);
+  if (threadIdx.x == 0) L.P[b] = t;
+}
+
+__global__ __launch_bounds__(kT) void k_lz_update(LzArgs A, int step) {
+  __shared__ double sh[kT / 64];
+  const LzLevel& L = A.L[lz_level(A)];
+  const int b = blockIdx.x - L.b0;
+  const double pq = sum_partials_all<kT>(L.P, L.nb, sh);
+  const double rz = sum_partials_all<kT>(L.P + (1 + (step & 1)) * kLzBlocks, L.nb, sh);
+  if (b == 0 && threadIdx.x == 0) {
+    L.coef[2 * step] = rz;
+    L.coef[2 * step + 1] = pq;
+  }
+  const double alpha = rz / pq;
+  double rzn = 0.0;
+  for (int n = b * kT + threadIdx.x; n < L.nn; n += L.nb * kT) {
+    const size_t o = 3 * (size_t)n;
+    double v[3], z[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) v[i] = L.r[o + i] - alpha * L.q[o + i];
+    dinv3(L.dinv + 9 * (size_t)n, v, z);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      L.r[o + i] = v[i];
+      L.z[o + i] = z[i];
+      rzn += v[i] * z[i];
+    }
+  }
+  const double t = block_reduce_all<kT>(rzn, sh);
+  if (threadIdx.x == 0) L.P[(1 + ((step + 1) & 1)) * kLzBlocks + b] = t;
+}
+
+__global__ __launch_bounds__(kT) void k_lz_dir(LzArgs A, int step) {
+  __shared__ double sh[kT / 64];
+  const LzLevel& L = A.L[lz_level(A)];
+  const int b = blockIdx.x - L.b0;
+  const double rz = sum_partials_all<kT>(L.P + (1 + (step & 1)) * kLzBlocks, L.nb, sh);
+  const double rzn = sum_partials_all<kT>(L.P + (1 + ((step + 1) & 1)) * kLzBlocks, L.nb, sh);
+  const double beta = rzn / rz;
+  for (size_t i = b * (size_t)kT + threadIdx.x; i < 3 * (size_t)L.nn; i += (size_t)L.nb * kT)
+    L.p[i] = fma(beta, L.p[i], L.z[i]);
+}
+
+// Dense copy of a block-CRS matrix, one work-group per block row.
+__global__ __launch_bounds__(64) void k_crs_to_dense(const double* __restrict__ vals, const int* __restrict__ rowmap,
+                                                     const int* __restrict__ col, int nn, double* __restrict__ A,
+                                                     double* flag) {
+  const int r = blockIdx.x, n = 3 * nn;
+  if (r == 0 && threadIdx.x == 0) *flag = 0.0;
+  double* a = A + (size_t)3 * r * n;
+  for (int k = threadIdx.x; k < 3 * n; k += 64) a[k] = 0.0;
+  __syncthreads();
+  const int s0 = rowmap[r], len = 9 * (rowmap[r + 1] - s0);
+  for (int k = threadIdx.x; k < len; k += 64) {
+    const int s = s0 + k / 9, i = (k % 9) / 3, j = k % 3;
+    a[(size_t)i * n + 3 * col[s] + j] = vals[9 * (size_t)s + 3 * i + j];
+  }
+}
+
+// In-place Gauss-Jordan inverse of an n x n matrix, n <= 32 kGjTile, by one work-group of
+// 32 x 32 threads that holds it in registers (thread (ty, tx) the elements (ty + 32 a,
+// tx + 32 b)); a step exchanges its pivot row and column through LDS, one barrier a step.
+// 135 dofs (4x2x2 hexes): ~60 us, where the host's Cholesky with its two copies and waits
+// took ~0.6 ms.
+constexpr int kGjTile = 5;
+__global__ __launch_bounds__(1024) void k_gj_small(double* A, int n, double* flag) {
+  __shared__ double prow[2][32 * kGjTile], pcol[2][32 * kGjTile];
+  const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+  double m[kGjTile][kGjTile];
+#pragma unroll
+  for (int a = 0; a < kGjTile; ++a)
+#pragma unroll
+    for (int b = 0; b < kGjTile; ++b) {
+      const int i = ty + 32 * a, j = tx + 32 * b;
+      m[a][b] = i < n && j < n ? A[(size_t)i * n + j] : (i == j ? 1.0 : 0.0);
+    }
+#pragma unroll
+  for (int ka = 0; ka < kGjTile; ++ka)
+    for (int kr = 0; kr < 32; ++kr) {
+      const int k = 32 * ka + kr;
+      if (k >= n) break;
+      const int h = k & 1;
+      if (ty == kr)
+#pragma unroll
+        for (int b = 0; b < kGjTile; ++b) prow[h][tx + 32 * b] = m[ka][b];
+      if (tx == kr)
+#pragma unroll
+        for (int a = 0; a < kGjTile; ++a) pcol[h][ty + 32 * a] = m[a][ka];
+      __syncthreads();  // the other half's readers are one barrier behind
+      const double piv = prow[h][k], inv = 1.0 / piv;
+      if (!(piv > 0.0) && threadIdx.x == 0) *flag = 1.0;
+#pragma unroll
+      for (int a = 0; a < kGjTile; ++a) {
+        const bool ik = ty + 32 * a == k;
+        const double c = pcol[h][ty + 32 * a];
+#pragma unroll
+        for (int b = 0; b < kGjTile; ++b) {
+          const bool jk = tx + 32 * b == k;
+          const double r = (jk ? 1.0 : prow[h][tx + 32 * b]) * inv;
+          m[a][b] = ik ? r : (jk ? 0.0 : m[a][b]) - c * r;
+        }
+      }
+    }
+#pragma unroll
+  for (int a = 0; a < kGjTile; ++a)
+#pragma unroll
+    for (int b = 0; b < kGjTile; ++b) {
+      const int i = ty + 32 * a, j = tx + 32 * b;
+      if (i < n && j < n) A[(size_t)i * n + j] = m[a][b];
+    }
+}
+
+// One Gauss-Jordan step of a larger matrix, S -> D (two buffers: every element reads the
+// pivot row and column of S).
+__global__ __launch_bounds__(kT) void k_gj_step(const double* __restrict__ S, double* __restrict__ D, int n, int k,
+                                                double* flag) {
+  const double piv = S[(size_t)k * n + k], inv = 1.0 / piv;
+  if (!(piv > 0.0) && blockIdx.x == 0 && threadIdx.x == 0) *flag = 1.0;
+  for (int i = blockIdx.x; i < n; i += gridDim.x) {
+    const double c = S[(size_t)i * n + k];
+    for (int j = threadIdx.x; j < n; j += kT) {
+      const double r = (j == k ? 1.0 : S[(size_t)k * n + j]) * inv;
+      D[(size_t)i * n + j] = i == k ? r : (j == k ? 0.0 : S[(size_t)i * n + j]) - c * r;
+    }
+  }
 }
 
 }  // namespace
@@ -330,10 +497,6 @@ hipError_t launch_mg_rows(int mode, const MgRowArgs& a, hipStream_t s) {
 }
 hipError_t launch_to_f32(const double* a, float* b, size_t n, hipStream_t s) {
   k_to_f32<<<blocks_of(n), kT, 0, s>>>(a, b, n);
-  return hipGetLastError();
-}
-hipError_t launch_scale_rsqrt(double* y, size_t n, const double* scal, int slot, hipStream_t s) {
-  k_scale_rsqrt<<<blocks_of(n), kT, 0, s>>>(y, n, scal, slot);
   return hipGetLastError();
 }
 hipError_t launch_mg_prolong_add(const double* ec, double* xf, const int32_t* fgrid, const int32_t* cnode_of_grid,
@@ -372,10 +535,6 @@ hipError_t launch_add2(double* out, const double* a, const double* b, size_t n, 
   k_add2<<<blocks_of(n), kT, 0, s>>>(out, a, b, n);
   return hipGetLastError();
 }
-hipError_t launch_dinv_apply(double* y, const double* dinv, const double* x, int nn, hipStream_t s) {
-  k_dinv_apply<<<blocks_of(nn), kT, 0, s>>>(y, dinv, x, nn);
-  return hipGetLastError();
-}
 hipError_t launch_dense_gemv(const double* A, const double* x, double* y, int n, hipStream_t s) {
   k_dense_gemv<<<std::max(1, std::min(1024, (n + 3) / 4)), kT, 0, s>>>(A, x, y, n);
   return hipGetLastError();
@@ -387,6 +546,41 @@ hipError_t launch_mg_update(double* x, double* r, const double* p, const double*
 }
 hipError_t launch_mg_pupdate(double* p, const double* z, const double* scal, size_t n, hipStream_t s) {
   k_mg_pupdate<<<blocks_of(n), kT, 0, s>>>(p, z, scal, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_lz_init(const LzArgs& a, hipStream_t s) {
+  k_lz_init<<<a.blocks, kT, 0, s>>>(a);
+  return hipGetLastError();
+}
+hipError_t launch_lz_spmv(const LzArgs& a, hipStream_t s) {
+  k_lz_spmv<<<a.blocks, kT, 0, s>>>(a);
+  return hipGetLastError();
+}
+hipError_t launch_lz_update(const LzArgs& a, int step, hipStream_t s) {
+  k_lz_update<<<a.blocks, kT, 0, s>>>(a, step);
+  return hipGetLastError();
+}
+hipError_t launch_lz_dir(const LzArgs& a, int step, hipStream_t s) {
+  k_lz_dir<<<a.blocks, kT, 0, s>>>(a, step);
+  return hipGetLastError();
+}
+hipError_t launch_mg_dense_inverse(const double* vals, const int32_t* rowmap, const int32_t* col, int nn, double* A,
+                                   double* T, double* flag, hipStream_t s) {
+  const int n = 3 * nn;
+  if (n <= 32 * kGjTile) {
+    k_crs_to_dense<<<nn, 64, 0, s>>>(vals, rowmap, col, nn, A, flag);
+    k_gj_small<<<1, 1024, 0, s>>>(A, n, flag);
+    return hipGetLastError();
+  }
+  // n steps between the two buffers, ending in A
+  double* src = n % 2 ? T : A;
+  k_crs_to_dense<<<nn, 64, 0, s>>>(vals, rowmap, col, nn, src, flag);
+  for (int k = 0; k < n; ++k) {
+    double* dst = src == A ? T : A;
+    k_gj_step<<<std::min(n, 2048), kT, 0, s>>>(src, dst, n, k, flag);
+    src = dst;
+  }
   return hipGetLastError();
 }
 

@@ -41,11 +41,10 @@ hipError_t launch_cheb_first(double* x, double* d, const double* r, const double
                              hipStream_t s, const double* t = nullptr);
 hipError_t launch_cheb_next(double* x, double* d, const double* r, const double* Kx, const double* dinv, double c1,
                             double c2, int nn, hipStream_t s);
-// out = a - b ; y += x ; y = D^-1 x
+// out = a - b ; y += x
 hipError_t launch_sub(double* out, const double* a, const double* b, size_t n, hipStream_t s);
 hipError_t launch_add(double* y, const double* x, size_t n, hipStream_t s);
 hipError_t launch_add2(double* out, const double* a, const double* b, size_t n, hipStream_t s);  // out = a + b
-hipError_t launch_dinv_apply(double* y, const double* dinv, const double* x, int nn, hipStream_t s);
 // y = A x with A dense n x n (row major)
 hipError_t launch_dense_gemv(const double* A, const double* x, double* y, int n, hipStream_t s);
 
@@ -73,8 +72,42 @@ struct MgRowArgs {
 hipError_t launch_mg_rows(int mode, const MgRowArgs& a, hipStream_t s);
 // b = (float) a, n values
 hipError_t launch_to_f32(const double* a, float* b, size_t n, hipStream_t s);
-// y *= 1 / sqrt(scal[slot])  (power-iteration normalisation without a host round trip)
-hipError_t launch_scale_rsqrt(double* y, size_t n, const double* scal, int slot, hipStream_t s);
+
+// Spectral estimates of every smoothed level at once (block-Jacobi PCG on K x = v with a
+// fixed pseudo-random v; its coefficients are the Lanczos tridiagonal): each kernel works
+// on all levels in one launch, a level owning the work-groups [b0, b0 + nb) of the grid.
+// The scalars stay on the device: rz_j and pq_j of step j go to coef[2j], coef[2j + 1].
+//   init:   r = v, z = D^-1 r, p = z; partials of r.z
+//   spmv:   q = K p on the levels with a matrix (vals), q as given on the others; partials of p.q
+//   update: alpha = rz / pq; r -= alpha q; z = D^-1 r; partials of the next r.z
+//   dir:    p = z + beta p, beta = rz_next / rz
+constexpr int kMgLevelsMax = 12;  // below 2^28 elements the shortest axis halves at most 9 times
+constexpr int kLzBlocks = 1024;   // work-groups (and partials) of a level at most
+constexpr int kLzSteps = 16;
+struct LzLevel {
+  const double* vals;  // null: q is computed by the caller
+  const int32_t* rowmap;
+  const int32_t* col;
+  const double* dinv;
+  double *r, *z, *p, *q;
+  double* coef;  // 2 kLzSteps
+  double* P;     // 3 x kLzBlocks partials: p.q, r.z of even steps, r.z of odd steps
+  int nn, b0, nb;
+};
+struct LzArgs {
+  LzLevel L[kMgLevelsMax];
+  int nlev, blocks;
+};
+hipError_t launch_lz_init(const LzArgs& a, hipStream_t s);
+hipError_t launch_lz_spmv(const LzArgs& a, hipStream_t s);
+hipError_t launch_lz_update(const LzArgs& a, int step, hipStream_t s);
+hipError_t launch_lz_dir(const LzArgs& a, int step, hipStream_t s);
+
+// Inverse of the coarsest level's matrix (symmetric positive definite, 3 nn square) into A,
+// by Gauss-Jordan elimination on the device; T is scratch of the same size.  *flag (device)
+// becomes 1 when a pivot is not positive, else 0.
+hipError_t launch_mg_dense_inverse(const double* vals, const int32_t* rowmap, const int32_t* col, int nn, double* A,
+                                   double* T, double* flag, hipStream_t s);
 
 // PCG steps of the multigrid-preconditioned solve (scalars in scal, see ScalarSlot):
 //   update: x += alpha p; r -= alpha q (alpha = scal[kAlpha]); partials of r.r
