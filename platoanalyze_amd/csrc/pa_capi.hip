@@ -774,7 +774,7 @@ int pa_apply_constraints(pa_handle h, double* vals, double* rhs, double scale) {
   if (nbc == 0) return PA_OK;
   const int g = grid_for(nbc);
   pa::k_bc_lift<<<g, 256, 0, h->stream>>>(vals, h->rowmap.p, h->colidx.p, h->bc_d.p, h->bc_v.p, nbc, scale, rhs);
-  pa::k_bc_zero<<<g, 256, 0, h->stream>>>(vals, h->rowmap.p, h->colidx.p, h->bc_d.p, nbc);
+  pa::k_bc_zero<<<grid_for(nbc, 16), 256, 0, h->stream>>>(vals, h->rowmap.p, h->colidx.p, h->bc_d.p, nbc);
   pa::k_bc_set<<<g, 256, 0, h->stream>>>(rhs, h->bc_d.p, h->bc_v.p, nbc, scale);
   PA_HIP(hipGetLastError());
   return PA_OK;

@@ -274,19 +274,26 @@ __global__ __launch_bounds__(kT) void k_bc_lift(const double* vals, const int* r
 }
 
 // applyBlockConstraints first loop, matrix part: BC row -> unit diagonal, zero
-// elsewhere; the symmetric (col,row) entries zeroed too.
+// elsewhere; the symmetric (col,row) entries zeroed too.  16 lanes per BC dof, a lane per
+// block of its row, the partner row searched once without a data-dependent exit (its loads
+// are independent): a thread per dof walked ~15 blocks x 3 components x ~15 dependent loads
+// and took 68-96 us whatever the size (20x10x10: 84 us).
 __global__ __launch_bounds__(kT) void k_bc_zero(double* vals, const int* rowmap, const int* col,
                                                 const int* dofs, int nbc) {
-  for (int k = blockIdx.x * kT + threadIdx.x; k < nbc; k += gridDim.x * kT) {
+  const int lane = threadIdx.x % kLanesPerRow;
+  for (int k = (blockIdx.x * kT + threadIdx.x) / kLanesPerRow; k < nbc; k += gridDim.x * kRowsPerBlock) {
     const int d = dofs[k], n = d / 3, i = d % 3;
-    for (int s = rowmap[n]; s < rowmap[n + 1]; ++s) {
+    for (int s = rowmap[n] + lane; s < rowmap[n + 1]; s += kLanesPerRow) {
       const int c = col[s];
+      int p = -1;  // slot of block (c, n)
+      const int t1 = rowmap[c + 1];
+#pragma unroll 4
+      for (int t = rowmap[c]; t < t1; ++t) p = col[t] == n ? t : p;
+#pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const int cd = 3 * c + j;
-        vals[9 * (size_t)s + 3 * i + j] = (cd == d) ? 1.0 : 0.0;
-        if (cd == d) continue;
-        for (int t = rowmap[c]; t < rowmap[c + 1]; ++t)
-          if (col[t] == n) vals[9 * (size_t)t + 3 * j + i] = 0.0;
+        const bool diag = 3 * c + j == d;
+        vals[9 * (size_t)s + 3 * i + j] = diag ? 1.0 : 0.0;
+        if (!diag && p >= 0) vals[9 * (size_t)p + 3 * j + i] = 0.0;
       }
     }
   }
