@@ -771,8 +771,14 @@ __global__ __launch_bounds__(256) void k_box_diag_inv(BoxArgs A, const uint8_t* 
 }
 
 __global__ __launch_bounds__(256) void k_boxmf_scatter(BoxMfArgs A) {
+  __shared__ double sh[2 * 256 / 64];
   const int px = A.nx + 2, py = A.ny + 2;
-  const double beta = A.first ? 0.0 : A.scal[kBeta];
+  double beta = 0.0;
+  if (!A.first) {
+    double a, b;
+    sum_partials_two<256>(A.P_rz_new, A.np_rz, A.P_rz_old, A.np_rz, sh, a, b);
+    beta = a / b;
+  }
   for (int n = blockIdx.x * 256 + threadIdx.x; n < A.nrows; n += gridDim.x * 256) {
     const int g = A.gpack[n];
     const size_t hp = (size_t)((g & 1023) + 1) + (size_t)px * ((((g >> 10) & 1023) + 1) + (size_t)py * ((g >> 20) + 1));

@@ -109,8 +109,11 @@ struct BoxMfArgs {
   const double* z;         // FP64 vectors in node order
   const double* p_prev;
   double* p_cur;           // null: no FP64 copy of p (constrained rows give y = 0)
-  int first;               // p = z (else p = z + scal[kBeta] p_prev)
-  const double* scal;
+  int first;               // p = z (else p = z + beta p_prev, beta the quotient of the
+                           // sums of the np_rz partials P_rz_new and P_rz_old)
+  const double* P_rz_new;
+  const double* P_rz_old;
+  int np_rz;
   float4* plat;            // [padded lattice] p (FP32) at the node's lattice point
   double* y;
   double* partials;        // one p.y partial per work-group of k_boxmf_apply

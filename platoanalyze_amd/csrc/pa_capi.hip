@@ -162,7 +162,7 @@ struct pa_problem {
   // E = V^T A V, its inverse, mu
   DevArray<double> d_V, d_AV, d_P, d_E, d_Einv, d_mu;
   // solver workspace (lazily allocated)
-  DevArray<double> w_r, w_z, w_p, w_q, w_dinv, w_vals, w_adj, w_adjz, w_K;
+  DevArray<double> w_r, w_z, w_p, w_p2, w_q, w_dinv, w_vals, w_adj, w_adjz, w_K;
   // shape derivative of the traction load: value positions in the transposed dR/dX
   // matrix and their (constant) contributions, built on first use
   bool gx_built = false;
@@ -708,6 +708,13 @@ int pa_sf_gradient_x(pa_handle h, const double* u, const double* z, double* g) {
 
 static int energy_value(pa_handle h, double* value);
 static int ensure_solver_ws(pa_handle h);
+// fixed-order sum of n partials into scal[slot] and, once the stream is waited for,
+// h->host_scal[slot]
+static int sum_to_host(pa_handle h, const double* partials, int n, double* scal, int slot) {
+  pa::k_sum<<<1, pa::kSumThreads, 0, h->stream>>>(partials, n, scal, slot, h->host_scal);
+  PA_HIP(hipGetLastError());
+  return PA_OK;
+}
 
 // Plato::Geometric::Volume (src/geometric/Volume.hpp:49-96) with its own penalty
 // function, through GeometryScalarFunction value / gradient_z / gradient_x
@@ -736,10 +743,7 @@ int pa_volume(pa_handle h, const double* z, int model, double exponent, double m
 
 // --------------------------------------------------------------- scalar function
 static int energy_value(pa_handle h, double* value) {
-  pa::k_sum<<<1, 256, 0, h->stream>>>(h->chunk_partials.p, h->chunks.count, h->scal.p, pa::kEnergy);
-  PA_HIP(hipGetLastError());
-  PA_HIP(hipMemcpyAsync(h->host_scal, h->scal.p, pa::kNumScal * sizeof(double), hipMemcpyDeviceToHost,
-                        h->stream));
+  if (int rc = sum_to_host(h, h->chunk_partials.p, h->chunks.count, h->scal.p, pa::kEnergy)) return rc;
   PA_HIP(hipStreamSynchronize(h->stream));
   *value = h->host_scal[pa::kEnergy];
   return PA_OK;
@@ -786,24 +790,24 @@ static int ensure_solver_ws(pa_handle h) {
     PA_HIP(h->w_r.alloc(ndof));
     PA_HIP(h->w_z.alloc(ndof));
     PA_HIP(h->w_p.alloc(ndof));
+    PA_HIP(h->w_p2.alloc(ndof));
     PA_HIP(h->w_q.alloc(ndof));
     PA_HIP(h->w_dinv.alloc(9 * (size_t)h->nn));
   }
   return PA_OK;
 }
 
-static int read_scal(pa_handle h, const double* scal) {
-  PA_HIP(hipMemcpyAsync(h->host_scal, scal, pa::kNumScal * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+static int read_scal(pa_handle h) {
+  PA_HIP(hipMemcpyAsync(h->host_scal, h->scal.p, pa::kNumScal * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   PA_HIP(hipStreamSynchronize(h->stream));
   return PA_OK;
 }
-static int read_scal(pa_handle h) { return read_scal(h, h->scal.p); }
 
-// Device workspace of the block-Jacobi PCG: four node vectors (3N doubles each), the 3x3
+// Device workspace of the block-Jacobi PCG: five node vectors (3N doubles each), the 3x3
 // block-diagonal inverse (9N), kNumPartialSlots x kRedBlocks reduction partials and
 // kNumScal scalars.  Every entry is written before it is read.
 struct PcgWork {
-  double *r, *z, *p, *q, *dinv, *partials, *scal;
+  double *r, *z, *p, *p2, *q, *dinv, *partials, *scal;
 };
 
 static int solve_opts(const pa_solver_opts* o, pa_solver_opts& opts, const char* who) {
@@ -838,6 +842,13 @@ static int deflate_apply(pa_handle h, const Deflation& D, const double* X, const
   return PA_OK;
 }
 
+// Meshes up to this many nodes form the direction inside the product (k_pcg_dir_spmv):
+// an iteration takes 10.7 us instead of 13.9 at 2541 nodes and 25.1 instead of 27.1 at
+// 70785 (both with the other changes of the update kernel); at 136161 nodes the second
+// gathered vector costs more than the launch (40.1 us against 38.9), at 545025 198 us
+// against 180.
+constexpr int kFusedDirNodes = 100000;
+
 // Jacobi(3x3 block)-PCG in FP64 on the handle's graph, on the workspace W; with a
 // deflation space D, deflated PCG (the start corrected by V E^-1 V^T r, every direction
 // projected: p -= V E^-1 (A V)^T z).
@@ -866,30 +877,37 @@ static int pcg_block_jacobi(pa_handle h, const double* vals, double* x, const do
                                     PS(pa::kPBB));
   if (D)
     if (int rc = deflate_apply(h, *D, D->AV, W.z, W.p, D->V, -1.0, G)) return rc;
-  pa::k_sum<<<1, 256, 0, s>>>(PS(pa::kPRR), G, W.scal, pa::kRR);
-  pa::k_sum<<<1, 256, 0, s>>>(PS(pa::kPBB), G, W.scal, pa::kBB);
-  PA_HIP(hipGetLastError());
-  if (int rc = read_scal(h, W.scal)) return rc;
+  if (int rc = sum_to_host(h, PS(pa::kPRR), G, W.scal, pa::kRR)) return rc;
+  if (int rc = sum_to_host(h, PS(pa::kPBB), G, W.scal, pa::kBB)) return rc;
+  PA_HIP(hipStreamSynchronize(s));
   const double bb = h->host_scal[pa::kBB];
   double rel = bb > 0 ? std::sqrt(h->host_scal[pa::kRR] / bb) : 0.0;
   int it = 0;
   bool conv = bb == 0.0 || rel <= opts.tolerance;
   if (bb == 0.0) pa::k_fill<<<grid_for(ndof), 256, 0, s>>>(x, ndof, 0.0);  // b = 0: the solution is 0, whatever x0
+  // a deflated direction is projected after its update, so it cannot be formed in the product
+  const bool fused = !D && nn <= kFusedDirNodes;
+  double* pb[2] = {W.p, W.p2};
   while (!conv && it < opts.max_iters) {
     // rz of this iteration in P_RZ[cur]; the update writes the next one into P_RZ[cur ^ 1]
     const int cur = it & 1;
-    pa::k_pcg_spmv<<<Gs, 256, 0, s>>>(vals, h->rowmap.p, h->colidx.p, W.p, W.q, nn, PS(pa::kPPQ));
-    pa::k_pcg_update<<<G, 256, 0, s>>>(x, W.r, W.z, W.p, W.q, W.dinv, nn, PS(pa::kPPQ),
+    double* p = fused ? pb[cur] : W.p;
+    if (fused)
+      pa::k_pcg_dir_spmv<<<Gs, 256, 0, s>>>(vals, h->rowmap.p, h->colidx.p, W.z, pb[cur ^ 1], p, W.q, nn, it == 0,
+                                            PS(pa::kPRZ0 + cur), PS(pa::kPRZ0 + (cur ^ 1)), G, PS(pa::kPPQ));
+    else
+      pa::k_pcg_spmv<<<Gs, 256, 0, s>>>(vals, h->rowmap.p, h->colidx.p, p, W.q, nn, PS(pa::kPPQ));
+    pa::k_pcg_update<<<G, 256, 0, s>>>(x, W.r, W.z, p, W.q, W.dinv, nn, PS(pa::kPPQ),
                                        Gs, PS(pa::kPRZ0 + cur), G, PS(pa::kPRZ0 + (cur ^ 1)), PS(pa::kPRR),
                                        W.scal);
-    pa::k_pcg_pupdate<<<G, 256, 0, s>>>(W.p, W.z, nn, PS(pa::kPRZ0 + (cur ^ 1)), PS(pa::kPRZ0 + cur), G);
+    if (!fused)
+      pa::k_pcg_pupdate<<<G, 256, 0, s>>>(W.p, W.z, nn, PS(pa::kPRZ0 + (cur ^ 1)), PS(pa::kPRZ0 + cur), G);
     if (D)
       if (int rc = deflate_apply(h, *D, D->AV, W.z, W.p, D->V, -1.0, G)) return rc;
     ++it;
     if (it % opts.check_every == 0 || it == opts.max_iters) {
-      pa::k_sum<<<1, 256, 0, s>>>(PS(pa::kPRR), G, W.scal, pa::kRR);
-      PA_HIP(hipGetLastError());
-      if (int rc = read_scal(h, W.scal)) return rc;
+      if (int rc = sum_to_host(h, PS(pa::kPRR), G, W.scal, pa::kRR)) return rc;
+      PA_HIP(hipStreamSynchronize(s));
       rel = std::sqrt(h->host_scal[pa::kRR] / bb);
       if (!std::isfinite(rel)) return fail(PA_ERR_NOT_CONVERGED, "PCG produced a non-finite residual");
       conv = rel <= opts.tolerance;
@@ -898,9 +916,8 @@ static int pcg_block_jacobi(pa_handle h, const double* vals, double* x, const do
   // true residual
   pa::k_spmv<<<Gs, 256, 0, s>>>(vals, h->rowmap.p, h->colidx.p, x, b, W.r, nn, 1);
   pa::k_dot<<<G, 256, 0, s>>>(W.r, W.r, ndof, PS(pa::kPDot));
-  pa::k_sum<<<1, 256, 0, s>>>(PS(pa::kPDot), G, W.scal, pa::kDot0);
-  PA_HIP(hipGetLastError());
-  if (int rc = read_scal(h, W.scal)) return rc;
+  if (int rc = sum_to_host(h, PS(pa::kPDot), G, W.scal, pa::kDot0)) return rc;
+  PA_HIP(hipStreamSynchronize(s));
   const double true_rel = bb > 0 ? std::sqrt(h->host_scal[pa::kDot0] / bb) : 0.0;
   if (st) {
     st->iterations = it;
@@ -922,7 +939,7 @@ int pa_solve(pa_handle h, const double* vals, double* x, const double* b, const 
   if (int rc = solve_opts(o, opts, "pa_solve")) return rc;
   if (int rc = ensure_solver_ws(h)) return rc;
   return pcg_block_jacobi(h, vals, x, b, opts, st,
-                          PcgWork{h->w_r.p, h->w_z.p, h->w_p.p, h->w_q.p, h->w_dinv.p, h->partials.p, h->scal.p});
+                          PcgWork{h->w_r.p, h->w_z.p, h->w_p.p, h->w_p2.p, h->w_q.p, h->w_dinv.p, h->partials.p, h->scal.p});
 }
 
 // ------------------------------------------------------------ solve without allocation
@@ -932,7 +949,7 @@ int pa_solve(pa_handle h, const double* vals, double* x, const double* b, const 
 // each GPU's copy comes from hipGetSymbolAddress, taken once per device with that device
 // current, and only that address is handed to kernels.
 constexpr size_t kNoAllocPartials = (size_t)pa::kNumPartialSlots * pa::kRedBlocks;
-constexpr size_t kNoAllocDoubles = 21 * (size_t)PA_NOALLOC_MAX_NODES + kNoAllocPartials + pa::kNumScal;
+constexpr size_t kNoAllocDoubles = 24 * (size_t)PA_NOALLOC_MAX_NODES + kNoAllocPartials + pa::kNumScal;
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
 constexpr int kNoAllocMaxDevices = 64;
@@ -966,7 +983,7 @@ int pa_solve_noalloc(pa_handle h, const double* vals, double* x, const double* b
   double* ws = nullptr;
   if (int rc = noalloc_scratch(&ws)) return rc;
   const size_t nd = 3 * (size_t)h->nn;
-  PcgWork W{ws, ws + nd, ws + 2 * nd, ws + 3 * nd, ws + 4 * nd, ws + 4 * nd + 9 * (size_t)h->nn, nullptr};
+  PcgWork W{ws, ws + nd, ws + 2 * nd, ws + 3 * nd, ws + 4 * nd, ws + 5 * nd, ws + 5 * nd + 9 * (size_t)h->nn, nullptr};
   W.scal = W.partials + kNoAllocPartials;
   return pcg_block_jacobi(h, vals, x, b, opts, st, W);
 }
@@ -1056,7 +1073,9 @@ static int mf_apply(pa_handle h, const pa::MfArgs& ma, const double** P, int* np
     b.p_prev = ma.p_prev;
     b.p_cur = ma.p_cur;
     b.first = ma.first;
-    b.scal = ma.scal;
+    b.P_rz_new = ma.P_rz_new;
+    b.P_rz_old = ma.P_rz_old;
+    b.np_rz = ma.np_rz;
     b.plat = h->box_plat.p;
     b.y = ma.y;
     b.partials = h->box_mf_part.p;
@@ -1116,16 +1135,14 @@ static int solve_mixed(pa_handle h, const double* z, double* u, const double* b,
   ma.bcmask = h->bcmask.p;
   ma.z = h->m_z.p;
   ma.y = h->m_q.p;
-  ma.scal = h->scal.p;
   ma.partials = h->chunk_partials.p;
   ma.m = h->material();
   ma.gbound = h->chunk_gbound.p;
   // r = mask(b - R) into m_r and ||r||^2
   auto masked_residual = [&](const double* R, double* out) -> int {
     PA_HIP(pa::launch_neg_mask(R, b, h->bcmask.p, h->m_r.p, nn, PS(pa::kPDot), G, s));
-    pa::k_sum<<<1, 256, 0, s>>>(PS(pa::kPDot), G, h->scal.p, pa::kDot1);
-    PA_HIP(hipGetLastError());
-    if (int rc = read_scal(h)) return rc;
+    if (int rc = sum_to_host(h, PS(pa::kPDot), G, h->scal.p, pa::kDot1)) return rc;
+    PA_HIP(hipStreamSynchronize(s));
     *out = h->host_scal[pa::kDot1];
     return PA_OK;
   };
@@ -1154,10 +1171,10 @@ static int solve_mixed(pa_handle h, const double* z, double* u, const double* b,
   if (!std::isfinite(rel)) return fail(PA_ERR_NOT_CONVERGED, "mixed-precision solve: non-finite residual");
   conv = bb == 0.0 || rel <= opts.tolerance;
   if (bb == 0.0) pa::k_fill<<<grid_for(ndof), 256, 0, s>>>(u, ndof, 0.0);  // f = 0: the solution is 0, whatever u0
-  if (!conv) {
-    PA_HIP(pa::launch_pcgm_init(h->m_r.p, h->m_z.p, h->m_dinv.p, nn, PS(pa::kPRZ0), G, s));
-    PA_HIP(pa::launch_pcgm_beta(PS(pa::kPRZ0), nullptr, G, h->scal.p, pa::kBetaInit, s));
-  }
+  // r.z of the iteration in P_RZ[cur], the update writes the next one into P_RZ[cur ^ 1];
+  // the apply (or the lattice scatter) takes beta from both and the update alpha from the
+  // p.q partials, so an iteration has no one-group summing kernels of its own
+  if (!conv) PA_HIP(pa::launch_pcgm_init(h->m_r.p, h->m_z.p, h->m_dinv.p, nn, PS(pa::kPRZ0), G, s));
   int it = 0;
   bool restart = true;  // the next apply starts the direction from p = z
   while (!conv) {
@@ -1166,18 +1183,26 @@ static int solve_mixed(pa_handle h, const double* z, double* u, const double* b,
     restart = false;
     ma.p_prev = pbuf[cur ^ 1];
     ma.p_cur = pbuf[cur];
+    ma.P_rz_new = PS(pa::kPRZ0 + cur);
+    ma.P_rz_old = PS(pa::kPRZ0 + (cur ^ 1));
+    ma.np_rz = G;
     const double* Pq = nullptr;
     int npq = 0;
     if (int rc = mf_apply(h, ma, &Pq, &npq)) return rc;
-    PA_HIP(pa::launch_pcgm_alpha(Pq, npq, h->scal.p, s));
-    PA_HIP(pa::launch_pcgm_update(u, h->m_r.p, h->m_z.p, pbuf[cur], h->m_q.p, h->m_dinv.p, nn, h->scal.p,
-                                  PS(pa::kPRZ0), PS(pa::kPRR), G, s));
-    PA_HIP(pa::launch_pcgm_beta(PS(pa::kPRZ0), PS(pa::kPRR), G, h->scal.p, pa::kBetaStep, s));
+    if (npq > pa::kRedBlocks) {  // more partials than every work-group of the update should sum
+      pa::k_sum<<<1, pa::kSumThreads, 0, s>>>(Pq, npq, h->scal.p, pa::kDot0, nullptr);
+      Pq = h->scal.p + pa::kDot0;
+      npq = 1;
+    }
+    pa::k_pcg_update<<<G, 256, 0, s>>>(u, h->m_r.p, h->m_z.p, pbuf[cur], h->m_q.p, h->m_dinv.p, nn, Pq, npq,
+                                       PS(pa::kPRZ0 + cur), G, PS(pa::kPRZ0 + (cur ^ 1)), PS(pa::kPRR), h->scal.p);
+    PA_HIP(hipGetLastError());
     ++it;
     ++inner_total;
     const bool last = inner_total >= opts.max_iters;
     if (it % opts.check_every != 0 && !last) continue;
-    if (int rc = read_scal(h)) return rc;
+    if (int rc = sum_to_host(h, PS(pa::kPRR), G, h->scal.p, pa::kRR)) return rc;
+    PA_HIP(hipStreamSynchronize(s));
     const double rr_it = h->host_scal[pa::kRR];
     if (!std::isfinite(rr_it)) return fail(PA_ERR_NOT_CONVERGED, "mixed-precision PCG: non-finite residual");
     // replace when the iterated residual has dropped enough, or could already meet the
@@ -1196,9 +1221,7 @@ static int solve_mixed(pa_handle h, const double* z, double* u, const double* b,
     // continue from the replaced residual: z = Dinv r, beta = (r.z) / rz of the last step;
     // restart from p = z instead when the true residual is well above the iterated one
     restart = rr_ref > 4.0 * rr_it;
-    PA_HIP(pa::launch_pcgm_init(h->m_r.p, h->m_z.p, h->m_dinv.p, nn, PS(pa::kPRZ0), G, s));
-    PA_HIP(pa::launch_pcgm_beta(PS(pa::kPRZ0), nullptr, G, h->scal.p, restart ? pa::kBetaInit : pa::kBetaReplace,
-                                s));
+    PA_HIP(pa::launch_pcgm_init(h->m_r.p, h->m_z.p, h->m_dinv.p, nn, PS(pa::kPRZ0 + (cur ^ 1)), G, s));
   }
   if (st) {
     st->iterations = inner_total;
@@ -1769,7 +1792,6 @@ static int mg_apply(pa_handle h, size_t l, const double* x, double* y, const dou
       // masked value, and the p.y partials go unused); the chunk apply writes one
       ma.p_cur = h->box_fast && h->box_mf ? nullptr : h->g_pc.p;
       ma.first = 1;
-      ma.scal = h->scal.p;
       ma.y = y;
       ma.partials = h->chunk_partials.p;
       ma.m = h->material();
@@ -1894,10 +1916,9 @@ static int mg_dot(pa_handle h, const double* a, const double* b, size_t n, int s
   double* P = h->partials.p + (size_t)pa::kPDot * pa::kRedBlocks;
   const int G = pa::red_grid(n / 3 + 1, 256);
   pa::k_dot<<<G, 256, 0, h->stream>>>(a, b, n, P);
-  pa::k_sum<<<1, 256, 0, h->stream>>>(P, G, h->scal.p, slot);
-  PA_HIP(hipGetLastError());
+  if (int rc = sum_to_host(h, P, G, h->scal.p, slot)) return rc;
   if (out) {
-    if (int rc = read_scal(h)) return rc;
+    PA_HIP(hipStreamSynchronize(h->stream));
     *out = h->host_scal[slot];
   }
   return PA_OK;
@@ -2079,9 +2100,8 @@ static int solve_mg(pa_handle h, const double* z, double* x, const double* b, co
   auto true_residual = [&](double* rr) -> int {
     if (int rc = residual(h, x, z, h->m_R.p, b == nullptr)) return rc;
     PA_HIP(pa::launch_neg_mask(h->m_R.p, b, h->bcmask.p, h->g_r.p, nn, PS(pa::kPDot), G, s));
-    pa::k_sum<<<1, 256, 0, s>>>(PS(pa::kPDot), G, h->scal.p, pa::kDot1);
-    PA_HIP(hipGetLastError());
-    if (int rc = read_scal(h)) return rc;
+    if (int rc = sum_to_host(h, PS(pa::kPDot), G, h->scal.p, pa::kDot1)) return rc;
+    PA_HIP(hipStreamSynchronize(s));
     *rr = h->host_scal[pa::kDot1];
     return PA_OK;
   };
@@ -2095,9 +2115,8 @@ static int solve_mg(pa_handle h, const double* z, double* x, const double* b, co
     if (b) {  // ||mask(b)||^2
       pa::k_fill<<<grid_for(ndof), 256, 0, s>>>(h->m_R.p, ndof, 0.0);
       PA_HIP(pa::launch_neg_mask(h->m_R.p, b, h->bcmask.p, h->g_r.p, nn, PS(pa::kPDot), G, s));
-      pa::k_sum<<<1, 256, 0, s>>>(PS(pa::kPDot), G, h->scal.p, pa::kDot1);
-      PA_HIP(hipGetLastError());
-      if (int rc = read_scal(h)) return rc;
+      if (int rc = sum_to_host(h, PS(pa::kPDot), G, h->scal.p, pa::kDot1)) return rc;
+      PA_HIP(hipStreamSynchronize(s));
       bb = h->host_scal[pa::kDot1];
     }
     if (int rc = true_residual(&rr0)) return rc;
@@ -2286,7 +2305,7 @@ int pa_solution_deflated(pa_handle h, const double* z, double* u, double* vals, 
   if (int rc = pa_apply_constraints(h, vals, rhs, 1.0)) return rc;
   const int nbc = (int)h->bc_dofs.size();
   if (opts.use_x0 && nbc) pa::k_bc_set<<<grid_for(nbc), 256, 0, s>>>(u, h->bc_d.p, h->bc_v.p, nbc, 1.0);
-  PcgWork work{h->w_r.p, h->w_z.p, h->w_p.p, h->w_q.p, h->w_dinv.p, h->partials.p, h->scal.p};
+  PcgWork work{h->w_r.p, h->w_z.p, h->w_p.p, h->w_p2.p, h->w_q.p, h->w_dinv.p, h->partials.p, h->scal.p};
   if (k == 0) return pcg_block_jacobi(h, vals, u, rhs, opts, st, work);
   // V = W with the constrained dofs zeroed, A V, E = V^T A V
   const size_t kn = (size_t)k * ndof;

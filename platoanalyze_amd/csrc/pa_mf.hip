@@ -67,10 +67,15 @@ __global__ __launch_bounds__(NT) void k_mf_apply(MfArgs A) {
   double* acc = pown + 3 * mr2;
   float4* nd4 = reinterpret_cast<float4*>(acc + 3 * mr2);
   float* xl = reinterpret_cast<float*>(nd4 + A.max_nodes);
-  __shared__ double sh[NT / 64];
+  __shared__ double sh[2 * NT / 64];
   __shared__ double red[NT / 64];
 
-  const double beta = A.first ? 0.0 : A.scal[kBeta];
+  double beta = 0.0;
+  if (!A.first) {
+    double a, b;
+    sum_partials_two<NT>(A.P_rz_new, A.np_rz, A.P_rz_old, A.np_rz, sh, a, b);
+    beta = a / b;
+  }
   const int c = xcd_map(blockIdx.x, A.nchunks);
   const int r0 = A.chunk_rows[c], r1 = A.chunk_rows[c + 1], nr = r1 - r0;
   const int n0 = A.node_offs[c], nnode = A.node_offs[c + 1] - n0;
@@ -251,41 +256,6 @@ __global__ __launch_bounds__(kFin) void k_pcgm_alpha(const double* partials, int
   }
 }
 
-// x += alpha p; r -= alpha q; z = Dinv r (alpha = scal[kAlpha]); partials of r.z, r.r
-__global__ __launch_bounds__(kT) void k_pcgm_update(double* __restrict__ x, double* __restrict__ r,
-                                                    double* __restrict__ z, const double* __restrict__ p,
-                                                    const double* __restrict__ q, const double* __restrict__ dinv,
-                                                    int nn, const double* __restrict__ scal,
-                                                    double* __restrict__ P_rz, double* __restrict__ P_rr) {
-  __shared__ double sh[kT / 64];
-  const double alpha = scal[kAlpha];
-  double rzn = 0.0, rr = 0.0;
-  const XcdSpan sp = xcd_span(nn);
-  for (int n = sp.lo + sp.j * kT + threadIdx.x; n < sp.hi; n += sp.bx * kT) {
-    const size_t d = 3 * (size_t)n;
-    double rv[3], zv[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      x[d + i] += alpha * p[d + i];
-      rv[i] = r[d + i] - alpha * q[d + i];
-      r[d + i] = rv[i];
-    }
-    dinv3(dinv + 9 * (size_t)n, rv, zv);
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      z[d + i] = zv[i];
-      rzn += rv[i] * zv[i];
-      rr += rv[i] * rv[i];
-    }
-  }
-  const double t0 = block_reduce_all<kT>(rzn, sh);
-  const double t1 = block_reduce_all<kT>(rr, sh);
-  if (threadIdx.x == 0) {
-    P_rz[blockIdx.x] = t0;
-    P_rr[blockIdx.x] = t1;
-  }
-}
-
 __global__ __launch_bounds__(kFin) void k_pcgm_beta(const double* P_rz, const double* P_rr, int n, double* scal,
                                                     int mode) {
   __shared__ double sh[kFin / 64];
@@ -369,11 +339,6 @@ hipError_t launch_pcgm_init(const double* r, double* z, const double* dinv, int 
 }
 hipError_t launch_pcgm_alpha(const double* partials, int n, double* scal, hipStream_t s) {
   k_pcgm_alpha<<<1, kFin, 0, s>>>(partials, n, scal);
-  return hipGetLastError();
-}
-hipError_t launch_pcgm_update(double* x, double* r, double* z, const double* p, const double* q, const double* dinv,
-                              int nn, const double* scal, double* P_rz, double* P_rr, int grid, hipStream_t s) {
-  k_pcgm_update<<<grid, kT, 0, s>>>(x, r, z, p, q, dinv, nn, scal, P_rz, P_rr);
   return hipGetLastError();
 }
 hipError_t launch_pcgm_beta(const double* P_rz, const double* P_rr, int n, double* scal, int mode, hipStream_t s) {

@@ -20,13 +20,15 @@ struct MfArgs {
   int nchunks, max_rows, max_nodes;
   const float4* Xz;       // FP32 x, y, z, density per node
   const uint8_t* bcmask;  // bit i set: dof 3n+i constrained
-  // direction update fused into the apply: p_cur = z + beta p_prev with beta =
-  // scal[kBeta] (p_cur = z when first); FP64 vectors
+  // direction update fused into the apply: p_cur = z + beta p_prev with beta the quotient
+  // of two sums of np_rz partials, P_rz_new / P_rz_old (p_cur = z when first); FP64 vectors
   const double* z;
   const double* p_prev;
   double* p_cur;
   int first;
-  const double* scal;
+  const double* P_rz_new;
+  const double* P_rz_old;
+  int np_rz;
   double* y;         // y = K p_cur through the FP32 operator (constrained rows: y = p_cur)
   double* partials;  // per-chunk partial of p_cur . y
   Material m;
@@ -58,9 +60,6 @@ hipError_t launch_pcgm_init(const double* r, double* z, const double* dinv, int 
                             hipStream_t s);
 // pq = sum of the n apply partials; scal[kAlpha] = scal[kRZ] / pq
 hipError_t launch_pcgm_alpha(const double* partials, int n, double* scal, hipStream_t s);
-// x += alpha p; r -= alpha q; z = Dinv r (alpha = scal[kAlpha]); partials of r.z, r.r
-hipError_t launch_pcgm_update(double* x, double* r, double* z, const double* p, const double* q, const double* dinv,
-                              int nnodes, const double* scal, double* P_rz, double* P_rr, int grid, hipStream_t s);
 // rz_new = sum P_rz; scal[kRR] = sum P_rr (when P_rr is given), then by mode:
 //   kBetaInit:    scal[kRZ] = rz_new
 //   kBetaStep:    scal[kBeta] = rz_new / scal[kRZ]; scal[kRZPrev] = scal[kRZ]; scal[kRZ] = rz_new

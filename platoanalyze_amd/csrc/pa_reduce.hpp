@@ -8,6 +8,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "pa_dpp.hpp"
 #include "pa_kernels.hpp"
 
 namespace pa {
@@ -25,12 +26,28 @@ inline int red_grid(size_t work, int per_block) {
   return (int)g;
 }
 
+// Sum over a wavefront, the same bits in every lane: DPP sums of the four 16-lane rows,
+// then the rows' values through scalar registers (no LDS crossbar: six shuffles of a double
+// were most of a small kernel's reduction time).
+__device__ __forceinline__ double wave_sum(double v) {
+  v = sum16(v);
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  double r[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, 16 * q);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), 16 * q);
+    r[q] = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+  }
+  return (r[0] + r[1]) + (r[2] + r[3]);
+}
+
 // Sum of one value per thread over the work-group, returned in every thread
-// (fixed order).  `sh` holds NT/64 doubles; safe to call repeatedly.
+// (fixed order).  `sh` holds NT/64 doubles; safe to call repeatedly.  Every lane of the
+// work-group takes part.
 template <int NT>
 __device__ __forceinline__ double block_reduce_all(double v, double* sh) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -40,12 +57,41 @@ __device__ __forceinline__ double block_reduce_all(double v, double* sh) {
   return t;
 }
 
+// Two sums at once (one pair of barriers); `sh` holds 2 NT/64 doubles.
+template <int NT>
+__device__ __forceinline__ void block_reduce_two(double& a, double& b, double* sh) {
+  a = wave_sum(a);
+  b = wave_sum(b);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = a;
+    sh[NT / 64 + (threadIdx.x >> 6)] = b;
+  }
+  __syncthreads();
+  a = b = 0.0;
+#pragma unroll
+  for (int q = 0; q < NT / 64; ++q) {
+    a += sh[q];
+    b += sh[NT / 64 + q];
+  }
+}
+
 // Fixed-order total of n partials written by an earlier kernel, in every thread.
 template <int NT>
 __device__ __forceinline__ double sum_partials_all(const double* p, int n, double* sh) {
   double v = 0.0;
   for (int i = threadIdx.x; i < n; i += NT) v += p[i];
   return block_reduce_all<NT>(v, sh);
+}
+
+// Totals of two partial arrays at once; `sh` holds 2 NT/64 doubles.
+template <int NT>
+__device__ __forceinline__ void sum_partials_two(const double* p, int np, const double* q, int nq, double* sh,
+                                                 double& a, double& b) {
+  a = b = 0.0;
+  for (int i = threadIdx.x; i < np; i += NT) a += p[i];
+  for (int i = threadIdx.x; i < nq; i += NT) b += q[i];
+  block_reduce_two<NT>(a, b, sh);
 }
 
 // Same, with four independent accumulators per thread (for long partial arrays read by

@@ -88,6 +88,71 @@ __global__ __launch_bounds__(kT) void k_pcg_spmv(const double* __restrict__ vals
   if (threadIdx.x == 0) P_pq[blockIdx.x] = t;
 }
 
+// The direction update fused into the product: p = z + beta p_prev (beta = rz_new / rz_old
+// from the partials of the last two updates; p = z when first), q = A p; per-group partial
+// of p.q.  Each row recomputes its neighbours' p, so p is written to a second buffer.  The
+// products with z and p_prev are summed apart and joined by beta afterwards, so no load
+// waits for the partial sums.  One launch less per iteration and no separate pass over
+// p and z; the row gathers two vectors instead of one, so the caller takes it where
+// launches, not gathers, set the pace.
+__global__ __launch_bounds__(kT) void k_pcg_dir_spmv(const double* __restrict__ vals, const int* __restrict__ rowmap,
+                                                     const int* __restrict__ col, const double* __restrict__ z,
+                                                     const double* __restrict__ p_prev, double* __restrict__ p,
+                                                     double* __restrict__ q, int nrows, int first,
+                                                     const double* P_rz_new, const double* P_rz_old, int np,
+                                                     double* __restrict__ P_pq) {
+  __shared__ double sh[2 * kT / 64];
+  const int lane = threadIdx.x % kLanesPerRow;
+  const XcdSpan sp = xcd_span(nrows);
+  double beta = 0.0, dot = 0.0;
+  bool have = first != 0;
+  // every thread makes the same number of trips: the reduction inside is work-group-wide
+  const int trips = (sp.hi - sp.lo + sp.bx * kRowsPerBlock - 1) / (sp.bx * kRowsPerBlock);
+  for (int k = 0; k < trips || !have; ++k) {
+    const int row = sp.lo + (k * sp.bx + sp.j) * kRowsPerBlock + (int)threadIdx.x / kLanesPerRow;
+    const bool live = row < sp.hi;
+    double az[3] = {0.0, 0.0, 0.0}, ap[3] = {0.0, 0.0, 0.0}, zi = 0.0, pi = 0.0;
+    if (live) {
+      if (lane < 3) {
+        zi = z[3 * (size_t)row + lane];
+        pi = first ? 0.0 : p_prev[3 * (size_t)row + lane];
+      }
+      const int s1 = rowmap[row + 1];
+      for (int s = rowmap[row] + lane; s < s1; s += kLanesPerRow) {
+        const size_t c = 3 * (size_t)col[s];
+        const double* v = vals + 9 * (size_t)s;
+        const double z0 = z[c], z1 = z[c + 1], z2 = z[c + 2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) az[i] += v[3 * i] * z0 + v[3 * i + 1] * z1 + v[3 * i + 2] * z2;
+        if (!first) {
+          const double p0 = p_prev[c], p1 = p_prev[c + 1], p2 = p_prev[c + 2];
+#pragma unroll
+          for (int i = 0; i < 3; ++i) ap[i] += v[3 * i] * p0 + v[3 * i + 1] * p1 + v[3 * i + 2] * p2;
+        }
+      }
+    }
+    if (!have) {
+      double a, b;
+      sum_partials_two<kT>(P_rz_new, np, P_rz_old, np, sh, a, b);
+      beta = a / b;
+      have = true;
+    }
+    double acc[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) acc[i] = sum16(first ? az[i] : fma(beta, ap[i], az[i]));
+    if (live && lane < 3) {
+      const double a = lane == 0 ? acc[0] : (lane == 1 ? acc[1] : acc[2]);
+      const double pv = first ? zi : fma(beta, pi, zi);
+      const size_t d = 3 * (size_t)row + lane;
+      p[d] = pv;
+      q[d] = a;
+      dot += pv * a;
+    }
+  }
+  const double t = block_reduce_all<kT>(dot, sh);
+  if (threadIdx.x == 0) P_pq[blockIdx.x] = t;
+}
+
 // beta = rz_new / rz_old from the partials of the last two update kernels; p = z + beta p.
 __global__ __launch_bounds__(kT) void k_pcg_pupdate(double* __restrict__ p, const double* __restrict__ z,
                                                     int nnodes, const double* P_rz_new, const double* P_rz_old,
@@ -119,9 +184,27 @@ __global__ __launch_bounds__(kT) void k_pcg_update(double* __restrict__ x, doubl
                                                    int nnodes, const double* P_pq, int np_pq, const double* P_rz,
                                                    int np, double* __restrict__ P_rz_next,
                                                    double* __restrict__ P_rr, double* __restrict__ scal) {
-  __shared__ double sh[kT / 64];
-  const double pq = sum_partials_all<kT>(P_pq, np_pq, sh);
-  const double rz = sum_partials_all<kT>(P_rz, np, sh);
+  __shared__ double sh[2 * kT / 64];
+  const XcdSpan sp = xcd_span(nnodes);
+  const int step = sp.bx * kT;
+  int n = sp.lo + sp.j * kT + threadIdx.x;
+  // the first node's vectors are on their way while the partials are summed
+  double xv[3], rv[3], pv[3], qv[3], D[9];
+  auto load = [&](int m) {
+    const size_t d = 3 * (size_t)m;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      xv[i] = x[d + i];
+      rv[i] = r[d + i];
+      pv[i] = p[d + i];
+      qv[i] = q[d + i];
+    }
+#pragma unroll
+    for (int i = 0; i < 9; ++i) D[i] = dinv[3 * d + i];
+  };
+  if (n < sp.hi) load(n);
+  double pq, rz;
+  sum_partials_two<kT>(P_pq, np_pq, P_rz, np, sh, pq, rz);
   const double alpha = rz / pq;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     scal[kPQ] = pq;
@@ -129,29 +212,29 @@ __global__ __launch_bounds__(kT) void k_pcg_update(double* __restrict__ x, doubl
     scal[kAlpha] = alpha;
   }
   double rzn = 0.0, rr = 0.0;
-  const XcdSpan sp = xcd_span(nnodes);
-  for (int n = sp.lo + sp.j * kT + threadIdx.x; n < sp.hi; n += sp.bx * kT) {
+  while (n < sp.hi) {
     const size_t d = 3 * (size_t)n;
-    double rv[3], zv[3];
+    double zv[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      x[d + i] += alpha * p[d + i];
-      rv[i] = r[d + i] - alpha * q[d + i];
+      x[d + i] = xv[i] + alpha * pv[i];
+      rv[i] -= alpha * qv[i];
       r[d + i] = rv[i];
     }
-    dinv3(dinv + 9 * (size_t)n, rv, zv);
+    dinv3(D, rv, zv);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       z[d + i] = zv[i];
       rzn += rv[i] * zv[i];
       rr += rv[i] * rv[i];
     }
+    n += step;
+    if (n < sp.hi) load(n);
   }
-  const double t0 = block_reduce_all<kT>(rzn, sh);
-  const double t1 = block_reduce_all<kT>(rr, sh);
+  block_reduce_two<kT>(rzn, rr, sh);
   if (threadIdx.x == 0) {
-    P_rz_next[blockIdx.x] = t0;
-    P_rr[blockIdx.x] = t1;
+    P_rz_next[blockIdx.x] = rzn;
+    P_rr[blockIdx.x] = rr;
   }
 }
 
@@ -197,13 +280,17 @@ __global__ __launch_bounds__(kT) void k_dot(const double* __restrict__ a, const 
   if (threadIdx.x == 0) P[blockIdx.x] = t;
 }
 
-// fixed-order sum of n partials into scal[slot] (one work-group)
-__global__ __launch_bounds__(kT) void k_sum(const double* partials, int n, double* scal, int slot) {
-  __shared__ double sh[kT / 64];
-  const double t = sum_partials_all<kT>(partials, n, sh);
-  if (threadIdx.x == 0) scal[slot] = t;
+// fixed-order sum of n partials into scal[slot] (one work-group), and into *host (pinned
+// memory the device can write, null: none): a value the host waits for then needs no copy
+// command behind the kernel
+__global__ __launch_bounds__(kSumThreads) void k_sum(const double* partials, int n, double* scal, int slot, double* host) {
+  __shared__ double sh[kSumThreads / 64];
+  const double t = sum_partials_wide<kSumThreads>(partials, n, sh);
+  if (threadIdx.x == 0) {
+    scal[slot] = t;
+    if (host) host[slot] = t;
+  }
 }
-
 
 // 3x3 block-diagonal inverse (cofactors)
 __global__ __launch_bounds__(kT) void k_diag_inv(const double* vals, const int* diag_slot, double* dinv,
@@ -275,8 +362,8 @@ __global__ __launch_bounds__(kT) void k_bc_lift(const double* vals, const int* r
 
 // applyBlockConstraints first loop, matrix part: BC row -> unit diagonal, zero
 // elsewhere; the symmetric (col,row) entries zeroed too.  16 lanes per BC dof, a lane per
-// block of its row, the partner row searched once without a data-dependent exit (its loads
-// are independent): a thread per dof walked ~15 blocks x 3 components x ~15 dependent loads
+// block of its row, the partner row searched once for all components (its column loads are
+// independent; a caller's graph may repeat a column, so every match is cleared): a thread per dof walked ~15 blocks x 3 components x ~15 dependent loads
 // and took 68-96 us whatever the size (20x10x10: 84 us).
 __global__ __launch_bounds__(kT) void k_bc_zero(double* vals, const int* rowmap, const int* col,
                                                 const int* dofs, int nbc) {
@@ -285,16 +372,16 @@ __global__ __launch_bounds__(kT) void k_bc_zero(double* vals, const int* rowmap,
     const int d = dofs[k], n = d / 3, i = d % 3;
     for (int s = rowmap[n] + lane; s < rowmap[n + 1]; s += kLanesPerRow) {
       const int c = col[s];
-      int p = -1;  // slot of block (c, n)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) vals[9 * (size_t)s + 3 * i + j] = 3 * c + j == d ? 1.0 : 0.0;
       const int t1 = rowmap[c + 1];
 #pragma unroll 4
-      for (int t = rowmap[c]; t < t1; ++t) p = col[t] == n ? t : p;
+      for (int t = rowmap[c]; t < t1; ++t)
+        if (col[t] == n) {
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const bool diag = 3 * c + j == d;
-        vals[9 * (size_t)s + 3 * i + j] = diag ? 1.0 : 0.0;
-        if (!diag && p >= 0) vals[9 * (size_t)p + 3 * j + i] = 0.0;
-      }
+          for (int j = 0; j < 3; ++j)
+            if (3 * c + j != d) vals[9 * (size_t)t + 3 * j + i] = 0.0;
+        }
     }
   }
 }

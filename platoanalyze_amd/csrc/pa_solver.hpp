@@ -20,13 +20,17 @@ __global__ void k_pcg_spmv(const double* vals, const int* rowmap, const int* col
                            int nrows, double* P_pq);
 __global__ void k_pcg_pupdate(double* p, const double* z, int nnodes, const double* P_rz_new,
                               const double* P_rz_old, int np);
+__global__ void k_pcg_dir_spmv(const double* vals, const int* rowmap, const int* col, const double* z,
+                               const double* p_prev, double* p, double* q, int nrows, int first,
+                               const double* P_rz_new, const double* P_rz_old, int np, double* P_pq);
 __global__ void k_pcg_update(double* x, double* r, double* z, const double* p, const double* q,
                              const double* dinv, int nnodes, const double* P_pq, int np_pq, const double* P_rz,
                              int np, double* P_rz_next, double* P_rr, double* scal);
 __global__ void k_pcg_init(const double* r, double* z, double* p, const double* b, const double* dinv,
                            int nnodes, double* P_rz, double* P_rr, double* P_bb);
 __global__ void k_dot(const double* a, const double* b, size_t n, double* P);
-__global__ void k_sum(const double* partials, int n, double* scal, int slot);
+constexpr int kSumThreads = 1024;
+__global__ void k_sum(const double* partials, int n, double* scal, int slot, double* host);
 __global__ void k_diag_inv(const double* vals, const int* diag_slot, double* dinv, int nnodes);
 __global__ void k_add_load(double* y, const int* nodes, const double* f, int n, double s);
 __global__ void k_fill(double* y, size_t n, double v);
