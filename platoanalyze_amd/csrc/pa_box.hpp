@@ -54,7 +54,7 @@ struct BoxArgs {
   int nx, ny, nz;          // hexes per axis
   int seg_cap;             // k_box_jac_ws: blocks of one staged tile (kBoxRows x longest row)
   Material m;
-  // k_box_res_kuhn: mesh tet index of each Kuhn path, 1 / spacing per axis, tet volume
+  // k_box_diag_inv_kuhn: mesh tet index of each Kuhn path, 1 / spacing per axis, tet volume
   int tperm[6];
   double ih[3];
   double vol;
@@ -133,13 +133,8 @@ constexpr int kKuhnPath[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2,
 // weights A.W and u at the lattice points (A.ulat); the rows sum in a fixed order.
 __global__ void k_box_res(BoxArgs A, int sub_load);
 
-// The same residual tet by tet on lattices split into the six main-diagonal Kuhn tets
-// (see k_boxmf_apply_kuhn), all in FP64: one row per lane, u at the 15 lattice points its
-// 24 tets reach (A.ulat zero on the ghost layer and one padded plane and row past the
-// end), each tet's force vol w sigma g_m added in a fixed order.
-__global__ void k_box_res_kuhn(BoxArgs A, int sub_load);
-
-// Inverted 3x3 diagonal blocks from the same Kuhn tets, in FP64: K_rr = sum over the
+// Inverted 3x3 diagonal blocks on lattices split into the six main-diagonal Kuhn tets (see
+// k_boxmf_apply_kuhn), in FP64: K_rr = sum over the
 // row's 24 tets of vol w ((lambda + mu) g g^T + mu |g|^2 I), g the row vertex's gradient.
 __global__ void k_box_diag_inv_kuhn(BoxArgs A, const uint8_t* bcmask, double* dinv);
 

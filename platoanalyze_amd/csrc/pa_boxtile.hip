@@ -1,0 +1,338 @@
+// Brick kernels of Kuhn-split box lattices (pa_boxtile.hpp).
+//
+// A work-group owns a 4x4x4 brick of lattice points.  It gathers u and z of the 6x6x6
+// points around it once (through the lattice-to-node map: no lattice copies of u and z and
+// no array of element weights), a thread computes all six tets of one of the 5x5x5 hexes
+// that touch the brick from its eight corners in registers, leaves the hex's eight corner
+// contributions in LDS, and the brick's points sum theirs from eight hexes in a fixed order.
+// A tet is evaluated 125 / 64 = 1.95 times on average; one row per lane from its 24 tets
+// evaluates it four times, reads 15 points and 24 weights a row, and needs a scatter pass
+// and a weight pass before it.  In the tet of axis path (a, b, c) the displacement
+// gradient's columns are the three edge differences over the spacings.
+//
+// What bounds it: FP64 arithmetic and the latency of the two dependent gathers (map, then
+// u and z) at ten to twelve waves a CU.
+#include "pa_boxtile.hpp"
+
+#include <type_traits>
+
+#include "pa_box.hpp"
+#include "pa_reduce.hpp"
+
+namespace pa {
+
+namespace {
+
+constexpr int kT = 128;                            // threads; 125 of them have a hex
+constexpr int kOwn = kTileNodes, kHex = kOwn + 1, kPts = kOwn + 2;
+constexpr int kHexes = kHex * kHex * kHex, kPoints = kPts * kPts * kPts;
+static_assert(kHexes <= kT, "a thread per hex");
+
+__device__ __forceinline__ double powi(double x, int n) {  // n >= 1
+  double r = 1.0;
+  for (; n > 0; n >>= 1, x *= x)
+    if (n & 1) r *= x;
+  return r;
+}
+
+// x^p: integer exponents to 16 by multiplication, 1/2 by the square root
+__device__ __forceinline__ double pow_of(double x, double p, int pint) {
+  if (pint > 0) return powi(x, pint);
+  if (p == 0.5) return sqrt(x);
+  return pow(x, p);
+}
+
+// Voigt strain (engineering shear) of tet Q of the hex with corner displacements U
+template <int Q>
+__device__ __forceinline__ void tet_strain_of(const double U[8][3], const double ih[3], double e[6]) {
+  constexpr int a = kKuhnPath[Q][0], b = kKuhnPath[Q][1], c = kKuhnPath[Q][2];
+  constexpr int v1 = 1 << a, v2 = (1 << a) | (1 << b);
+  double G[3][3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    G[i][a] = (U[v1][i] - U[0][i]) * ih[a];
+    G[i][b] = (U[v2][i] - U[v1][i]) * ih[b];
+    G[i][c] = (U[7][i] - U[v2][i]) * ih[c];
+  }
+  e[0] = G[0][0];
+  e[1] = G[1][1];
+  e[2] = G[2][2];
+  e[3] = G[1][2] + G[2][1];
+  e[4] = G[0][2] + G[2][0];
+  e[5] = G[0][1] + G[1][0];
+}
+
+__device__ __forceinline__ void stress_of(const Material& m, const double e[6], double s[6]) {
+  const double l = m.c01 * (e[0] + e[1] + e[2]), d = m.c00 - m.c01;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s[k] = fma(d, e[k], l);
+#pragma unroll
+  for (int k = 3; k < 6; ++k) s[k] = m.c33 * e[k];
+}
+
+template <int Q>
+__device__ __forceinline__ double tet_rho(const double Z[8]) {
+  constexpr int v1 = 1 << kKuhnPath[Q][0], v2 = v1 | (1 << kKuhnPath[Q][1]);
+  return (Z[0] + Z[v1] + Z[v2] + Z[7]) / 4.0;
+}
+
+// F[corner] += force of the stress k * s on the tet's vertices: edge l along axis c adds
+// k s[:, c] / h_c to its upper vertex and subtracts it from its lower one
+template <int Q>
+__device__ __forceinline__ void tet_force(const double s[6], double k, const double ih[3], double F[8][3]) {
+  constexpr int V[3][3] = {{0, 5, 4}, {5, 1, 3}, {4, 3, 2}};  // Voigt index of (i, j)
+  constexpr int a = kKuhnPath[Q][0], b = kKuhnPath[Q][1];
+  constexpr int v[4] = {0, 1 << a, (1 << a) | (1 << b), 7};
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    const int c = kKuhnPath[Q][l];
+    const double kh = k * ih[c];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const double t = kh * s[V[i][c]];
+      F[v[l + 1]][i] += t;
+      F[v[l]][i] -= t;
+    }
+  }
+}
+
+template <int Q>
+__device__ __forceinline__ void tet_scalar(double k, double F[8]) {
+  constexpr int v1 = 1 << kKuhnPath[Q][0], v2 = v1 | (1 << kKuhnPath[Q][1]);
+  F[0] += k;
+  F[v1] += k;
+  F[v2] += k;
+  F[7] += k;
+}
+
+template <int N, typename F>
+__device__ __forceinline__ void each_tet(const F& f) {
+  if constexpr (N < 6) {
+    f(std::integral_constant<int, N>{});
+    each_tet<N + 1>(f);
+  }
+}
+
+// von Mises direction t = dJ/dsigma and J = vm^2
+__device__ __forceinline__ double von_mises2(const double s[6]) {
+  const double d01 = s[0] - s[1], d12 = s[1] - s[2], d20 = s[2] - s[0];
+  return 0.5 * (d01 * d01 + d12 * d12 + d20 * d20) + 3.0 * (s[3] * s[3] + s[4] * s[4] + s[5] * s[5]);
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kT) void k_box_tile(BoxTileArgs A) {
+  constexpr bool kRes = MODE == kTileResidual, kGradZ = MODE == kTileEnergyGradZ, kPnG = MODE == kTilePNormGrad;
+  constexpr bool kAdj = MODE == kTileAdjZ, kPn = MODE == kTilePNorm || kPnG;
+  constexpr bool kVec = kRes || kPnG, kScal = kGradZ || kPnG || kAdj;  // corner vectors, corner scalars
+  constexpr bool kSum = MODE == kTileEnergy || kGradZ || MODE == kTilePNorm;
+  constexpr int kOut = (kVec ? 3 : 0) + (kScal ? 1 : 0);
+  constexpr int kStage = kPoints * (kAdj ? 7 : 4), kCorner = 8 * kOut * kT;
+  // the staged points and the corner contributions share one region (a barrier between)
+  __shared__ double sm[kStage > kCorner ? kStage : kCorner];
+  // per hex and tet: density and strain measure, then coefficients (the residual needs no
+  // strain measure: its densities start in cl)
+  __shared__ double cl[6][kT], rl_[kRes ? 1 : 6][kT];
+  auto& rl = [&]() -> auto& {
+    if constexpr (kRes) return cl;
+    else return rl_;
+  }();
+  __shared__ int ids[kPoints];
+  __shared__ double sh[kT / 64];
+
+  const int t = threadIdx.x;
+  // contiguous runs of bricks per XCD (work-group b runs on XCD b % 8)
+  const int nb = A.bx * A.by * A.bz, qd = nb / kNumXcd, rd = nb % kNumXcd, xc = blockIdx.x % kNumXcd;
+  const int brick = xc * qd + min(xc, rd) + (int)blockIdx.x / kNumXcd;
+  const int i0 = brick % A.bx * kOwn, j0 = brick / A.bx % A.by * kOwn, k0 = brick / (A.bx * A.by) * kOwn;
+  for (int p = t; p < kPoints; p += kT) {
+    const int i = i0 - 1 + p % kPts, j = j0 - 1 + p / kPts % kPts, k = k0 - 1 + p / (kPts * kPts);
+    const bool in = (unsigned)i < (unsigned)A.nx && (unsigned)j < (unsigned)A.ny && (unsigned)k < (unsigned)A.nz;
+    const int id = in ? A.node_of[i + (size_t)A.nx * (j + (size_t)A.ny * k)] : -1;
+    ids[p] = id;
+    if (id >= 0) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) sm[c * kPoints + p] = A.u[3 * (size_t)id + c];
+      sm[3 * kPoints + p] = A.z[id];
+      if constexpr (kAdj) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) sm[(4 + c) * kPoints + p] = A.u2[3 * (size_t)id + c];
+      }
+    }
+  }
+  __syncthreads();
+  // hex t: lower corner at lattice point (i0 - 1 + hx, ...)
+  const int hx = t % kHex, hy = t / kHex % kHex, hz = t / (kHex * kHex);
+  const int gi = i0 - 1 + hx, gj = j0 - 1 + hy, gk = k0 - 1 + hz;
+  const bool hex = t < kHexes && gi >= 0 && gj >= 0 && gk >= 0 && gi < A.nx - 1 && gj < A.ny - 1 && gk < A.nz - 1;
+  const int at = hx + kPts * (hy + kPts * hz);
+  double U[8][3], L[8][3], Z[8];
+  if (hex) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int p = at + (c & 1) + kPts * ((c >> 1) & 1) + kPts * kPts * (c >> 2);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        U[c][i] = sm[i * kPoints + p];
+        if constexpr (kAdj) L[c][i] = sm[(4 + i) * kPoints + p];
+      }
+      Z[c] = sm[3 * kPoints + p];
+    }
+  }
+  __syncthreads();  // sm becomes the corner contributions
+  double sum = 0.0, F[8][3], S[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) F[c][i] = 0.0;
+    S[c] = 0.0;
+  }
+  if (hex) {
+    const double ih[3] = {A.ih[0], A.ih[1], A.ih[2]};
+    // per tet: its density and the strain measure its coefficient needs
+    each_tet<0>([&](auto q) {
+      constexpr int Q = decltype(q)::value;
+      rl[Q][t] = tet_rho<Q>(Z);
+      if constexpr (!kRes) {
+        double e[6], s[6], v = 0.0;
+        tet_strain_of<Q>(U, ih, e);
+        stress_of(A.m, e, s);
+        if constexpr (kPn) {
+          if (A.measure == 0) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) v += s[k] * s[k];
+          } else {
+            v = von_mises2(s);
+          }
+        } else if constexpr (kAdj) {
+          double l[6];
+          tet_strain_of<Q>(L, ih, l);
+#pragma unroll
+          for (int k = 0; k < 6; ++k) v += s[k] * l[k];
+        } else {
+#pragma unroll
+          for (int k = 0; k < 6; ++k) v += s[k] * e[k];
+        }
+        cl[Q][t] = v;
+      }
+    });
+    // coefficients; a rolled loop, so the penalty models' and powers' code exists once
+    const int pni = (A.pn <= 16.0 && A.pn == floor(A.pn)) ? (int)A.pn : 0;
+#pragma unroll 1
+    for (int q = 0; q < 6; ++q) {
+      const double rho = rl[q][t];
+      if constexpr (kRes) {
+        cl[q][t] = A.vol * penalty_w(A.m, rho);
+      } else if constexpr (kAdj) {
+        cl[q][t] *= 0.25 * penalty_dw(A.m, rho) * A.vol;
+      } else if constexpr (!kPn) {
+        const double v = cl[q][t];
+        sum += 0.5 * A.vol * penalty_w(A.m, rho) * v;
+        if constexpr (kGradZ) cl[q][t] = A.scale * (0.125 * A.vol * v * penalty_dw(A.m, rho));
+      } else {
+        // m, with dm/du = c_u B^T C0 t and dm/drho = c_z m (t: see the forces below)
+        double mval, cu, cz;
+        if (A.measure == 0) {
+          const double w = penalty_w(A.m, rho);
+          mval = fabs(w) * sqrt(cl[q][t]);
+          cu = mval > 0.0 ? w * w / mval : 0.0;
+          cz = kPnG ? penalty_dw(A.m, rho) / w : 0.0;
+        } else {
+          const double vm0 = sqrt(cl[q][t]), rq = pow_of(rho, A.q, 0);
+          mval = rq * vm0;
+          cu = vm0 > 0.0 ? rq / (2.0 * vm0) : 0.0;
+          cz = kPnG ? A.q / rho : 0.0;
+        }
+        const double mp = pow_of(mval, A.pn, pni);
+        sum += mp * A.vol;
+        if constexpr (kPnG) {
+          const double k = A.pscale * A.vol * A.pn;
+          cl[q][t] = k * (mval > 0.0 ? mp / mval : 0.0) * cu;
+          rl[q][t] = 0.25 * k * mp * cz;
+        }
+      }
+    }
+    if constexpr (kOut > 0) {
+      each_tet<0>([&](auto q) {
+        constexpr int Q = decltype(q)::value;
+        if constexpr (kVec) {
+          double e[6], s[6];
+          tet_strain_of<Q>(U, ih, e);
+          stress_of(A.m, e, s);
+          if constexpr (kPnG) {
+            if (A.measure != 0) {  // t = dJ/dsigma; measure 0: t = sigma
+              const double tr = s[0] + s[1] + s[2];
+#pragma unroll
+              for (int k = 0; k < 3; ++k) s[k] = 3.0 * s[k] - tr;
+#pragma unroll
+              for (int k = 3; k < 6; ++k) s[k] *= 6.0;
+            }
+            double tau[6];
+            stress_of(A.m, s, tau);
+            tet_force<Q>(tau, cl[Q][t], ih, F);
+          } else {
+            tet_force<Q>(s, cl[Q][t], ih, F);
+          }
+        }
+        if constexpr (kScal) tet_scalar<Q>(kPnG ? rl[Q][t] : cl[Q][t], S);
+      });
+    }
+  }
+  if constexpr (kOut > 0) {
+    if (t < kHexes) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        if constexpr (kVec) {
+#pragma unroll
+          for (int i = 0; i < 3; ++i) sm[(kOut * c + i) * kT + t] = F[c][i];
+        }
+        if constexpr (kScal) sm[(kOut * c + kOut - 1) * kT + t] = S[c];
+      }
+    }
+    __syncthreads();
+    constexpr int kNodes = kOwn * kOwn * kOwn;
+    for (int w = t; w < kOut * kNodes; w += kT) {
+      const int n = w / kOut, o = w - kOut * n;
+      const int a = n % kOwn, b = n / kOwn % kOwn, c = n / (kOwn * kOwn);
+      const int id = ids[(a + 1) + kPts * ((b + 1) + kPts * (c + 1))];
+      if (id < 0) continue;
+      double v = 0.0;
+#pragma unroll
+      for (int cc = 0; cc < 8; ++cc) {  // the node is corner cc of hex (a + 1 - bits of cc)
+        const int hh = (a + 1 - (cc & 1)) + kHex * ((b + 1 - ((cc >> 1) & 1)) + kHex * (c + 1 - (cc >> 2)));
+        v += sm[(kOut * cc + o) * kT + hh];
+      }
+      if constexpr (kRes) {
+        const int k = A.lidx ? A.lidx[id] : -1;
+        A.out[3 * (size_t)id + o] = v - (k >= 0 ? A.load_f[3 * (size_t)k + o] : 0.0);
+      } else if constexpr (kPnG) {
+        if (o < 3) A.out[3 * (size_t)id + o] = v;
+        else A.out2[id] = v;
+      } else {
+        A.out[id] = v;
+      }
+    }
+  }
+  if constexpr (kSum) {  // every hex is summed by the brick that owns its lower corner
+    const double own = hex && hx > 0 && hy > 0 && hz > 0 ? sum : 0.0;
+    const double r = block_reduce_all<kT>(own, sh);
+    if (t == 0) A.partials[brick] = r;
+  }
+}
+
+}  // namespace
+
+hipError_t launch_box_tile(int mode, const BoxTileArgs& a, hipStream_t s) {
+  const int grid = a.bx * a.by * a.bz;
+  switch (mode) {
+    case kTileResidual: k_box_tile<kTileResidual><<<grid, kT, 0, s>>>(a); break;
+    case kTileEnergy: k_box_tile<kTileEnergy><<<grid, kT, 0, s>>>(a); break;
+    case kTileEnergyGradZ: k_box_tile<kTileEnergyGradZ><<<grid, kT, 0, s>>>(a); break;
+    case kTilePNorm: k_box_tile<kTilePNorm><<<grid, kT, 0, s>>>(a); break;
+    case kTilePNormGrad: k_box_tile<kTilePNormGrad><<<grid, kT, 0, s>>>(a); break;
+    case kTileAdjZ: k_box_tile<kTileAdjZ><<<grid, kT, 0, s>>>(a); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+}  // namespace pa

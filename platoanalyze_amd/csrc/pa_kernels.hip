@@ -201,7 +201,7 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
 #pragma unroll
         for (int q = 0; q < 6; ++q) sr += s[q] * eps[q];
         const double dw = penalty_dw(A.m, rho);
-        const double gz = 0.5 * vol * sr * dw * 0.25;
+        const double gz = A.scale * (0.5 * vol * sr * dw * 0.25);
 #pragma unroll
         for (int a = 0; a < 4; ++a)
           if (ln[a] < nr) lds_add(&res[ln[a]], gz);

@@ -134,6 +134,7 @@ struct ChunkArgs {
   // the gradients (pow(S,(1-p)/p)/p, known after the value pass)
   int measure;
   double pn, q, pscale;
+  double scale;       // factor of the energy gradient (1; -1 for the total derivative)
   Material m;
 };
 

@@ -336,10 +336,6 @@ __global__ __launch_bounds__(kT) void k_axpy(double* y, const double* x, size_t 
   for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n; i += (size_t)gridDim.x * kT) y[i] += a * x[i];
 }
 
-__global__ __launch_bounds__(kT) void k_scale(double* y, size_t n, double s) {
-  for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n; i += (size_t)gridDim.x * kT) y[i] *= s;
-}
-
 // applyBlockConstraints first loop, rhs part: rhs[col] -= A(dof,col) * value for the
 // BC rows (runs before any entry is zeroed, so each lift sees the assembled matrix).
 __global__ __launch_bounds__(kT) void k_bc_lift(const double* vals, const int* rowmap, const int* col,

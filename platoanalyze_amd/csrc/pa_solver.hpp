@@ -36,7 +36,6 @@ __global__ void k_add_load(double* y, const int* nodes, const double* f, int n, 
 __global__ void k_fill(double* y, size_t n, double v);
 // y[idx[k]] += v[k] (distinct positions)
 __global__ void k_scatter_add(double* y, const int64_t* idx, const double* v, size_t n);
-__global__ void k_scale(double* y, size_t n, double s);
 __global__ void k_axpy(double* y, const double* x, size_t n, double a);
 __global__ void k_bc_lift(const double* vals, const int* rowmap, const int* col, const int* dofs,
                           const double* bcv, int nbc, double scale, double* rhs);
