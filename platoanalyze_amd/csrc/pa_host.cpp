@@ -4,6 +4,7 @@
 #include <cmath>
 #include <functional>
 #include <numeric>
+#include <random>
 #include <thread>
 #include <unordered_map>
 
@@ -445,6 +446,14 @@ Chunks build_chunks(const Graph& g, const NodeElems& adj, const int32_t* conn, c
     }
   });
   return ch;
+}
+
+void normal_runs(unsigned long long seed, const std::vector<NormalRun>& runs, float* dst) {
+  std::mt19937_64 rng(seed);
+  for (const NormalRun& r : runs) {
+    std::normal_distribution<float> nd(0.0f, r.sigma);
+    for (size_t i = 0; i < r.count; ++i) dst[r.offset + i] = nd(rng);
+  }
 }
 
 }  // namespace pa

@@ -87,6 +87,16 @@ struct Chunks {
 Chunks build_chunks(const Graph& g, const NodeElems& ne_adj, const int32_t* conn, const std::vector<uint32_t>& codes,
                     int words_per_code, int max_blocks, int max_rows, int max_nodes);
 
+// Runs of normally distributed values from one mt19937_64 seeded with `seed`: run k fills
+// dst[offset, offset + count) with N(0, sigma).  Here and not beside its caller because the
+// host compiler of this file folds generate_canonical's long double logarithms (36 ms for
+// 1.47 million values against 61-104 ms in a HIP source, the same values to the bit).
+struct NormalRun {
+  size_t offset, count;
+  float sigma;
+};
+void normal_runs(unsigned long long seed, const std::vector<NormalRun>& runs, float* dst);
+
 // Minimal thread pool helper for setup loops.
 void parallel_for(int64_t n, const std::function<void(int64_t, int64_t)>& body);
 

@@ -155,73 +155,218 @@ __global__ __launch_bounds__(kT) void k_conv_reduce(ConvArgs A, int nslices) {
   }
 }
 
-// Weight gradient.  Work-group (split, tap x ci-tile, co-tile); each wavefront takes
-// 32-voxel K steps of its share of output voxels; fp32 results added atomically.
-constexpr int kWgradSplit = 64;
+// Weight and bias gradients of one layer.
+//
+// Every form of the convolution pairs a voxel b of a base grid with the voxels s b + d - 1
+// of a halo grid (d the tap): a direct layer's base is its output and its halo its input, a
+// transposed layer's the other way round.  So dW[tap] = sum_b Q[s b + d - 1] (x) P[b] with Q
+// the halo tensor and P the base tensor: a GEMM over voxels whose 27 taps read the same two
+// tiles.  A work-group takes 16 halo x PB base channels and a share of the tiles (a run of y
+// lines and z at one x), stages P and the three planes of Q in LDS as BF16 rows of channels
+// (dY rounded from FP32 once, its bias sums taken on the way), and each wave accumulates
+// seven taps in registers.  The MFMA operands need eight consecutive voxels per lane where
+// memory has consecutive channels: ds_read_b64_tr_b16 turns four voxel rows into columns, at
+// row addresses of any stride, so a tap is only an address offset.
+// Each work-group writes its sums to a slab; k_slab_sum adds the slabs in order, so the
+// gradient repeats to the bit.
+//
+// Before, each (tap, 16 input channels) had work-groups of its own that gathered X and dY
+// from global memory 2 and 4 bytes a lane and added with atomics: 65x33x33, batch 4, base
+// 16: 3300 us for the 15 layers and 515 us for the bias sums; now %WGRAD% us together.
+// LDS reads (one operand per two MFMAs) and the staging loads bound it.
+constexpr int kWgradBlocks = 512;   // work-groups of one layer: two per CU
+constexpr int kWgradLds = 64 * 1024;  // staged tiles, so that two work-groups share a CU
+constexpr int kQB = 16;             // halo channels of a work-group
 
-__global__ __launch_bounds__(kT) void k_wgrad(WgradArgs A) {
+struct WgradTile {
+  int ty, tz, nty, ntz, ntiles;  // base lines and z per tile, tiles per axis
+  int lq, qz, kp;                // halo lines and z per plane; base voxels padded to 32
+  int pt, slabs;                 // base channel blocks; voxel shares
+  size_t slab;                   // floats of a slab: the layer's weights and biases
+};
+
+__device__ __forceinline__ bf16x8 tr_pair(const bf16_t* lo, const bf16_t* hi) {
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s4* lds_s4;
+  const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(lo));
+  const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(hi));
+  return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+}
+
+__device__ __forceinline__ bf16x8 to_bf16x8(const float v[8]) {
+  bf16x8 r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] = (short)f2bf(v[i]);
+  return r;
+}
+
+template <int PB, bool TR>
+__global__ __launch_bounds__(kT, 2) void k_wgrad(WgradArgs A, WgradTile T) {
+  extern __shared__ char wg_lds[];
+  const int rq = 3 * T.lq * T.qz;
+  bf16_t* Pl = reinterpret_cast<bf16_t*>(wg_lds);              // [kp][PB]
+  bf16_t* Ql = Pl + T.kp * PB;                                 // [rq][kQB]
+  unsigned short* koff = reinterpret_cast<unsigned short*>(Ql + rq * kQB);  // [kp] halo row of a base voxel
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nct = (A.cin + 15) / 16;
-  const int t = blockIdx.y / nct, ci0 = (blockIdx.y % nct) * 16;
-  const int co0 = blockIdx.z * 64;
-  const int dx = t / 9, dy = (t / 3) % 3, dz = t % 3;
-  const int Vo = A.go.count(), Vi = A.gi.count();
-  const int Mtot = A.batch * Vo;
-  const int per = (Mtot + gridDim.x - 1) / gridDim.x;
-  const int ms = blockIdx.x * per, me = min(Mtot, ms + per);
-  const int ci = ci0 + (lane & 15);
-  const int kq = 8 * (lane >> 4);
-  f32x4 acc[4];
+  const int q0 = (int)blockIdx.y / T.pt * kQB, p0 = (int)blockIdx.y % T.pt * PB;
+  const Grid gb = TR ? A.gi : A.go, gq = TR ? A.go : A.gi;
+  const int cq = TR ? A.cout : A.cin, cp = TR ? A.cin : A.cout;
+  const int s = A.stride;
+  for (int k = threadIdx.x; k < T.kp; k += kT) {
+    const int y = k / T.tz, z = k - y * T.tz;
+    koff[k] = (unsigned short)(k < T.ty * T.tz ? y * s * T.qz + z * s : 0);
+  }
+  f32x4 acc[7][PB / 16];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int mb = ms + wave * 32; mb < me; mb += 4 * 32) {
-    bf16x8 a;
-    int vin[8];
+  for (int u = 0; u < 7; ++u)
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int m = mb + kq + q;
-      vin[q] = -1;
-      if (m < me) {
-        const int b = m / Vo;
-        int ox, oy, oz, vi;
-        decode(A.go, m - b * Vo, ox, oy, oz);
-        if (link(A.gi, A.stride, A.transposed, ox, oy, oz, dx, dy, dz, vi)) vin[q] = b * Vi + vi;
+    for (int j = 0; j < PB / 16; ++j) acc[u][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float bias[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) bias[i] = 0.0f;
+  const bool sum_bias = TR ? p0 == 0 : q0 == 0;
+  int tap[7];  // halo rows from a voxel's first tap
+#pragma unroll
+  for (int u = 0; u < 7; ++u) {
+    const int t = min(wave + 4 * u, 26);
+    tap[u] = (t / 9 * T.lq + t / 3 % 3) * T.qz + t % 3;
+  }
+  const int g = lane >> 4, i4 = (lane & 15) >> 2, ch = (lane & 3) * 4;
+
+  for (int tile = blockIdx.x; tile < T.ntiles; tile += gridDim.x) {
+    int r = tile;
+    const int z0 = r % T.ntz * T.tz;
+    r /= T.ntz;
+    const int y0 = r % T.nty * T.ty;
+    r /= T.nty;
+    const int bx = r % gb.nx, b = r / gb.nx;
+    __syncthreads();  // the last tile has been read
+    // base rows: 8 channels a thread
+    constexpr int kPc = PB / 8;
+    for (int e = threadIdx.x; e < T.kp * kPc; e += kT) {
+      const int k = e / kPc, c = p0 + e % kPc * 8;
+      const int y = k / T.tz, z = z0 + k - y * T.tz;
+      const bool in = k < T.ty * T.tz && y0 + y < gb.ny && z < gb.nz && c < cp;
+      const size_t v = in ? (((size_t)b * gb.nx + bx) * gb.ny + y0 + y) * gb.nz + z : 0;
+      bf16x8 w = {0, 0, 0, 0, 0, 0, 0, 0};
+      if constexpr (TR) {
+        if (in) w = *reinterpret_cast<const bf16x8*>(A.X + v * A.ldx + A.xcol + c);
+      } else if (in) {
+        float f[8];
+        *reinterpret_cast<float4*>(f) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c);
+        *reinterpret_cast<float4*>(f + 4) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c + 4);
+        w = to_bf16x8(f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) bias[i] += f[i];
       }
-      a[q] = (vin[q] >= 0 && ci < A.cin) ? (short)A.X[(size_t)vin[q] * A.ldx + A.xcol + ci] : (short)0;
+      *reinterpret_cast<bf16x8*>(Pl + k * PB + e % kPc * 8) = w;
     }
+    // halo rows: three planes of lines
+    for (int e = threadIdx.x; e < rq * 2; e += kT) {
+      const int row = e >> 1, c = q0 + (e & 1) * 8;
+      const int d = row / (T.lq * T.qz), rest = row - d * T.lq * T.qz, ly = rest / T.qz, lz = rest - ly * T.qz;
+      const int x = s * bx + d - 1, y = s * y0 + ly - 1, z = s * z0 + lz - 1;
+      const bool in = (unsigned)x < (unsigned)gq.nx && (unsigned)y < (unsigned)gq.ny && (unsigned)z < (unsigned)gq.nz &&
+                      c < cq;
+      const size_t v = in ? (((size_t)b * gq.nx + x) * gq.ny + y) * gq.nz + z : 0;
+      bf16x8 w = {0, 0, 0, 0, 0, 0, 0, 0};
+      if constexpr (!TR) {
+        if (in) w = *reinterpret_cast<const bf16x8*>(A.X + v * A.ldx + A.xcol + c);
+      } else if (in) {
+        float f[8];
+        *reinterpret_cast<float4*>(f) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c);
+        *reinterpret_cast<float4*>(f + 4) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c + 4);
+        w = to_bf16x8(f);
+        // each voxel of the halo grid belongs to one tile: the positions s b .. s b + s - 1
+        if (d >= 1 && d <= s && ly >= 1 && ly <= s * T.ty && lz >= 1 && lz <= s * T.tz) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int co = co0 + 16 * j + (lane & 15);
-      bf16x8 bv;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int m = mb + kq + q;
-        bv[q] = (m < me && co < A.cout) ? (short)f2bf(A.dY[(size_t)m * A.lddy + A.dycol + co]) : (short)0;
+          for (int i = 0; i < 8; ++i) bias[i] += f[i];
+        }
       }
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[j], 0, 0, 0);
+      *reinterpret_cast<bf16x8*>(Ql + row * kQB + (e & 1) * 8) = w;
+    }
+    __syncthreads();
+    for (int k0 = 0; k0 < T.kp; k0 += 32) {
+      // lane (g, i4): rows k0 + 8 g + i4 and + 4 of both operands
+      const int k = k0 + 8 * g + i4;
+      const bf16_t* pr = Pl + k * PB + ch;
+      const bf16_t* ql = Ql + (int)koff[k] * kQB + ch;
+      const bf16_t* qh = Ql + (int)koff[k + 4] * kQB + ch;
+      bf16x8 pb[PB / 16];
+#pragma unroll
+      for (int j = 0; j < PB / 16; ++j) pb[j] = tr_pair(pr + 16 * j, pr + 4 * PB + 16 * j);
+#pragma unroll
+      for (int u = 0; u < 7; ++u) {
+        const bf16x8 qa = tr_pair(ql + tap[u] * kQB, qh + tap[u] * kQB);
+#pragma unroll
+        for (int j = 0; j < PB / 16; ++j) acc[u][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa, pb[j], acc[u][j], 0, 0, 0);
+      }
     }
   }
-  // C rows = ci (4 (l / 16) + i), columns = co (l % 16)
+  // C rows: halo channel 4 (l / 16) + i, columns: base channel l % 16
+  float* out = A.part + (size_t)blockIdx.x * T.slab;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int co = co0 + 16 * j + (lane & 15);
-    if (co >= A.cout) continue;
+  for (int u = 0; u < 7; ++u) {
+    const int t = wave + 4 * u;
+    if (t >= 27) continue;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = ci0 + 4 * (lane >> 4) + i;
-      if (c < A.cin) atomicAdd(&A.dW[((size_t)t * A.cin + c) * A.cout + co], acc[j][i]);
+    for (int j = 0; j < PB / 16; ++j) {
+      const int p = p0 + 16 * j + (lane & 15);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int q = q0 + 4 * g + i;
+        if (q < cq && p < cp) out[((size_t)t * A.cin + (TR ? p : q)) * A.cout + (TR ? q : p)] = acc[u][j][i];
+      }
+    }
+  }
+  if (sum_bias) {  // a thread's chunk of 8 channels is fixed: sum the threads of each chunk
+    __syncthreads();
+    float* bs = reinterpret_cast<float*>(wg_lds);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bs[threadIdx.x * 8 + i] = bias[i];
+    __syncthreads();
+    constexpr int kC = TR ? 2 : PB / 8;  // chunks
+    const int c0 = TR ? q0 : p0;
+    if (threadIdx.x < kC * 8 && c0 + (int)threadIdx.x < A.cout) {
+      float v = 0.0f;
+      for (int k = threadIdx.x / 8; k < kT; k += kC) v += bs[k * 8 + threadIdx.x % 8];
+      out[(size_t)27 * A.cin * A.cout + c0 + threadIdx.x] = v;
     }
   }
 }
 
-// db[co] += sum over voxels of dY[m][co]
-__global__ __launch_bounds__(kT) void k_bias_grad(const float* dY, int ld, int col, int cout, int M, float* db) {
-  const int co = threadIdx.x % 64 + 64 * blockIdx.y;
-  const int r = threadIdx.x / 64;
-  if (co >= cout) return;
-  float s = 0.0f;
-  for (int m = blockIdx.x * 4 + r; m < M; m += gridDim.x * 4) s += dY[(size_t)m * ld + col + co];
-  atomicAdd(&db[co], s);
+// dst[e] = sum of the slabs' e-th values: 16 lanes of four values, 16 runs of slabs added in
+// parallel, then in order.
+__global__ __launch_bounds__(kT) void k_slab_sum(const float* __restrict__ part, int slabs, size_t n,
+                                                 float* __restrict__ dst) {
+  __shared__ float4 sh[16][16];
+  const int l = threadIdx.x % 16, r = threadIdx.x / 16;
+  const int per = (slabs + 15) / 16, b0 = min(slabs, r * per), b1 = min(slabs, b0 + per);
+  for (size_t e0 = blockIdx.x * (size_t)64; e0 < n; e0 += (size_t)gridDim.x * 64) {
+    const size_t e = e0 + 4 * l;  // n is a multiple of 8 (channels), and so are the offsets
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (e < n)
+      for (int b = b0; b < b1; ++b) {
+        const float4 p = *reinterpret_cast<const float4*>(part + (size_t)b * n + e);
+        v.x += p.x;
+        v.y += p.y;
+        v.z += p.z;
+        v.w += p.w;
+      }
+    sh[r][l] = v;
+    __syncthreads();
+    if (r == 0 && e < n) {
+      for (int k = 1; k < 16; ++k) {
+        const float4 p = sh[k][l];
+        v.x += p.x;
+        v.y += p.y;
+        v.z += p.z;
+        v.w += p.w;
+      }
+      *reinterpret_cast<float4*>(dst + e) = v;
+    }
+    __syncthreads();
+  }
 }
 
 __global__ __launch_bounds__(kT) void k_pack(const float* W, int cin, int cout, bf16_t* Bf, bf16_t* Bd) {
@@ -262,10 +407,6 @@ __global__ __launch_bounds__(kT) void k_mse(const float* p, const float* y, size
   if (threadIdx.x == 0) P[blockIdx.x] = t / (double)n;
 }
 
-__global__ __launch_bounds__(kT) void k_zero(float* y, size_t n) {
-  for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n; i += (size_t)gridDim.x * kT) y[i] = 0.0f;
-}
-
 int blocks_for(size_t n, int cap = 4096) {
   size_t g = (n + kT - 1) / kT;
   return (int)(g < 1 ? 1 : (g > (size_t)cap ? cap : g));
@@ -299,14 +440,54 @@ hipError_t launch_conv(const ConvArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s) {
-  const int M = a.batch * a.go.count();
-  const int split = std::max(1, std::min(kWgradSplit, M / 512));
-  dim3 grid(split, 27 * ((a.cin + 15) / 16), (a.cout + 63) / 64);
-  k_wgrad<<<grid, kT, 0, s>>>(a);
-  if (a.db) {
-    dim3 g2(std::max(1, std::min(256, M / 256)), (a.cout + 63) / 64);
-    k_bias_grad<<<g2, kT, 0, s>>>(a.dY, a.lddy, a.dycol, a.cout, M, a.db);
+  const bool tr = a.transposed != 0;
+  const Grid gb = tr ? a.gi : a.go;
+  const int cq = tr ? a.cout : a.cin, cp = tr ? a.cin : a.cout;
+  const int pb = cp > 16 ? 32 : 16;
+  WgradTile t{};
+  auto even = [](int n, int most) {  // n split evenly into runs of at most `most`
+    const int runs = (n + most - 1) / most;
+    return (n + runs - 1) / runs;
+  };
+  auto bytes = [&]() {
+    t.lq = (t.ty - 1) * a.stride + 3;
+    t.qz = (t.tz - 1) * a.stride + 3;
+    t.kp = (t.ty * t.tz + 31) / 32 * 32;
+    return (size_t)t.kp * pb * 2 + (size_t)3 * t.lq * t.qz * kQB * 2 + (size_t)t.kp * 2;
+  };
+  // z runs of at most 64, then as many lines as fit (at least one: 3 x 3 x 131 halo rows)
+  t.tz = even(gb.nz, 64);
+  t.ty = 1;
+  for (int y = 2; y <= std::min(gb.ny, 16); ++y) {
+    const int keep = t.ty;
+    t.ty = y;
+    if (bytes() > kWgradLds) {
+      t.ty = keep;
+      break;
+    }
   }
+  t.ty = even(gb.ny, t.ty);
+  const size_t lds = std::max(bytes(), (size_t)kT * 8 * sizeof(float));
+  t.nty = (gb.ny + t.ty - 1) / t.ty;
+  t.ntz = (gb.nz + t.tz - 1) / t.tz;
+  t.ntiles = a.batch * gb.nx * t.nty * t.ntz;
+  t.pt = (cp + pb - 1) / pb;
+  t.slab = (size_t)27 * a.cin * a.cout + a.cout;
+  const int by = (cq + kQB - 1) / kQB * t.pt;
+  t.slabs = (int)std::min<size_t>({(size_t)std::max(1, kWgradBlocks / by), (size_t)t.ntiles,
+                                   std::max<size_t>(1, a.part_cap / t.slab)});
+  WgradArgs w = a;
+  if (t.slabs == 1) w.part = a.dW;  // biases follow the weights in the parameter vector
+  const dim3 grid(t.slabs, by);
+  if (pb == 32) {
+    if (tr) k_wgrad<32, true><<<grid, kT, lds, s>>>(w, t);
+    else k_wgrad<32, false><<<grid, kT, lds, s>>>(w, t);
+  } else {
+    if (tr) k_wgrad<16, true><<<grid, kT, lds, s>>>(w, t);
+    else k_wgrad<16, false><<<grid, kT, lds, s>>>(w, t);
+  }
+  if (t.slabs > 1)
+    k_slab_sum<<<(int)std::min<size_t>(2048, (t.slab + 63) / 64), kT, 0, s>>>(w.part, t.slabs, t.slab, a.dW);
   return hipGetLastError();
 }
 
@@ -328,22 +509,17 @@ hipError_t launch_mse(const float* pred, const float* target, size_t n, float* d
   return hipGetLastError();
 }
 
-hipError_t launch_zero(float* y, size_t n, hipStream_t s) {
-  k_zero<<<blocks_for(n), kT, 0, s>>>(y, n);
-  return hipGetLastError();
-}
-
 }  // namespace unet
 }  // namespace pa
 
 // ------------------------------------------------------------------ network (host)
 #include <cmath>
 #include <cstring>
-#include <random>
 #include <string>
 #include <vector>
 
 #include "../../include/plato_mi355x.h"
+#include "pa_host.hpp"
 
 namespace {
 
@@ -555,7 +731,6 @@ int forward(pa_unet h) {
 }
 
 int backward(pa_unet h) {
-  PA_UHIP(h, pa::unet::launch_zero(h->G.p, h->nparams, h->stream));
   for (int k = (int)h->L.size() - 1; k >= 0; --k) {
     const Layer& l = h->L[k];
     const int bi = (int)(intptr_t)l.in.p;
@@ -577,7 +752,8 @@ int backward(pa_unet h) {
     w.dycol = dycol;
     w.cout = l.cout;
     w.dW = h->G.p + l.w_off;
-    w.db = h->G.p + l.b_off;
+    w.part = h->split.p;
+    w.part_cap = h->split.n;
     PA_UHIP(h, pa::unet::launch_wgrad(w, h->stream));
     if (k == 0) continue;  // no gradient for the network input
     pa::unet::ConvArgs a{};
@@ -672,11 +848,9 @@ int pa_unet_create(pa_unet* out, int nx, int ny, int nz, int base_channels, unsi
   }
   // He-normal weights (fan-in 27 cin), zero biases
   std::vector<float> p(h->nparams, 0.0f);
-  std::mt19937_64 rng(seed);
-  for (const Layer& l : h->L) {
-    std::normal_distribution<float> nd(0.0f, std::sqrt(2.0f / (27.0f * l.cin)));
-    for (size_t i = 0; i < (size_t)27 * l.cin * l.cout; ++i) p[l.w_off + i] = nd(rng);
-  }
+  std::vector<pa::NormalRun> runs;
+  for (const Layer& l : h->L) runs.push_back({l.w_off, (size_t)27 * l.cin * l.cout, std::sqrt(2.0f / (27.0f * l.cin))});
+  pa::normal_runs(seed, runs, p.data());
   if (hipMemcpy(h->P.p, p.data(), p.size() * sizeof(float), hipMemcpyHostToDevice) ||
       hipMemset(h->M.p, 0, h->nparams * sizeof(float)) || hipMemset(h->V.p, 0, h->nparams * sizeof(float)))
     return cleanup(ufail(nullptr, PA_ERR_HIP, "pa_unet_create: upload failed"));

@@ -51,8 +51,9 @@ struct ConvArgs {
 };
 hipError_t launch_conv(const ConvArgs& a, hipStream_t s);
 
-// dW[t][ci][co] += sum over linked (i, o) of X[i][ci] * dY[o][co]; dY fp32 (already
-// multiplied by the ReLU derivative).  dW fp32 [27][cin][cout].
+// dW[t][ci][co] = sum over linked (i, o) of X[i][ci] * dY[o][co] and, behind the weights,
+// db[co] = sum over o of dY[o][co]; dY fp32 (already multiplied by the ReLU derivative).
+// dW fp32 [27][cin][cout] then [cout].  part: part_cap floats of scratch.
 struct WgradArgs {
   const bf16_t* X;
   int ldx, xcol, cin;
@@ -62,7 +63,8 @@ struct WgradArgs {
   const float* dY;
   int lddy, dycol, cout;
   float* dW;
-  float* db;  // bias gradient (may be null): db[co] += sum_o dY[o][co]
+  float* part;
+  size_t part_cap;
 };
 hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s);
 
@@ -78,8 +80,6 @@ hipError_t launch_adam(float* w, const float* g, float* m, float* v, size_t n, f
 // Mean-squared error over n values: loss partials and gradient 2 (p - y) / n into dp.
 hipError_t launch_mse(const float* pred, const float* target, size_t n, float* dp, double* partials, int grid,
                       hipStream_t s);
-
-hipError_t launch_zero(float* y, size_t n, hipStream_t s);
 
 }  // namespace unet
 }  // namespace pa
