@@ -7,6 +7,9 @@
 //   C (16 x 16): column l % 16, rows 4 (l / 16) .. 4 (l / 16) + 3
 #include "pa_unet.hpp"
 
+#include <atomic>
+#include <type_traits>
+
 #include "pa_reduce.hpp"
 
 namespace pa {
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(kT) void k_conv(ConvArgs A, int kper) {
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + 16 * j + (lane & 15);
       bf16x8 bv = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (n < A.cout && k0 < Ktot) bv = *reinterpret_cast<const bf16x8*>(A.Bt + (size_t)n * Ktot + k0);
+      if (n < A.cout && k0 < Ktot) bv = *reinterpret_cast<const bf16x8*>(A.Bt + (size_t)n * A.ldb + k0);
       acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[j], 0, 0, 0);
     }
     ch += 32;
@@ -155,6 +158,328 @@ __global__ __launch_bounds__(kT) void k_conv_reduce(ConvArgs A, int nslices) {
   }
 }
 
+// Convolution with the input staged in LDS (every layer whose tile fits; k_conv above
+// serves the others).
+//
+// A work-group takes the output voxels of a run of y lines and z at one x, stages the input
+// lines their taps reach once as rows of channels in BF16 (FP32 gradients converted here and
+// not at each of 27 uses), and computes tiles of 16 voxels x 16 channels, up to kConvM a
+// wave, with the weights of the next kConvAhead steps on their way from L2.
+// A staged row is an odd number of 16-byte banks long, so the 16 rows of an operand read
+// spread over them and its address is one addition.  The weights are the MFMA's row operand:
+// a lane then holds four consecutive channels of one voxel and the epilogue moves 8 or 16
+// bytes a lane.
+// Transposed stride-2 links reach 1, 2, 4 or 8 of the 27 taps by the voxel's parities:
+// voxels are grouped by parity and the steps without a linked tap skipped.
+// The sums are those of k_conv to the bit: the same K steps in the same order (a skipped
+// step would have added zeros), the same slices of a split reduction, added in slice order;
+// eight waves share the slices and exchange them through LDS instead of a workspace and a
+// second kernel.
+//
+// 65x33x33, base 16, against k_conv for all layers: the forward call at batch 1 271 ->
+// 174 us, the 29 convolutions of a gradient at batch 4 1280 -> 644 us.  What is left is
+// latency: a launch has about one round of work-groups, each with its staging loads, a
+// barrier and a serial chain of at most 27 cin / 32 K steps.
+constexpr int kConvM = 4, kConvAhead = 4;
+constexpr size_t kConvLdsGoal = 80 * 1024, kConvLdsMax = 120 * 1024;
+constexpr int kConvGroups = 512;  // work-groups a launch should keep: two per CU
+
+struct ConvTile {
+  int kind;                      // 0 direct, 1 transposed stride 1, 2 transposed stride 2
+  int ty, tz, nty, ntz;          // output lines and z per tile, tiles per axis
+  int mt;                        // split: 16-voxel tiles of a work-group
+  int planes, lq, qz;            // staged planes, lines, z
+  int nch, row;                  // 8-channel chunks, bytes of a staged row
+  int ksteps, kper, nsl;         // K steps of 32, per slice, slices
+  int nty_n;                     // runs of NT channel tiles per work-group
+  int tzc;                       // z of a parity class (kind 2; else of the tile)
+  // staging strides of a thread's next chunk: rows, and those as planes, lines and z
+  int nthr, srow, sd, sl, sz;
+  unsigned div_nch, div_lq, div_qz, div_tzc;  // small_div factors
+};
+
+// a / d for a, d < 2^16 by the host's factor floor(2^32 / d) + 1 (0 for d = 1)
+__device__ __forceinline__ int small_div(int a, unsigned f) { return f ? (int)__umulhi((unsigned)a, f) : a; }
+inline unsigned small_div_factor(int d) { return d == 1 ? 0u : (unsigned)((1ull << 32) / d) + 1u; }
+
+// Eight floats to BF16, nearest even (v_cvt_pk_bf16_f32; f2bf costs seven operations each).
+__device__ __forceinline__ bf16x8 cvt_bf16x8(const float4& p, const float4& q) {
+  typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+  typedef float f8 __attribute__((ext_vector_type(8)));
+  const b8 r = __builtin_convertvector(f8{p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w}, b8);
+  return __builtin_bit_cast(bf16x8, r);
+}
+
+// Epilogue of channels n .. n + 3 of output voxel m.
+__device__ __forceinline__ void conv_epilogue4(const ConvArgs& A, size_t m, int n, f32x4 v) {
+  if (A.bias) {
+    const float4 b = *reinterpret_cast<const float4*>(A.bias + n);
+    v[0] += b.x;
+    v[1] += b.y;
+    v[2] += b.z;
+    v[3] += b.w;
+  }
+  if (A.relu) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.0f);
+  }
+  if (A.gate) {
+    const ushort4 g = *reinterpret_cast<const ushort4*>(A.gate + m * A.ldg + A.gcol + n);
+    if (!bf_pos(g.x)) v[0] = 0.0f;
+    if (!bf_pos(g.y)) v[1] = 0.0f;
+    if (!bf_pos(g.z)) v[2] = 0.0f;
+    if (!bf_pos(g.w)) v[3] = 0.0f;
+  }
+  if (A.Y) {
+    typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<b4*>(A.Y + m * A.ldy + A.ycol + n) = __builtin_convertvector(v, b4);
+  }
+  if (A.Yf) {
+    float4* d = reinterpret_cast<float4*>(A.Yf + m * A.ldyf + A.yfcol + n);
+    if (A.accumulate) {
+      const float4 o = *d;
+      *d = make_float4(o.x + v[0], o.y + v[1], o.z + v[2], o.w + v[3]);
+    } else {
+      *d = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  }
+}
+
+template <int NT, bool XF32, int SPLIT>  // SPLIT: waves sharing the slices, 0: one pass
+__global__ __launch_bounds__(SPLIT ? 64 * SPLIT : kT) void k_conv_tile(ConvArgs A, ConvTile T) {
+  extern __shared__ char cv_lds[];
+  constexpr int NTHR = SPLIT ? 64 * SPLIT : kT, kWaves = NTHR / 64;
+  const int nline = T.planes * T.lq;
+  // split sums [kWaves][mt][NT][64]; a zero operand; the staged rows; per K step and lane
+  // group: byte offset of its chunk from a voxel's row, and its tap; steps with a linked tap
+  // and how many precede a step (kind 2)
+  f32x4* red = reinterpret_cast<f32x4*>(cv_lds);
+  char* Al = cv_lds + (SPLIT ? (size_t)kWaves * T.mt * NT * 1024 : 0);
+  unsigned* kt = reinterpret_cast<unsigned*>(Al + 16 + (size_t)nline * T.qz * T.row);
+  unsigned short* ks = reinterpret_cast<unsigned short*>(kt + 4 * T.ksteps);
+  unsigned short* kn = ks + T.ksteps;
+  const int lane = threadIdx.x & 63, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int Ktot = 27 * A.cin;
+  int r = blockIdx.x;
+  const int z0 = r % T.ntz * T.tz;
+  r /= T.ntz;
+  const int y0 = r % T.nty * T.ty;
+  r /= T.nty;
+  const int ox = r % A.go.nx, b = r / A.go.nx;
+  const int s = T.kind == 0 ? A.stride : 1;
+  // the work-group's parity class and its linked taps: a parity bit links the outer taps of
+  // its axis, none the middle one
+  const int py = (int)blockIdx.z >> 1, pz = (int)blockIdx.z & 1;
+  unsigned allow = (1u << 27) - 1;
+  int nsteps = T.ksteps;
+  if (T.kind == 2) {
+    auto axis = [](int p) { return p ? 5u : 2u; };
+    const unsigned az = axis(pz), ay = axis(py), ax = axis(ox & 1);
+    const unsigned line = (ay & 1 ? az : 0) | (ay & 2 ? az << 3 : 0) | (ay & 4 ? az << 6 : 0);
+    allow = (ax & 1 ? line : 0) | (ax & 2 ? line << 9 : 0) | (ax & 4 ? line << 18 : 0);
+    // every wave counts, the first writes: the count is then known without a barrier
+    int n = 0;
+    for (int e0 = 0; e0 < T.ksteps; e0 += 64) {
+      const int e = e0 + lane;
+      const int t0 = 32 * e / A.cin, t1 = min(26, (32 * e + 31) / A.cin);
+      const bool on = e < T.ksteps && ((2u << t1) - (1u << t0)) & allow;
+      const unsigned long long m = __ballot(on);
+      const int before = n + __popcll(m & ((1ull << lane) - 1));
+      if (wave == 0 && e < T.ksteps) kn[e] = (unsigned short)before;
+      if (wave == 0 && on) ks[before] = (unsigned short)e;
+      n += __popcll(m);
+    }
+    if (threadIdx.x == 0) kn[T.ksteps] = (unsigned short)n;
+    nsteps = __builtin_amdgcn_readfirstlane(n);
+  }
+  for (int e = threadIdx.x; e < 4 * T.ksteps; e += NTHR) {
+    const int t = min(27, small_div(e, T.div_nch));  // entry e: chunk e of the 27 nch, step e / 4
+    const int dx = t / 9, dy = t / 3 % 3, dz = t % 3;
+    const int ax = T.kind == 0 ? dx : T.kind == 1 ? 2 - dx : dx == 0, ay = T.kind == 0 ? dy : T.kind == 1 ? 2 - dy : dy == 0,
+              az = T.kind == 0 ? dz : T.kind == 1 ? 2 - dz : dz == 0;
+    const int off = ((ax * T.lq + ay) * T.qz + az) * T.row + (e - t * T.nch) * 16;
+    kt[e] = t < 27 ? (unsigned)t << 27 | (unsigned)off : 27u << 27;  // past the end: no tap
+  }
+  if (threadIdx.x < 4) reinterpret_cast<int*>(Al)[threadIdx.x] = 0;
+  // Input rows, a chunk a thread, kB chunks in flight; outside the grid: zeros.  A thread's
+  // chunks are nthr apart (a multiple of nch), so its position advances by constants.
+  {
+    const int xq = T.kind == 2 ? ox >> 1 : s * ox - 1, yq = T.kind == 2 ? y0 >> 1 : s * y0 - 1,
+              zq = T.kind == 2 ? z0 >> 1 : s * z0 - 1;
+    constexpr int kB = XF32 ? 4 : 8;
+    const int rows = nline * T.qz;
+    int row = small_div(threadIdx.x, T.div_nch);
+    const int c = (int)threadIdx.x - row * T.nch;
+    int line = small_div(row, T.div_qz), z = row - line * T.qz, d = small_div(line, T.div_lq), l = line - d * T.lq;
+    if ((int)threadIdx.x >= T.nthr) row = rows;  // no chunk of its own
+    const size_t xb = (size_t)b * A.gi.count() * A.ldx + A.xcol + 8 * c;
+    while (row < rows) {
+      bf16x8 w[kB];
+      float4 f[kB][2];
+      const int row0 = row;
+#pragma unroll
+      for (int u = 0; u < kB; ++u) {
+        const int x = xq + d, y = yq + l, zz = zq + z;
+        w[u] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        f[u][0] = f[u][1] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row < rows && (unsigned)x < (unsigned)A.gi.nx && (unsigned)y < (unsigned)A.gi.ny && (unsigned)zz < (unsigned)A.gi.nz) {
+          const size_t off = xb + (size_t)((x * A.gi.ny + y) * A.gi.nz + zz) * A.ldx;
+          if constexpr (XF32) {
+            f[u][0] = *reinterpret_cast<const float4*>(A.Xf + off);
+            f[u][1] = *reinterpret_cast<const float4*>(A.Xf + off + 4);
+          } else {
+            w[u] = *reinterpret_cast<const bf16x8*>(A.X + off);
+          }
+        }
+        row += T.srow;
+        z += T.sz;
+        l += T.sl;
+        d += T.sd;
+        if (z >= T.qz) {
+          z -= T.qz;
+          ++l;
+        }
+        if (l >= T.lq) {
+          l -= T.lq;
+          ++d;
+        }
+      }
+      char* to = Al + 16 + row0 * T.row + 16 * c;
+#pragma unroll
+      for (int u = 0; u < kB; ++u)
+        if (row0 + u * T.srow < rows)
+          *reinterpret_cast<bf16x8*>(to + u * T.srow * T.row) = XF32 ? cvt_bf16x8(f[u][0], f[u][1]) : w[u];
+    }
+  }
+  __syncthreads();
+
+  const int tye = min(T.ty, A.go.ny - y0), tze = min(T.tz, A.go.nz - z0);
+  const int nyc = T.kind == 2 ? (tye - py + 1) / 2 : tye, nzc = T.kind == 2 ? (tze - pz + 1) / 2 : tze;
+  // voxel positions of the class, at most 16 kConvM a wave (split: in all)
+  const int cnt = nyc * T.tzc;
+  const int v0 = SPLIT ? 0 : 16 * kConvM * wave;
+  const int tiles = max(0, min(kConvM, (cnt - v0 + 15) / 16));
+  const char* row[kConvM];
+#pragma unroll
+  for (int j = 0; j < kConvM; ++j) {
+    const int idx = v0 + 16 * j + (lane & 15);
+    const int yy = small_div(idx, T.div_tzc), zz = idx - yy * T.tzc;
+    row[j] = Al + 16 + (idx < cnt ? (yy * s * T.qz + zz * s) * T.row : 0);
+  }
+  const bool partial = T.kind == 2 || A.cin % 32;  // a step may hold chunks without a linked tap
+  auto step = [&](int k) { return T.kind == 2 ? __builtin_amdgcn_readfirstlane((int)ks[k]) : k; };
+  for (int nt = 0; nt < T.nty_n; ++nt) {
+    const int n0 = ((int)blockIdx.y * T.nty_n + nt) * 16 * NT;
+    if (n0 >= A.cout) break;
+    unsigned wo[NT];  // channels past the last read the last one's weights; never stored
+#pragma unroll
+    for (int q = 0; q < NT; ++q) wo[q] = (unsigned)(min(n0 + 16 * q + (lane & 15), A.cout - 1) * A.ldb + 8 * g) * 2u;
+    f32x4 acc[kConvM][NT], tot[SPLIT ? 1 : kConvM][NT];
+    // steps [i, iend) of the step list into acc; the next kConvAhead steps' weights load
+    // from L2 while this run is multiplied.  The number of tiles N is a template argument and
+    // not a branch around the products: this compiler does not keep the wait states between
+    // an MFMA and a read of its result when a taken branch shortens the way between them.
+    auto run = [&](int i, int iend, auto N) {
+#pragma unroll
+      for (int j = 0; j < kConvM; ++j)
+#pragma unroll
+        for (int q = 0; q < NT; ++q) acc[j][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+      bf16x8 w[kConvAhead][NT];
+      int st[kConvAhead];
+      auto load = [&](int k, int u) {
+        st[u] = step(min(k, iend - 1));
+        const char* base = reinterpret_cast<const char*>(A.Bt) + (size_t)64 * st[u];  // wave-uniform
+#pragma unroll
+        for (int q = 0; q < NT; ++q) w[u][q] = *reinterpret_cast<const bf16x8*>(base + wo[q]);
+      };
+      auto multiply = [&](int u) {
+        const unsigned e = kt[4 * st[u] + g];
+        const int off = (int)(e & 0x7FFFFFFu);
+        const bool linked = (allow >> (e >> 27)) & 1u;
+#pragma unroll
+        for (int j = 0; j < decltype(N)::value; ++j) {
+          const char* p = row[j] + off;
+          if (partial) p = linked ? p : Al;
+          const bf16x8 x = *reinterpret_cast<const bf16x8*>(p);
+#pragma unroll
+          for (int q = 0; q < NT; ++q) acc[j][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][q], x, acc[j][q], 0, 0, 0);
+        }
+      };
+      if (i >= iend) return;
+#pragma unroll
+      for (int u = 0; u < kConvAhead; ++u) load(i + u, u);
+      for (; i + kConvAhead <= iend; i += kConvAhead) {
+#pragma unroll
+        for (int u = 0; u < kConvAhead; ++u) {
+          multiply(u);
+          load(i + kConvAhead + u, u);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kConvAhead - 1; ++u)
+        if (i + u < iend) multiply(u);
+    };
+    auto run_tiles = [&](int i, int iend) {
+      if (tiles == 4) run(i, iend, std::integral_constant<int, 4>{});
+      else if (tiles == 3) run(i, iend, std::integral_constant<int, 3>{});
+      else if (tiles == 2) run(i, iend, std::integral_constant<int, 2>{});
+      else run(i, iend, std::integral_constant<int, 1>{});
+    };
+    if constexpr (SPLIT > 0) {
+      for (int rd = 0; rd * kWaves < T.nsl; ++rd) {  // the waves take the slices in turn
+        const int slice = rd * kWaves + wave;
+        int i = min(T.ksteps, slice * T.kper), iend = min(T.ksteps, (slice + 1) * T.kper);
+        if (T.kind == 2) {
+          i = __builtin_amdgcn_readfirstlane((int)kn[i]);
+          iend = __builtin_amdgcn_readfirstlane((int)kn[iend]);
+        }
+        run_tiles(i, iend);
+        __syncthreads();  // the last round's sums have been read
+#pragma unroll
+        for (int j = 0; j < kConvM; ++j)
+          if (j < T.mt)
+#pragma unroll
+            for (int q = 0; q < NT; ++q) red[((wave * T.mt + j) * NT + q) * 64 + lane] = acc[j][q];
+        __syncthreads();
+        // wave w adds the slices of tile w in order
+        if (wave < T.mt) {
+          const int have = min(kWaves, T.nsl - kWaves * rd);
+#pragma unroll
+          for (int q = 0; q < NT; ++q)
+            for (int k = 0; k < have; ++k) {
+              const f32x4 v = red[((k * T.mt + wave) * NT + q) * 64 + lane];
+              if (rd == 0 && k == 0) tot[0][q] = v;
+              else
+#pragma unroll
+                for (int c = 0; c < 4; ++c) tot[0][q][c] += v[c];
+            }
+        }
+      }
+    } else {
+      run_tiles(0, nsteps);
+#pragma unroll
+      for (int j = 0; j < kConvM; ++j)
+#pragma unroll
+        for (int q = 0; q < NT; ++q) tot[j][q] = acc[j][q];
+    }
+#pragma unroll
+    for (int j = 0; j < (SPLIT ? 1 : kConvM); ++j) {
+      const int tile = SPLIT ? wave : j;
+      const int idx = v0 + 16 * tile + (lane & 15);
+      const int yy = small_div(idx, T.div_tzc), zz = idx - yy * T.tzc;
+      if (tile >= tiles || idx >= cnt || zz >= nzc) continue;
+      const int oy = y0 + (T.kind == 2 ? 2 * yy + py : yy), oz = z0 + (T.kind == 2 ? 2 * zz + pz : zz);
+      const size_t m = (((size_t)b * A.go.nx + ox) * A.go.ny + oy) * A.go.nz + oz;
+#pragma unroll
+      for (int q = 0; q < NT; ++q) {
+        const int n = n0 + 16 * q + 4 * g;
+        if (n < A.cout) conv_epilogue4(A, m, n, tot[j][q]);
+      }
+    }
+  }
+}
+
 // Weight and bias gradients of one layer.
 //
 // Every form of the convolution pairs a voxel b of a base grid with the voxels s b + d - 1
@@ -172,7 +497,7 @@ __global__ __launch_bounds__(kT) void k_conv_reduce(ConvArgs A, int nslices) {
 //
 // Before, each (tap, 16 input channels) had work-groups of its own that gathered X and dY
 // from global memory 2 and 4 bytes a lane and added with atomics: 65x33x33, batch 4, base
-// 16: 3300 us for the 15 layers and 515 us for the bias sums; now %WGRAD% us together.
+// 16: 3300 us for the 15 layers and 515 us for the bias sums; now 378 us and 113 us for the slab sums.
 // LDS reads (one operand per two MFMAs) and the staging loads bound it.
 constexpr int kWgradBlocks = 512;   // work-groups of one layer: two per CU
 constexpr int kWgradLds = 64 * 1024;  // staged tiles, so that two work-groups share a CU
@@ -191,13 +516,6 @@ __device__ __forceinline__ bf16x8 tr_pair(const bf16_t* lo, const bf16_t* hi) {
   const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(lo));
   const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(hi));
   return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-}
-
-__device__ __forceinline__ bf16x8 to_bf16x8(const float v[8]) {
-  bf16x8 r;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = (short)f2bf(v[i]);
-  return r;
 }
 
 template <int PB, bool TR>
@@ -255,7 +573,7 @@ __global__ __launch_bounds__(kT, 2) void k_wgrad(WgradArgs A, WgradTile T) {
         float f[8];
         *reinterpret_cast<float4*>(f) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c);
         *reinterpret_cast<float4*>(f + 4) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c + 4);
-        w = to_bf16x8(f);
+        w = cvt_bf16x8(*reinterpret_cast<float4*>(f), *reinterpret_cast<float4*>(f + 4));
 #pragma unroll
         for (int i = 0; i < 8; ++i) bias[i] += f[i];
       }
@@ -276,7 +594,7 @@ __global__ __launch_bounds__(kT, 2) void k_wgrad(WgradArgs A, WgradTile T) {
         float f[8];
         *reinterpret_cast<float4*>(f) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c);
         *reinterpret_cast<float4*>(f + 4) = *reinterpret_cast<const float4*>(A.dY + v * A.lddy + A.dycol + c + 4);
-        w = to_bf16x8(f);
+        w = cvt_bf16x8(*reinterpret_cast<float4*>(f), *reinterpret_cast<float4*>(f + 4));
         // each voxel of the halo grid belongs to one tile: the positions s b .. s b + s - 1
         if (d >= 1 && d <= s && ly >= 1 && ly <= s * T.ty && lz >= 1 && lz <= s * T.tz) {
 #pragma unroll
@@ -369,7 +687,7 @@ __global__ __launch_bounds__(kT) void k_slab_sum(const float* __restrict__ part,
   }
 }
 
-__global__ __launch_bounds__(kT) void k_pack(const float* W, int cin, int cout, bf16_t* Bf, bf16_t* Bd) {
+__global__ __launch_bounds__(kT) void k_pack(const float* W, int cin, int cout, bf16_t* Bf, int ldf, bf16_t* Bd, int ldd) {
   const size_t n = (size_t)27 * cin * cout;
   for (size_t e = blockIdx.x * (size_t)kT + threadIdx.x; e < n; e += (size_t)gridDim.x * kT) {
     const int co = (int)(e % cout);
@@ -377,8 +695,8 @@ __global__ __launch_bounds__(kT) void k_pack(const float* W, int cin, int cout, 
     const int ci = (int)(r % cin);
     const int t = (int)(r / cin);
     const bf16_t v = f2bf(W[e]);
-    if (Bf) Bf[(size_t)co * 27 * cin + (size_t)t * cin + ci] = v;
-    if (Bd) Bd[(size_t)ci * 27 * cout + (size_t)t * cout + co] = v;
+    Bf[(size_t)co * ldf + (size_t)t * cin + ci] = v;
+    Bd[(size_t)ci * ldd + (size_t)t * cout + co] = v;
   }
 }
 
@@ -414,15 +732,125 @@ int blocks_for(size_t n, int cap = 4096) {
 
 }  // namespace
 
+// n split evenly into runs of at most `most`, each a multiple of `unit`
+static int even_runs(int n, int most, int unit = 1) {
+  const int runs = (n + most - 1) / most;
+  return ((n + runs - 1) / runs + unit - 1) / unit * unit;
+}
+
+// Tile of a staged convolution (`waves` sharing the slices, 0: one pass); false when no tile
+// fits the LDS budget.
+static bool conv_tile(const ConvArgs& a, int ksteps, int kper, int nsl, int nt, int waves, ConvTile& t, size_t& lds) {
+  t.kind = a.transposed ? (a.stride == 2 ? 2 : 1) : 0;
+  const int unit = t.kind == 2 ? 2 : 1, s = t.kind == 0 ? a.stride : 1, ncls = t.kind == 2 ? 4 : 1;
+  t.nch = a.cin / 8;
+  t.row = 16 * (t.nch | 1);  // an odd number of 16-byte banks: 16 consecutive rows hit all of them
+  t.ksteps = ksteps;
+  t.kper = kper;
+  t.nsl = nsl;
+  t.planes = t.kind == 2 ? 2 : 3;
+  // 16-voxel tiles of a work-group (kind 2: of one parity class)
+  auto tiles = [&](int ty, int tz) { return t.kind == 2 ? (ty / 2 * (tz / 2) + 15) / 16 : (ty * tz + 15) / 16; };
+  auto bytes = [&]() {
+    t.lq = t.kind == 2 ? t.ty / 2 + 1 : (t.ty - 1) * s + 3;
+    t.qz = t.kind == 2 ? t.tz / 2 + 1 : (t.tz - 1) * s + 3;
+    t.mt = std::min(kConvM, tiles(t.ty, t.tz));
+    return (size_t)waves * t.mt * nt * 1024 + 16 + (size_t)t.planes * t.lq * t.qz * t.row + (size_t)16 * ksteps +
+           4 * (size_t)ksteps + 2;
+  };
+  // z runs of at most 64; shorter ones where a single line of wide channels does not fit
+  for (int most = 64; most >= 8; most /= 2) {
+    t.tz = even_runs(a.go.nz, most, unit);
+    t.ty = unit;
+    if (bytes() <= kConvLdsMax) break;
+  }
+  if (bytes() > kConvLdsMax) return false;
+  // lines: enough tiles for four waves of kConvM (or kConvM, the waves sharing the slices),
+  // while two work-groups fit a CU and the grid still covers the CUs twice
+  const int most = nsl > 1 ? kConvM : 4 * kConvM;
+  const int nb = ((a.cout + 15) / 16 + nt - 1) / nt;
+  int best = t.ty;
+  for (int y = t.ty + unit; y <= a.go.ny + unit - 1 && y <= 32; y += unit) {
+    t.ty = y;
+    const long wgs = (long)a.batch * a.go.nx * ((a.go.ny + y - 1) / y) * ((a.go.nz + t.tz - 1) / t.tz) * nb * ncls;
+    if (bytes() > kConvLdsGoal || tiles(y, t.tz) > most || wgs < kConvGroups) break;
+    best = y;
+  }
+  t.ty = even_runs(a.go.ny, best, unit);
+  lds = bytes();
+  t.nty = (a.go.ny + t.ty - 1) / t.ty;
+  t.ntz = (a.go.nz + t.tz - 1) / t.tz;
+  // channel tiles: in one work-group while the voxel tiles alone fill the chip
+  const long wgs = (long)a.batch * a.go.nx * t.nty * t.ntz * ncls;
+  t.nty_n = (int)std::max<long>(1, std::min<long>(nb, wgs * nb / 1024));
+  t.tzc = t.kind == 2 ? t.tz / 2 : t.tz;
+  t.div_nch = small_div_factor(t.nch);
+  t.div_lq = small_div_factor(t.lq);
+  t.div_qz = small_div_factor(t.qz);
+  t.div_tzc = small_div_factor(t.tzc);
+  const int threads = waves ? 64 * waves : kT;
+  t.srow = std::max(1, threads / t.nch);
+  t.nthr = t.srow * t.nch;
+  t.sz = t.srow % t.qz;
+  t.sl = t.srow / t.qz % t.lq;
+  t.sd = t.srow / t.qz / t.lq;
+  return t.nthr <= threads;
+}
+
+template <int NT, bool XF32, int SPLIT>
+static void launch_conv_tile(const ConvArgs& a, const ConvTile& t, dim3 grid, size_t lds, hipStream_t s) {
+  if (lds > 64 * 1024) {  // once per device
+    static std::atomic<unsigned long long> done{0};
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    const unsigned long long bit = 1ull << (dev & 63);
+    if (!(done.load() & bit)) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv_tile<NT, XF32, SPLIT>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kConvLdsMax);
+      done.fetch_or(bit);
+    }
+  }
+  k_conv_tile<NT, XF32, SPLIT><<<grid, SPLIT ? 64 * SPLIT : kT, lds, s>>>(a, t);
+}
+
 hipError_t launch_conv(const ConvArgs& a, hipStream_t s) {
   const int M = a.batch * a.go.count();
   const int waves = ((M + 15) / 16) * ((a.cout + 63) / 64);
   const int ksteps = (27 * a.cin + 31) / 32;
-  // slices of at least two K steps until the grid holds about kConvFillWaves waves
+  // slices of at least two K steps until 64-channel work-groups of 64 voxels would hold
+  // about kConvFillWaves waves
   int nsl = 1;
   if (a.part && waves < kConvFillWaves) {
     nsl = std::min({(kConvFillWaves + waves - 1) / waves, ksteps / 2, kConvMaxSlices});
     while (nsl > 1 && (size_t)nsl * M * a.cout > a.part_cap) --nsl;
+  }
+  int kper = ksteps;
+  if (nsl > 1) {
+    kper = (ksteps + nsl - 1) / nsl;
+    nsl = (ksteps + kper - 1) / kper;  // every slice non-empty
+  }
+  ConvTile t{};
+  size_t lds = 0;
+  // two channel tiles share an input operand where there are two; eight waves where there
+  // are slices for them
+  const int nt = a.cout > 16 && nsl == 1 ? 2 : 1, sw = nsl > 4 ? 8 : nsl > 1 ? 4 : 0;
+  if (conv_tile(a, ksteps, kper, nsl, nt, sw, t, lds)) {
+    const dim3 grid(a.batch * a.go.nx * t.nty * t.ntz, ((a.cout + 16 * nt - 1) / (16 * nt) + t.nty_n - 1) / t.nty_n,
+                    t.kind == 2 ? 4 : 1);
+    if (sw == 8) {
+      if (a.X) launch_conv_tile<1, false, 8>(a, t, grid, lds, s);
+      else launch_conv_tile<1, true, 8>(a, t, grid, lds, s);
+    } else if (sw == 4) {
+      if (a.X) launch_conv_tile<1, false, 4>(a, t, grid, lds, s);
+      else launch_conv_tile<1, true, 4>(a, t, grid, lds, s);
+    } else if (nt == 2) {
+      if (a.X) launch_conv_tile<2, false, 0>(a, t, grid, lds, s);
+      else launch_conv_tile<2, true, 0>(a, t, grid, lds, s);
+    } else {
+      if (a.X) launch_conv_tile<1, false, 0>(a, t, grid, lds, s);
+      else launch_conv_tile<1, true, 0>(a, t, grid, lds, s);
+    }
+    return hipGetLastError();
   }
   dim3 grid((M + 63) / 64, (a.cout + 63) / 64);
   if (nsl <= 1) {
@@ -430,8 +858,6 @@ hipError_t launch_conv(const ConvArgs& a, hipStream_t s) {
     else k_conv<true, false><<<grid, kT, 0, s>>>(a, ksteps);
     return hipGetLastError();
   }
-  const int kper = (ksteps + nsl - 1) / nsl;
-  nsl = (ksteps + kper - 1) / kper;  // every slice non-empty
   grid.z = nsl;
   if (a.X) k_conv<false, true><<<grid, kT, 0, s>>>(a, kper);
   else k_conv<true, true><<<grid, kT, 0, s>>>(a, kper);
@@ -445,10 +871,6 @@ hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s) {
   const int cq = tr ? a.cout : a.cin, cp = tr ? a.cin : a.cout;
   const int pb = cp > 16 ? 32 : 16;
   WgradTile t{};
-  auto even = [](int n, int most) {  // n split evenly into runs of at most `most`
-    const int runs = (n + most - 1) / most;
-    return (n + runs - 1) / runs;
-  };
   auto bytes = [&]() {
     t.lq = (t.ty - 1) * a.stride + 3;
     t.qz = (t.tz - 1) * a.stride + 3;
@@ -456,7 +878,7 @@ hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s) {
     return (size_t)t.kp * pb * 2 + (size_t)3 * t.lq * t.qz * kQB * 2 + (size_t)t.kp * 2;
   };
   // z runs of at most 64, then as many lines as fit (at least one: 3 x 3 x 131 halo rows)
-  t.tz = even(gb.nz, 64);
+  t.tz = even_runs(gb.nz, 64);
   t.ty = 1;
   for (int y = 2; y <= std::min(gb.ny, 16); ++y) {
     const int keep = t.ty;
@@ -466,7 +888,7 @@ hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s) {
       break;
     }
   }
-  t.ty = even(gb.ny, t.ty);
+  t.ty = even_runs(gb.ny, t.ty);
   const size_t lds = std::max(bytes(), (size_t)kT * 8 * sizeof(float));
   t.nty = (gb.ny + t.ty - 1) / t.ty;
   t.ntz = (gb.nz + t.tz - 1) / t.tz;
@@ -492,7 +914,7 @@ hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_pack(const float* W, int cin, int cout, bf16_t* Bfwd, bf16_t* Bdgrad, hipStream_t s) {
-  k_pack<<<blocks_for((size_t)27 * cin * cout), kT, 0, s>>>(W, cin, cout, Bfwd, Bdgrad);
+  k_pack<<<blocks_for((size_t)27 * cin * cout), kT, 0, s>>>(W, cin, cout, Bfwd, packed_row(cin), Bdgrad, packed_row(cout));
   return hipGetLastError();
 }
 
@@ -709,6 +1131,7 @@ pa::unet::ConvArgs fwd_args(pa_unet h, const Layer& l) {
   a.stride = l.stride;
   a.transposed = l.transposed;
   a.Bt = l.Bf;
+  a.ldb = pa::unet::packed_row(l.cin);
   a.cout = l.cout;
   a.bias = h->P.p + l.b_off;
   a.relu = l.relu;
@@ -767,6 +1190,7 @@ int backward(pa_unet h) {
     a.stride = l.stride;
     a.transposed = !l.transposed;
     a.Bt = l.Bd;
+    a.ldb = pa::unet::packed_row(l.cout);
     a.cout = l.cin;
     a.Yf = h->grad[bi].p;
     a.ldyf = l.in.ld;
@@ -837,14 +1261,17 @@ int pa_unet_create(pa_unet* out, int nx, int ny, int nz, int base_channels, unsi
       h->partials.alloc(1024) || hipHostMalloc(&h->host_partials, 1024 * sizeof(double)))
     return cleanup(ufail(nullptr, PA_ERR_HIP, "pa_unet_create: device allocation failed"));
   size_t nb = 0;
-  for (const Layer& l : h->L) nb += 2 * (size_t)27 * l.cin * l.cout;
-  if (h->B.alloc(nb)) return cleanup(ufail(nullptr, PA_ERR_HIP, "pa_unet_create: device allocation failed"));
+  auto fsize = [](const Layer& l) { return (size_t)l.cout * pa::unet::packed_row(l.cin); };
+  auto dsize = [](const Layer& l) { return (size_t)l.cin * pa::unet::packed_row(l.cout); };
+  for (const Layer& l : h->L) nb += fsize(l) + dsize(l);
+  // the rows' padding stays zero: the pack kernel writes the weights only
+  if (h->B.alloc(nb) || hipMemset(h->B.p, 0, nb * sizeof(bf16_t))) return cleanup(ufail(nullptr, PA_ERR_HIP, "pa_unet_create: device allocation failed"));
   size_t o = 0;
   for (Layer& l : h->L) {
     l.Bf = h->B.p + o;
-    o += (size_t)27 * l.cin * l.cout;
+    o += fsize(l);
     l.Bd = h->B.p + o;
-    o += (size_t)27 * l.cin * l.cout;
+    o += dsize(l);
   }
   // He-normal weights (fan-in 27 cin), zero biases
   std::vector<float> p(h->nparams, 0.0f);

@@ -22,9 +22,11 @@ struct Grid {
 // with the link
 //   direct:     i = s*o + d - 1     (per axis, d in {0,1,2}; stride s; zero padding)
 //   transposed: o = s*i + d - 1     (i = (o + 1 - d) / s when that is an integer)
-// B-operand layout Bt[n][27*K] (n = output channel, K input channels, tap-major rows).
+// B-operand layout Bt[n][packed_row(K)] (n = output channel, K input channels): tap-major rows
+// of 27*K values and zeros up to a multiple of 32, so that the last K step reads whole.
 // The same kernel computes data gradients: the gradient of a direct conv is the
 // transposed one with Bt built from W_t^T, and vice versa.
+inline int packed_row(int cin) { return (27 * cin + 31) / 32 * 32; }
 struct ConvArgs {
   const bf16_t* X;   // input activations (bf16), row stride ldx
   const float* Xf;   // or FP32 input (converted to bf16 on load) when X == nullptr
@@ -32,7 +34,8 @@ struct ConvArgs {
   Grid gi, go;
   int batch;
   int stride, transposed;
-  const bf16_t* Bt;  // [cout][27*cin]
+  const bf16_t* Bt;  // [cout][ldb], ldb = packed_row(cin)
+  int ldb;
   int cout;
   const float* bias;  // may be null
   int relu;           // apply max(0, .)
@@ -68,7 +71,8 @@ struct WgradArgs {
 };
 hipError_t launch_wgrad(const WgradArgs& a, hipStream_t s);
 
-// Pack FP32 W[27][cin][cout] into bf16 B operands: fwd Bt[co][t][ci] and dgrad
+// Pack FP32 W[27][cin][cout] into bf16 B operands (rows of packed_row values, whose padding
+// the caller has zeroed): fwd Bt[co][t][ci] and dgrad
 // Bd[ci][t][co] (W_t^T, same tap: the data gradient of a direct conv is the transposed
 // link with the same t, and the other way round).
 hipError_t launch_pack(const float* W, int cin, int cout, bf16_t* Bfwd, bf16_t* Bdgrad, hipStream_t s);
