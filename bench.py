@@ -242,15 +242,12 @@ def main() -> int:
 
     box = C.c_int(0)
     _capi.call("pa_box_assembly", h, C.byref(box))
-    # the library takes k_box_jac_ws_ahead when the lattice weights and u (72 B per padded
-    # hex) exceed 256 MB, unless PA_BOX_AHEAD says otherwise
-    c = w.cfg
-    ahead = 72 * (c.nx + 2) * (c.ny + 2) * (c.nz + 2) > (256 << 20)
-    if os.environ.get("PA_BOX_AHEAD"):
-        ahead = os.environ["PA_BOX_AHEAD"] != "0"
+    # build_box meshes are Kuhn-split; PA_BOX_AHEAD, PA_BOX_WS and PA_BOX_JAC_KUHN=0 select the
+    # general lattice kernels
+    general = any(os.environ.get(v) is not None for v in ("PA_BOX_AHEAD", "PA_BOX_WS")) or os.environ.get("PA_BOX_JAC_KUHN") == "0"
     kernel_name = ("k_jac_chunk<4,true> (Jacobian+residual)" if not box.value else
-                   "k_box_scatter + k_box_w + k_box_jac_ws_ahead<true> + k_add_load (lattice Jacobian+residual)"
-                   if ahead else "k_box_scatter + k_box_w + k_box_jac_ws<true> (lattice Jacobian+residual)")
+                   "k_box_scatter + k_box_w + k_box_jac* (general lattice Jacobian+residual)" if general else
+                   "k_box_jac_kuhn<true> (lattice Jacobian+residual)")
 
     def timed(fn, steps, warmup):
         for _ in range(warmup):

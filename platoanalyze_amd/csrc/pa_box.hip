@@ -89,10 +89,6 @@ template __global__ void k_box_w<false, float>(BoxArgs, float*);
 // over tiles within their XCD's range (a persistent grid: the block table and the lane
 // constants are loaded once per work-group).
 
-// Work-group barrier for LDS hand-offs only: waits for this wave's LDS operations, not
-// for its outstanding global stores.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Sums of 12 values over each aligned 8-lane group, scattered: lane j (0..7) receives
 // the group sums of value indices rs_first(j) (in s0) and, for even j, rs_first(j) + 1
 // (in s1).  Three DPP exchanges, each pairing a lane with the partner holding the

@@ -60,6 +60,10 @@ struct BoxArgs {
   double vol;
 };
 
+// Work-group barrier for LDS hand-offs only: waits for this wave's LDS operations, not
+// for its outstanding global stores.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // z (and u when ulat is set) of every node at its padded lattice position (one thread
 // per node: coalesced reads, scattered writes).
 __global__ void k_box_scatter(BoxArgs A);

@@ -17,6 +17,7 @@
 #include "../../include/plato_mi355x.h"
 #include "pa_host.hpp"
 #include "pa_box.hpp"
+#include "pa_boxjac.hpp"
 #include "pa_boxtile.hpp"
 #include "pa_deflate.hpp"
 #include "pa_kernels.hpp"
@@ -222,6 +223,7 @@ struct pa_problem {
   DevArray<double> box_tile_part;
   int box_tperm[6] = {0, 0, 0, 0, 0, 0};
   double box_step[3] = {0.0, 0.0, 0.0};
+  DevArray<pa::JacTile> box_jac;  // row tiles of k_box_jac_kuhn; none: the general lattice kernels
   // k_box_jac_ws (store and compute waves specialised; PA_BOX_WS=0 selects k_box_jac)
   bool box_ws = true;
   int box_seg_cap = 0, box_grid_ws = 512;
@@ -1381,6 +1383,7 @@ static void host_tet_gradients(const double x[4][3], double g[4][3], double& vol
 // PA_BOX_ASSEMBLY=0 keeps the general chunk kernel.
 static int box_fast_setup(pa_handle h) {
   h->box_fast = false;
+  h->box_jac.release();
   if (const char* e = std::getenv("PA_BOX_ASSEMBLY"))
     if (std::atoi(e) == 0) return PA_OK;
   const pa::BoxDims d = h->box;
@@ -1617,6 +1620,16 @@ static int box_fast_setup(pa_handle h) {
       PA_HIP(h->box_tile_part.alloc((size_t)pa::tile_bricks(d.nx) * pa::tile_bricks(d.ny) * pa::tile_bricks(d.nz)));
     }
     for (int k = 0; k < 3; ++k) h->box_step[k] = step[k];
+    // PA_BOX_WS and PA_BOX_AHEAD name a general kernel
+    bool jac = kuhn && !std::getenv("PA_BOX_WS") && !std::getenv("PA_BOX_AHEAD");
+    const char* e = std::getenv("PA_BOX_JAC_KUHN");
+    if (e && std::atoi(e) == 0) jac = false;
+    if (jac) {
+      const std::vector<pa::JacTile> tiles = pa::box_jac_tiles(gpack, g.rowmap.data());
+      if (e || tiles.size() <= (size_t)pa::kJacRound || tiles.size() * pa::kJacMinRows <= (size_t)h->nn)
+        PA_HIP(h->box_jac.upload(tiles));
+      if (h->box_jac.n && !h->box_res_kuhn) PA_HIP(h->box_node_of.upload(nog));
+    }
   }
   h->box_fast = true;
   return PA_OK;
@@ -1678,6 +1691,32 @@ static void box_weights(pa_handle h, const pa::BoxArgs& a, T* W) {
 
 // K (and R = K u - f) on the lattice: element weights, then the rows.
 static int box_jacobian(pa_handle h, const double* u, const double* z, double* vals, double* R) {
+  if (h->box_jac.n) {
+    pa::BoxJacArgs j{};
+    j.tiles = h->box_jac.p;
+    j.ntiles = (int)h->box_jac.n;
+    j.node_of = h->box_node_of.p;
+    j.rowmap = h->rowmap.p;
+    j.gpack = h->box_gpack.p;
+    j.perm = h->box_perm.p;
+    j.z = z;
+    j.u = u;
+    j.lidx = h->box_lidx.p;
+    j.load_f = h->load_f.p;
+    j.vals = vals;
+    j.R = R;
+    j.nx = h->box.nx;
+    j.ny = h->box.ny;
+    j.nz = h->box.nz;
+    j.vol = h->box_step[0] * h->box_step[1] * h->box_step[2] / 6.0;
+    j.m = h->material();
+    j.lam = j.m.c01;
+    j.mu = j.m.c33;
+    for (int a = 0; a < 3; ++a)
+      for (int b = 0; b < 3; ++b) j.h[a][b] = 1.0 / (h->box_step[a] * h->box_step[b]);
+    PA_HIP(pa::launch_box_jac_kuhn(j, h->stream));
+    return PA_OK;
+  }
   const pa::BoxArgs a = box_args(h, u, z, vals, R);
   box_weights(h, a, a.W);
   const int nblk = (h->nn + pa::kBoxRows - 1) / pa::kBoxRows;
