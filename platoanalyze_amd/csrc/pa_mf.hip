@@ -256,20 +256,12 @@ __global__ __launch_bounds__(kFin) void k_pcgm_alpha(const double* partials, int
   }
 }
 
-__global__ __launch_bounds__(kFin) void k_pcgm_beta(const double* P_rz, const double* P_rr, int n, double* scal,
-                                                    int mode) {
+__global__ __launch_bounds__(kFin) void k_pcgm_beta(const double* P_rz, int n, double* scal, int mode) {
   __shared__ double sh[kFin / 64];
   const double rz = sum_partials_wide<kFin>(P_rz, n, sh);
-  const double rr = P_rr ? sum_partials_wide<kFin>(P_rr, n, sh) : 0.0;
   if (threadIdx.x == 0) {
-    if (mode == kBetaStep) {
-      scal[kBeta] = rz / scal[kRZ];
-      scal[kRZPrev] = scal[kRZ];
-    } else if (mode == kBetaReplace) {
-      scal[kBeta] = rz / scal[kRZPrev];
-    }
+    if (mode == kBetaStep) scal[kBeta] = rz / scal[kRZ];
     scal[kRZ] = rz;
-    if (P_rr) scal[kRR] = rr;
   }
 }
 
@@ -341,8 +333,8 @@ hipError_t launch_pcgm_alpha(const double* partials, int n, double* scal, hipStr
   k_pcgm_alpha<<<1, kFin, 0, s>>>(partials, n, scal);
   return hipGetLastError();
 }
-hipError_t launch_pcgm_beta(const double* P_rz, const double* P_rr, int n, double* scal, int mode, hipStream_t s) {
-  k_pcgm_beta<<<1, kFin, 0, s>>>(P_rz, P_rr, n, scal, mode);
+hipError_t launch_pcgm_beta(const double* P_rz, int n, double* scal, int mode, hipStream_t s) {
+  k_pcgm_beta<<<1, kFin, 0, s>>>(P_rz, n, scal, mode);
   return hipGetLastError();
 }
 hipError_t launch_neg_mask(const double* R, const double* b, const uint8_t* bcmask, double* r, int nn, double* P,

@@ -60,13 +60,11 @@ hipError_t launch_pcgm_init(const double* r, double* z, const double* dinv, int 
                             hipStream_t s);
 // pq = sum of the n apply partials; scal[kAlpha] = scal[kRZ] / pq
 hipError_t launch_pcgm_alpha(const double* partials, int n, double* scal, hipStream_t s);
-// rz_new = sum P_rz; scal[kRR] = sum P_rr (when P_rr is given), then by mode:
+// rz_new = sum P_rz, then by mode:
 //   kBetaInit:    scal[kRZ] = rz_new
-//   kBetaStep:    scal[kBeta] = rz_new / scal[kRZ]; scal[kRZPrev] = scal[kRZ]; scal[kRZ] = rz_new
-//   kBetaReplace: scal[kBeta] = rz_new / scal[kRZPrev]; scal[kRZ] = rz_new  (rz_new of a
-//                 replaced residual)
-enum BetaMode { kBetaStep = 0, kBetaInit = 1, kBetaReplace = 2 };
-hipError_t launch_pcgm_beta(const double* P_rz, const double* P_rr, int n, double* scal, int mode, hipStream_t s);
+//   kBetaStep:    scal[kBeta] = rz_new / scal[kRZ]; scal[kRZ] = rz_new
+enum BetaMode { kBetaStep = 0, kBetaInit = 1 };
+hipError_t launch_pcgm_beta(const double* P_rz, int n, double* scal, int mode, hipStream_t s);
 // r = mask(b - R) with b optional (R = K u - f from the residual kernel, or K u);
 // partials of ||r||^2 into P, one per work-group of `grid`
 hipError_t launch_neg_mask(const double* R, const double* b, const uint8_t* bcmask, double* r, int nnodes, double* P,
