@@ -889,7 +889,8 @@ __global__ __launch_bounds__(256, 6) void k_boxmf_apply(BoxMfArgs A) {
 // of a hex from slot q of its record; each tet's force is formed in FP32 from FP32 p and
 // weights, summed in FP32 over the four tets of each path and in FP64 over the paths, in
 // a fixed order.
-__global__ __launch_bounds__(256) void k_boxmf_apply_kuhn(BoxMfArgs A) {
+template <int OUT>
+__global__ __launch_bounds__(256, 4) void k_boxmf_apply_kuhn(BoxMfArgs A) {
   __shared__ double sh[4];
   const int px = A.nx + 2, pxy = (A.nx + 2) * (A.ny + 2);
   const float ih[3] = {A.ih[0], A.ih[1], A.ih[2]};
@@ -971,22 +972,49 @@ __global__ __launch_bounds__(256) void k_boxmf_apply_kuhn(BoxMfArgs A) {
       for (int i = 0; i < 3; ++i) y[i] += (double)yq[i];
     }
     const uint32_t bm = A.bcmask[row];
-    // constrained rows: y = p there, which is 0 (masked); the p.y partial from the FP32 p
-    // the operator acts on (its rounding moves p.y by ~1e-7 relative, below the operator's
-    // own FP32 error), so the FP64 p is not read
-    const float3 pr = P[1][1][1];
-    const double pf[3] = {pr.x, pr.y, pr.z};
+    const size_t o = 3 * (size_t)row;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const size_t dd = 3 * (size_t)row + i;
-      const double yv = (bm >> i) & 1u ? 0.0 : y[i];
-      A.y[dd] = yv;
-      dot += pf[i] * yv;
+    for (int i = 0; i < 3; ++i)
+      if ((bm >> i) & 1u) y[i] = 0.0;
+    if constexpr (OUT == kMfProduct || OUT == kMfDot) {
+      // constrained rows: y = p there, which is 0 (masked); the p.y partial from the FP32 p
+      // the operator acts on (its rounding moves p.y by ~1e-7 relative, below the operator's
+      // own FP32 error), so the FP64 p is not read, unless the caller wants it
+      const float3 pr = P[1][1][1];
+      const double pf[3] = {pr.x, pr.y, pr.z};
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        A.y[o + i] = y[i];
+        dot += (OUT == kMfDot ? A.p[o + i] : pf[i]) * y[i];
+      }
+    } else if constexpr (OUT == kMfResidual) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) A.y[o + i] = A.r[o + i] - y[i];
+    } else {
+      const double* D = A.dinv + 3 * o;
+      double rv[3], t[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        rv[i] = A.r[o + i];
+        t[i] = rv[i] - y[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const double xv = A.x[o + i] + A.inv_theta * (D[3 * i] * t[0] + D[3 * i + 1] * t[1] + D[3 * i + 2] * t[2]);
+        A.x[o + i] = xv;
+        dot += rv[i] * xv;
+      }
     }
   }
-  const double t = block_reduce_all<256>(dot, sh);
-  if (threadIdx.x == 0) A.partials[blockIdx.x] = t;
+  if constexpr (OUT != kMfResidual) {
+    const double t = block_reduce_all<256>(dot, sh);
+    if (threadIdx.x == 0) A.partials[blockIdx.x] = t;
+  }
 }
+template __global__ void k_boxmf_apply_kuhn<kMfProduct>(BoxMfArgs);
+template __global__ void k_boxmf_apply_kuhn<kMfDot>(BoxMfArgs);
+template __global__ void k_boxmf_apply_kuhn<kMfResidual>(BoxMfArgs);
+template __global__ void k_boxmf_apply_kuhn<kMfJacobi>(BoxMfArgs);
 
 __global__ __launch_bounds__(256) void k_box_diag_inv_kuhn(BoxArgs A, const uint8_t* bcmask, double* dinv) {
   const int px = A.nx + 2, pxy = (A.nx + 2) * (A.ny + 2);

@@ -127,7 +127,20 @@ struct BoxMfArgs {
   // constants
   float ih[3];
   float vol, lam, mu;
+  // epilogue of k_boxmf_apply_kuhn (BoxMfOut), FP64 vectors in node order
+  const double* r;
+  const double* dinv;      // [node][9]
+  double inv_theta;
+  double* x;
+  const double* p;
 };
+
+// What k_boxmf_apply_kuhn does with a row of K p (0 in constrained dofs):
+//   kMfProduct:  y = K p; partials of p.y, from the FP32 p
+//   kMfDot:      y = K p; partials of p.y, from the FP64 p
+//   kMfResidual: y = r - K p
+//   kMfJacobi:   x += inv_theta D^-1 (r - K p); partials of r.x  (p the FP32 copy of x)
+enum BoxMfOut { kMfProduct = 0, kMfDot = 1, kMfResidual = 2, kMfJacobi = 3 };
 
 // The six tets of a hex split along its main diagonal: tet q visits corners 0,
 // e_a, e_a + e_b, e_a + e_b + e_c for the axis path (a, b, c) = kKuhnPath[q].
@@ -161,6 +174,7 @@ __global__ void k_boxmf_apply(BoxMfArgs A);
 // vol w sigma g_m with g_m = e_{path[m-1]} / h - e_{path[m]} / h (terms present for
 // 0 < m and m < 3).  No block tables; the lattice p must be zero on the ghost layer.
 // Persistent XCD-contiguous grid over the rows, one p.y partial per work-group.
+template <int OUT>
 __global__ void k_boxmf_apply_kuhn(BoxMfArgs A);
 
 }  // namespace pa

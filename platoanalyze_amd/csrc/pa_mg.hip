@@ -7,6 +7,7 @@
 
 #include <algorithm>
 
+#include "pa_dpp.hpp"
 #include "pa_reduce.hpp"
 #include "pa_solver.hpp"
 #include "pa_spmv.hpp"
@@ -28,45 +29,59 @@ __device__ __forceinline__ void dinv3(const double* __restrict__ D, const double
   z[2] = D[6] * r[0] + D[7] * r[1] + D[8] * r[2];
 }
 
+__device__ __forceinline__ void put_lattice(const MgLattice& L, int n, const double v[3]) {
+  const int g = L.gpack[n];
+  const uint32_t bm = L.bcmask[n];
+  L.plat[((g & 1023) + 1) + (size_t)L.px * ((((g >> 10) & 1023) + 1) + (size_t)L.py * ((g >> 20) + 1))] = make_float4(
+      (bm & 1u) ? 0.0f : (float)v[0], (bm & 2u) ? 0.0f : (float)v[1], (bm & 4u) ? 0.0f : (float)v[2], 0.0f);
+}
+
+// 8 lanes per coarse node, lane q the fine points q, q + 8, .. of its 27: two dependent
+// gathers, so lanes in flight bound it.  One thread per node took 23.4 us for 128x64x64 ->
+// 64x32x32 and 11.5, 10.1 and 7.7 us for the next three; now 12.0, 4.9, 4.6 and 4.4 us.
 __global__ __launch_bounds__(kT) void k_mg_restrict(const double* __restrict__ rf, double* __restrict__ rc,
                                                     const int32_t* __restrict__ cgrid,
                                                     const int32_t* __restrict__ fnode, BoxDims fd,
                                                     const uint8_t* __restrict__ cbc, int ncn,
                                                     const double* __restrict__ cdinv, double inv_theta,
                                                     double* __restrict__ cx, double* __restrict__ cd) {
-  for (int c = blockIdx.x * kT + threadIdx.x; c < ncn; c += gridDim.x * kT) {
+  const int q = threadIdx.x % 8;
+  for (int c = (blockIdx.x * kT + threadIdx.x) / 8; c < ncn; c += gridDim.x * (kT / 8)) {
     const int I = cgrid[3 * c], J = cgrid[3 * c + 1], K = cgrid[3 * c + 2];
-    // branch-free over the 27 fine points: one outside the fine grid reads the coarse
-    // node's own fine point with weight 0 (adds an exact zero), so all lookups issue at once
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-#pragma unroll
-    for (int a = -1; a <= 1; ++a)
-#pragma unroll
-      for (int b = -1; b <= 1; ++b)
-#pragma unroll
-        for (int e = -1; e <= 1; ++e) {
-          const int i = 2 * I + a, j = 2 * J + b, k = 2 * K + e;
-          const bool in = (unsigned)i < (unsigned)fd.nx && (unsigned)j < (unsigned)fd.ny && (unsigned)k < (unsigned)fd.nz;
-          const double w = in ? (a ? 0.5 : 1.0) * (b ? 0.5 : 1.0) * (e ? 0.5 : 1.0) : 0.0;
-          const size_t f = 3 * (size_t)fnode[((size_t)(in ? i : 2 * I) * fd.ny + (in ? j : 2 * J)) * fd.nz +
-                                             (in ? k : 2 * K)];
-          s0 += w * rf[f];
-          s1 += w * rf[f + 1];
-          s2 += w * rf[f + 2];
-        }
-    const uint32_t bm = cbc[c];
-    const double v[3] = {(bm & 1u) ? 0.0 : s0, (bm & 2u) ? 0.0 : s1, (bm & 4u) ? 0.0 : s2};
     const size_t o = 3 * (size_t)c;
-    rc[o] = v[0];
-    rc[o + 1] = v[1];
-    rc[o + 2] = v[2];
-    if (cx) {
-      double z[3];
-      dinv3(cdinv + 9 * (size_t)c, v, z);
+    double D[3] = {0.0, 0.0, 0.0};  // lane i < 3: row i of the node's block
+    if (cx && q < 3) {
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        cx[o + i] = inv_theta * z[i];
-        cd[o + i] = inv_theta * z[i];
+      for (int i = 0; i < 3; ++i) D[i] = cdinv[3 * o + 3 * q + i];
+    }
+    const uint32_t bm = cbc[c];
+    // branch-free: a point outside the fine grid (or past the 27) reads the coarse node's own
+    // fine point with weight 0 (adds an exact zero), so all lookups issue at once
+    double s[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int pt = q + 8 * m;
+      const int a = pt / 9 - 1, b = pt / 3 % 3 - 1, e = pt % 3 - 1;
+      const int i = 2 * I + a, j = 2 * J + b, k = 2 * K + e;
+      const bool in = pt < 27 && (unsigned)i < (unsigned)fd.nx && (unsigned)j < (unsigned)fd.ny && (unsigned)k < (unsigned)fd.nz;
+      const double w = in ? (a ? 0.5 : 1.0) * (b ? 0.5 : 1.0) * (e ? 0.5 : 1.0) : 0.0;
+      const size_t f = 3 * (size_t)fnode[((size_t)(in ? i : 2 * I) * fd.ny + (in ? j : 2 * J)) * fd.nz + (in ? k : 2 * K)];
+#pragma unroll
+      for (int l = 0; l < 3; ++l) s[l] += w * rf[f + l];
+    }
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {  // every lane of the eight receives the sums
+      s[l] += dpp_f64<kDppXor1>(s[l]);
+      s[l] += dpp_f64<kDppXor2>(s[l]);
+      s[l] += dpp_f64<kDppHalfMirror>(s[l]);
+      if ((bm >> l) & 1u) s[l] = 0.0;
+    }
+    if (q < 3) {
+      rc[o + q] = q == 0 ? s[0] : q == 1 ? s[1] : s[2];
+      if (cx) {
+        const double z = inv_theta * (D[0] * s[0] + D[1] * s[1] + D[2] * s[2]);
+        cx[o + q] = z;
+        cd[o + q] = z;
       }
     }
   }
@@ -75,7 +90,7 @@ __global__ __launch_bounds__(kT) void k_mg_restrict(const double* __restrict__ r
 __global__ __launch_bounds__(kT) void k_mg_prolong_add(const double* __restrict__ ec, double* __restrict__ xf,
                                                        const int32_t* __restrict__ fgrid,
                                                        const int32_t* __restrict__ cnode, BoxDims cd,
-                                                       const uint8_t* __restrict__ fbc, int nfn) {
+                                                       const uint8_t* __restrict__ fbc, int nfn, MgLattice lat) {
   for (int n = blockIdx.x * kT + threadIdx.x; n < nfn; n += gridDim.x * kT) {
     const int i = fgrid[3 * n], j = fgrid[3 * n + 1], k = fgrid[3 * n + 2];
     const int I0 = i >> 1, J0 = j >> 1, K0 = k >> 1;
@@ -100,9 +115,11 @@ __global__ __launch_bounds__(kT) void k_mg_prolong_add(const double* __restrict_
         }
     const uint32_t bm = fbc[n];
     const size_t d = 3 * (size_t)n;
-    if (!(bm & 1u)) xf[d] += s0;
-    if (!(bm & 2u)) xf[d + 1] += s1;
-    if (!(bm & 4u)) xf[d + 2] += s2;
+    const double v[3] = {xf[d] + ((bm & 1u) ? 0.0 : s0), xf[d + 1] + ((bm & 2u) ? 0.0 : s1),
+                         xf[d + 2] + ((bm & 4u) ? 0.0 : s2)};
+#pragma unroll
+    for (int l = 0; l < 3; ++l) xf[d + l] = v[l];
+    if (lat.plat) put_lattice(lat, n, v);
   }
 }
 
@@ -137,7 +154,8 @@ __global__ __launch_bounds__(kT) void k_simp_w(const double* z, double* w, int n
 
 __global__ __launch_bounds__(kT) void k_cheb_first(double* __restrict__ x, double* __restrict__ d,
                                                    const double* __restrict__ r, const double* __restrict__ dinv,
-                                                   double inv_theta, int nn, const double* __restrict__ t) {
+                                                   double inv_theta, int nn, const double* __restrict__ t,
+                                                   MgLattice lat) {
   for (int n = blockIdx.x * kT + threadIdx.x; n < nn; n += gridDim.x * kT) {
     const size_t o = 3 * (size_t)n;
     double rv[3] = {r[o], r[o + 1], r[o + 2]};
@@ -149,10 +167,11 @@ __global__ __launch_bounds__(kT) void k_cheb_first(double* __restrict__ x, doubl
     dinv3(dinv + 9 * (size_t)n, rv, zv);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      const double v = inv_theta * zv[i];
-      if (d) d[o + i] = v;
-      x[o + i] = v;
+      zv[i] *= inv_theta;
+      if (d) d[o + i] = zv[i];
+      x[o + i] = zv[i];
     }
+    if (lat.plat) put_lattice(lat, n, zv);
   }
 }
 
@@ -198,21 +217,33 @@ __global__ __launch_bounds__(kT) void k_dense_gemv(const double* __restrict__ A,
   }
 }
 
+// x += alpha p, r -= alpha q, partials of r.r; with z also the V-cycle's start
+// z = inv_theta D^-1 r and its lattice copy, while r is at hand
 __global__ __launch_bounds__(kT) void k_mg_update(double* __restrict__ x, double* __restrict__ r,
                                                   const double* __restrict__ p, const double* __restrict__ q,
-                                                  const double* __restrict__ scal, int nn, double* __restrict__ P_rr) {
+                                                  const double* __restrict__ scal, int nn, double* __restrict__ P_rr,
+                                                  double* __restrict__ z, const double* __restrict__ dinv,
+                                                  double inv_theta, MgLattice lat) {
   __shared__ double sh[kT / 64];
   const double alpha = scal[kAlpha];
   double rr = 0.0;
   const XcdSpan sp = xcd_span(nn);
   for (int n = sp.lo + sp.j * kT + threadIdx.x; n < sp.hi; n += sp.bx * kT) {
     const size_t d = 3 * (size_t)n;
+    double rv[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       x[d + i] += alpha * p[d + i];
-      const double rv = r[d + i] - alpha * q[d + i];
-      r[d + i] = rv;
-      rr += rv * rv;
+      rv[i] = r[d + i] - alpha * q[d + i];
+      r[d + i] = rv[i];
+      rr += rv[i] * rv[i];
+    }
+    if (z) {
+      double zv[3];
+      dinv3(dinv + 3 * d, rv, zv);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) z[d + i] = zv[i] *= inv_theta;
+      put_lattice(lat, n, zv);
     }
   }
   const double t = block_reduce_all<kT>(rr, sh);
@@ -220,10 +251,15 @@ __global__ __launch_bounds__(kT) void k_mg_update(double* __restrict__ x, double
 }
 
 __global__ __launch_bounds__(kT) void k_mg_pupdate(double* __restrict__ p, const double* __restrict__ z,
-                                                   const double* __restrict__ scal, size_t n) {
-  const double beta = scal[kBeta];
-  for (size_t i = blockIdx.x * (size_t)kT + threadIdx.x; i < n; i += (size_t)gridDim.x * kT)
-    p[i] = fma(beta, p[i], z[i]);
+                                                   const double* __restrict__ scal, int nn, int first, MgLattice lat) {
+  const double beta = first ? 0.0 : scal[kBeta];
+  for (int n = blockIdx.x * kT + threadIdx.x; n < nn; n += gridDim.x * kT) {
+    const size_t d = 3 * (size_t)n;
+    double v[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) p[d + i] = v[i] = first ? z[d + i] : fma(beta, p[d + i], z[d + i]);
+    if (lat.plat) put_lattice(lat, n, v);
+  }
 }
 
 // A row's epilogue operands are loaded by lanes 0..2 (one component each) before the
@@ -475,7 +511,7 @@ __global__ __launch_bounds__(kT) void k_gj_step(const double* __restrict__ S, do
 hipError_t launch_mg_restrict(const double* rf, double* rc, const int32_t* cgrid, const int32_t* fnode_of_grid,
                               BoxDims fd, const uint8_t* cbcmask, int ncn, hipStream_t s, const double* cdinv,
                               double inv_theta, double* cx, double* cd) {
-  k_mg_restrict<<<blocks_of(ncn), kT, 0, s>>>(rf, rc, cgrid, fnode_of_grid, fd, cbcmask, ncn, cdinv, inv_theta, cx,
+  k_mg_restrict<<<blocks_of(8 * (size_t)ncn), kT, 0, s>>>(rf, rc, cgrid, fnode_of_grid, fd, cbcmask, ncn, cdinv, inv_theta, cx,
                                               cd);
   return hipGetLastError();
 }
@@ -505,8 +541,9 @@ hipError_t launch_to_f32(const double* a, float* b, size_t n, hipStream_t s) {
   return hipGetLastError();
 }
 hipError_t launch_mg_prolong_add(const double* ec, double* xf, const int32_t* fgrid, const int32_t* cnode_of_grid,
-                                 BoxDims cd, const uint8_t* fbcmask, int nfn, hipStream_t s) {
-  k_mg_prolong_add<<<blocks_of(nfn), kT, 0, s>>>(ec, xf, fgrid, cnode_of_grid, cd, fbcmask, nfn);
+                                 BoxDims cd, const uint8_t* fbcmask, int nfn, hipStream_t s,
+                                 const MgLattice& lat) {
+  k_mg_prolong_add<<<blocks_of(nfn), kT, 0, s>>>(ec, xf, fgrid, cnode_of_grid, cd, fbcmask, nfn, lat);
   return hipGetLastError();
 }
 hipError_t launch_mg_wrestrict(const double* wf, double* wc, const int32_t* cgrid, const int32_t* fnode_of_grid,
@@ -519,8 +556,8 @@ hipError_t launch_simp_w(const double* z, double* w, int n, const Material& m, h
   return hipGetLastError();
 }
 hipError_t launch_cheb_first(double* x, double* d, const double* r, const double* dinv, double inv_theta, int nn,
-                             hipStream_t s, const double* t) {
-  k_cheb_first<<<blocks_of(nn), kT, 0, s>>>(x, d, r, dinv, inv_theta, nn, t);
+                             hipStream_t s, const double* t, const MgLattice& lat) {
+  k_cheb_first<<<blocks_of(nn), kT, 0, s>>>(x, d, r, dinv, inv_theta, nn, t, lat);
   return hipGetLastError();
 }
 hipError_t launch_cheb_next(double* x, double* d, const double* r, const double* Kx, const double* dinv, double c1,
@@ -545,12 +582,14 @@ hipError_t launch_dense_gemv(const double* A, const double* x, double* y, int n,
   return hipGetLastError();
 }
 hipError_t launch_mg_update(double* x, double* r, const double* p, const double* q, const double* scal, int nn,
-                            double* P_rr, int grid, hipStream_t s) {
-  k_mg_update<<<grid, kT, 0, s>>>(x, r, p, q, scal, nn, P_rr);
+                            double* P_rr, int grid, hipStream_t s, double* z, const double* dinv, double inv_theta,
+                            const MgLattice& lat) {
+  k_mg_update<<<grid, kT, 0, s>>>(x, r, p, q, scal, nn, P_rr, z, dinv, inv_theta, lat);
   return hipGetLastError();
 }
-hipError_t launch_mg_pupdate(double* p, const double* z, const double* scal, size_t n, hipStream_t s) {
-  k_mg_pupdate<<<blocks_of(n), kT, 0, s>>>(p, z, scal, n);
+hipError_t launch_mg_pupdate(double* p, const double* z, const double* scal, int nn, int first, hipStream_t s,
+                             const MgLattice& lat) {
+  k_mg_pupdate<<<blocks_of(nn), kT, 0, s>>>(p, z, scal, nn, first, lat);
   return hipGetLastError();
 }
 

@@ -13,6 +13,16 @@ struct BoxDims {
   int nx, ny, nz;  // node counts per axis
 };
 
+// FP32 copy of a level's vector at the padded lattice points, constrained dofs 0, for the
+// matrix-free operator (plat null: none).  Written by the kernel that makes the vector, so
+// that the operator needs no pass of its own over it.
+struct MgLattice {
+  const int* gpack;        // per node: i | j << 10 | k << 20
+  const uint8_t* bcmask;
+  float4* plat;
+  int px, py;              // padded points along x and y
+};
+
 // rc[c] = sum_{fine i within one fine spacing of coarse node c} w_i rf[i] with the
 // full-weighting weights (1, 1/2 per off-axis step), i.e. R = P^T of trilinear P;
 // constrained coarse dofs are set to 0.  3 components per node.
@@ -24,7 +34,8 @@ hipError_t launch_mg_restrict(const double* rf, double* rc, const int32_t* cgrid
                               double* cd = nullptr);
 // xf[i] += sum_parents w ec[parent] (trilinear), skipping constrained fine dofs.
 hipError_t launch_mg_prolong_add(const double* ec, double* xf, const int32_t* fgrid, const int32_t* cnode_of_grid,
-                                 BoxDims cd, const uint8_t* fbcmask, int nfn, hipStream_t s);
+                                 BoxDims cd, const uint8_t* fbcmask, int nfn, hipStream_t s,
+                                 const MgLattice& lat = {});
 // Normalised full weighting of a scalar nodal field (density homogenisation through the
 // SIMP stiffness weight): wc[c] = sum w_i wf[i] / sum w_i.
 hipError_t launch_mg_wrestrict(const double* wf, double* wc, const int32_t* cgrid, const int32_t* fnode_of_grid,
@@ -38,7 +49,7 @@ hipError_t launch_simp_w(const double* z, double* w, int n, const Material& m, h
 //          written when null)
 //   next:  d = c1 d + c2 D^-1 (r - Kx); x += d
 hipError_t launch_cheb_first(double* x, double* d, const double* r, const double* dinv, double inv_theta, int nn,
-                             hipStream_t s, const double* t = nullptr);
+                             hipStream_t s, const double* t = nullptr, const MgLattice& lat = {});
 hipError_t launch_cheb_next(double* x, double* d, const double* r, const double* Kx, const double* dinv, double c1,
                             double c2, int nn, hipStream_t s);
 // out = a - b ; y += x
@@ -113,7 +124,10 @@ hipError_t launch_mg_dense_inverse(const double* vals, const int32_t* rowmap, co
 //   update: x += alpha p; r -= alpha q (alpha = scal[kAlpha]); partials of r.r
 //   pupdate: p = z + beta p (beta = scal[kBeta])
 hipError_t launch_mg_update(double* x, double* r, const double* p, const double* q, const double* scal, int nn,
-                            double* P_rr, int grid, hipStream_t s);
-hipError_t launch_mg_pupdate(double* p, const double* z, const double* scal, size_t n, hipStream_t s);
+                            double* P_rr, int grid, hipStream_t s, double* z = nullptr, const double* dinv = nullptr,
+                            double inv_theta = 0.0, const MgLattice& lat = {});
+// p = z + beta p (p = z when first)
+hipError_t launch_mg_pupdate(double* p, const double* z, const double* scal, int nn, int first, hipStream_t s,
+                             const MgLattice& lat = {});
 
 }  // namespace pa
