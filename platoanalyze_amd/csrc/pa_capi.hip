@@ -159,6 +159,8 @@ struct pa_problem {
   DevArray<double> partials;  // kNumPartialSlots x kRedBlocks
   DevArray<double> scal;
   DevArray<double> chunk_partials;
+  DevArray<int32_t> inc_offs;
+  DevArray<uint16_t> inc;
   DevArray<float> chunk_gbound;  // per chunk: bound of vol |grad N|^2 (fixed-point Jacobian)
   // deflated solve (pa_solution_deflated): deflation vectors, their images, partials,
   // E = V^T A V, its inverse, mu
@@ -518,6 +520,8 @@ int pa_finalize(pa_handle h) {
   PA_HIP(h->ent_ln.upload(h->chunks.ent_ln));
   PA_HIP(h->ent_code.upload(h->chunks.ent_code));
   PA_HIP(h->tslot.upload(h->chunks.tslot));
+  PA_HIP(h->inc_offs.upload(h->chunks.inc_offs));
+  PA_HIP(h->inc.upload(h->chunks.inc));
   PA_HIP(h->load_nodes.upload(ln));
   PA_HIP(h->load_offs.upload(loffs));
   PA_HIP(h->load_row.upload(lrow));
@@ -1213,6 +1217,9 @@ static int solve_mixed(pa_handle h, const double* z, double* u, const double* b,
   ma.partials = h->chunk_partials.p;
   ma.m = h->material();
   ma.gbound = h->chunk_gbound.p;
+  ma.inc_offs = h->inc_offs.p;
+  ma.inc = h->inc.p;
+  ma.max_list = h->chunks.max_list;
   // r = mask(b - R) into m_r and ||r||^2
   auto masked_residual = [&](const double* R, double* out) -> int {
     PA_HIP(pa::launch_neg_mask(R, b, h->bcmask.p, h->m_r.p, nn, PS(pa::kPDot), G, s));
@@ -1903,6 +1910,9 @@ static int mg_apply(pa_handle h, size_t l, const double* x, double* y, const dou
       ma.partials = h->chunk_partials.p;
       ma.m = h->material();
       ma.gbound = h->chunk_gbound.p;
+      ma.inc_offs = h->inc_offs.p;
+      ma.inc = h->inc.p;
+      ma.max_list = h->chunks.max_list;
       const double* Pq = nullptr;
       int npq = 0;
       if (int rc = mf_apply(h, ma, &Pq, &npq)) return rc;

@@ -415,6 +415,7 @@ Chunks build_chunks(const Graph& g, const NodeElems& adj, const int32_t* conn, c
     ch.max_rows = std::max(ch.max_rows, mrows[c]);
     ch.max_blocks = std::max(ch.max_blocks, mblocks[c]);
     ch.max_nodes = std::max(ch.max_nodes, mnodes[c]);
+    ch.max_list = std::max(ch.max_list, (int)lists[c].size());
   }
   ch.list.resize(ch.list_offs[ch.count]);
   ch.nodes.resize(ch.node_offs[ch.count]);
@@ -432,6 +433,22 @@ Chunks build_chunks(const Graph& g, const NodeElems& adj, const int32_t* conn, c
       }
     }
   });
+  if (ch.max_list < 1 << 14) {  // a row's element vertices are its incidences
+    ch.inc_offs.assign(adj.offs.begin(), adj.offs.end());
+    ch.inc.resize(adj.offs[nn]);
+    parallel_for(ch.count, [&](int64_t b, int64_t e) {
+      std::vector<int32_t> at;
+      for (int64_t c = b; c < e; ++c) {
+        const int r0 = ch.row_begin[c], r1 = ch.row_begin[c + 1];
+        at.assign(ch.inc_offs.begin() + r0, ch.inc_offs.begin() + r1);
+        for (size_t i = 0; i < lists[c].size(); ++i) {
+          const uint32_t el = lists[c][i] & 0x0FFFFFFFu;
+          for (int a = 0; a < 4; ++a)
+            if (lists[c][i] >> (28 + a) & 1u) ch.inc[at[conn[4 * (size_t)el + a] - r0]++] = (uint16_t)(4 * i + a);
+        }
+      }
+    });
+  }
   ch.tslot.assign(g.colidx.size(), kNoSlot);
   parallel_for(ch.count, [&](int64_t b, int64_t e) {
     for (int64_t c = b; c < e; ++c) {

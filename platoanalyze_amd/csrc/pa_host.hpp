@@ -82,7 +82,11 @@ struct Chunks {
   // per graph block (row r, column c): chunk-local slot of block (c, r) when both rows
   // lie in the chunk and c < r, else kNoSlot
   std::vector<uint16_t> tslot;
-  int max_rows = 0, max_blocks = 0, max_nodes = 0;
+  // per row: its (entry, vertex) pairs within the chunk's list, 4 entry + vertex; empty when
+  // a chunk has more than 16383 entries
+  std::vector<int32_t> inc_offs;     // [rows+1]
+  std::vector<uint16_t> inc;
+  int max_rows = 0, max_blocks = 0, max_nodes = 0, max_list = 0;
 };
 Chunks build_chunks(const Graph& g, const NodeElems& ne_adj, const int32_t* conn, const std::vector<uint32_t>& codes,
                     int words_per_code, int max_blocks, int max_rows, int max_nodes);

@@ -33,6 +33,10 @@ struct MfArgs {
   double* partials;  // per-chunk partial of p_cur . y
   Material m;
   const float* gbound;  // per chunk: bound of vol |grad N|^2 (scale of the fixed-point sums)
+  // per row its (entry, vertex) pairs, 4 entry + vertex (null: none)
+  const int32_t* inc_offs;
+  const uint16_t* inc;
+  int max_list;         // entries of a chunk at most
 };
 hipError_t launch_mf_apply(const MfArgs& a, hipStream_t s);
 
