@@ -28,20 +28,6 @@ constexpr int kOwn = kTileNodes, kHex = kOwn + 1, kPts = kOwn + 2;
 constexpr int kHexes = kHex * kHex * kHex, kPoints = kPts * kPts * kPts;
 static_assert(kHexes <= kT, "a thread per hex");
 
-__device__ __forceinline__ double powi(double x, int n) {  // n >= 1
-  double r = 1.0;
-  for (; n > 0; n >>= 1, x *= x)
-    if (n & 1) r *= x;
-  return r;
-}
-
-// x^p: integer exponents to 16 by multiplication, 1/2 by the square root
-__device__ __forceinline__ double pow_of(double x, double p, int pint) {
-  if (pint > 0) return powi(x, pint);
-  if (p == 0.5) return sqrt(x);
-  return pow(x, p);
-}
-
 // Voigt strain (engineering shear) of tet Q of the hex with corner displacements U
 template <int Q>
 __device__ __forceinline__ void tet_strain_of(const double U[8][3], const double ih[3], double e[6]) {

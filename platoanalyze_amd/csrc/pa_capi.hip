@@ -266,6 +266,9 @@ struct pa_problem {
     a.tslot = tslot.p;
     a.max_nodes = chunks.max_nodes;
     a.partials = chunk_partials.p;
+    a.inc_offs = inc_offs.p;
+    a.inc = inc.p;
+    a.max_list = chunks.max_list;
     a.gbound = chunk_gbound.p;
     a.load_offs = load_offs.p;
     a.load_row = load_row.p;

@@ -433,7 +433,7 @@ Chunks build_chunks(const Graph& g, const NodeElems& adj, const int32_t* conn, c
       }
     }
   });
-  if (ch.max_list < 1 << 14) {  // a row's element vertices are its incidences
+  if (ch.max_list <= kMaxGatherList) {  // a row's element vertices are its incidences
     ch.inc_offs.assign(adj.offs.begin(), adj.offs.end());
     ch.inc.resize(adj.offs[nn]);
     parallel_for(ch.count, [&](int64_t b, int64_t e) {

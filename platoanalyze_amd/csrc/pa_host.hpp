@@ -69,6 +69,7 @@ std::vector<uint32_t> slot_codes(const Graph& g, const int32_t* conn, int ne, in
 //       ent_code the element's slot codes (words_per_code uint32 each),
 //     sorted by owned-vertex count and interleaved (see build_chunks).
 constexpr uint16_t kNoSlot = 0xFFFF;
+constexpr int kMaxGatherList = 4096;  // below 2^14: 16-bit pairs
 
 struct Chunks {
   int count = 0;
@@ -83,7 +84,7 @@ struct Chunks {
   // lie in the chunk and c < r, else kNoSlot
   std::vector<uint16_t> tslot;
   // per row: its (entry, vertex) pairs within the chunk's list, 4 entry + vertex; empty when
-  // a chunk has more than 16383 entries
+  // a chunk has more than kMaxGatherList entries (a value per entry then stays out of LDS)
   std::vector<int32_t> inc_offs;     // [rows+1]
   std::vector<uint16_t> inc;
   int max_rows = 0, max_blocks = 0, max_nodes = 0, max_list = 0;

@@ -3,6 +3,10 @@
 // (atomic-free in HBM: each CRS value and residual entry is written exactly once,
 // coalesced), then streams the finished segment out.
 #include "pa_kernels.hpp"
+
+#include <algorithm>
+#include <cmath>
+
 #include "pa_fixed.hpp"
 #include "pa_dpp.hpp"
 
@@ -100,7 +104,7 @@ __device__ __forceinline__ int sel4i(int a, int x0, int x1, int x2, int x3) {
 // Vector-valued element kernels (residual, dR/dz, energy and its gradient) over the
 // same chunks: node coordinates, density and state staged in LDS, elements streamed
 // as records of local node indices, owned rows accumulated in LDS.
-template <int BITS, int MODE, int NT>
+template <int BITS, int MODE, int NT, bool SIMP>
 __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
   extern __shared__ double lds[];
   constexpr bool kRes = MODE == kModeResidual;
@@ -109,6 +113,9 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
   constexpr bool kPnV = MODE == kModePNorm, kPnG = MODE == kModePNormGrad, kPnX = MODE == kModePNormGradX;
   constexpr bool kAdj = MODE == kModeAdjZ;
   constexpr bool kGx = MODE == kModeGradX, kEGx = MODE == kModeEnergyGradX, kVol = MODE == kModeVolume;
+  // one value per element, the same for its four vertices: kept in LDS and gathered by the
+  // rows, or added with atomics where the chunks' lists are too long (no incidences)
+  constexpr bool kGather = kGradZ || kAdj;
   constexpr bool kReduce = MODE == kModeEnergy || kGradZ || kPnV || kVol;
   constexpr int kBlkW = kGzT ? 3 : (kGx ? 9 : 0);                      // doubles per block in LDS
   constexpr int kRowW = (kRes || kPnG || kEGx || kVol || kPnX) ? 3 : ((kGradZ || kAdj) ? 1 : 0);  // doubles per row
@@ -128,6 +135,8 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
   double* res = seg + (size_t)A.max_blocks * kBlkW;
   double* res2 = res + (size_t)A.max_rows * kRowW;
   int* roff = reinterpret_cast<int*>(res2 + (size_t)A.max_rows * kRow2);
+  double* elem = res;  // kGather with incidences: [max_list]
+  const bool gather = kGather && A.inc;
 
   // the residual sums in fixed point (order-independent): the scale comes from the
   // largest |u| of the chunk's nodes, a NaN among them poisons it
@@ -154,7 +163,8 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
     for (int k = threadIdx.x; k <= nr; k += NT) roff[k] = A.rowmap[r0 + k] - b0;
   }
   if constexpr (kRowW > 0)
-    for (int k = threadIdx.x; k < nr * kRowW; k += NT) res[k] = 0.0;
+    if (!gather)
+      for (int k = threadIdx.x; k < nr * kRowW; k += NT) res[k] = 0.0;
   if constexpr (kRow2 > 0)
     for (int k = threadIdx.x; k < nr * kRow2; k += NT) res2[k] = 0.0;
   if constexpr (kRes) block_max_write<NT>(umax, red);
@@ -166,6 +176,15 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
     S = fixed_scale_54(24.0 * cs * (double)A.gbound[c] * block_max_read<NT>(red));
   }
 
+  auto add_element = [&](int e, const int ln[4], double v) {
+    if (gather) {
+      elem[e] = v;
+      return;
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      if (ln[a] < nr) lds_add(&res[ln[a]], v);
+  };
   double energy = 0.0;
   const int l0 = A.list_offs[c], l1 = A.list_offs[c + 1];
   for (int k = l0 + threadIdx.x; k < l1; k += NT) {
@@ -184,7 +203,7 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
     }
     tet_gradients(x, g, vol);
     rho = rho / 4.0;
-    const double w = penalty_w(A.m, rho);
+    const double w = penalty_w_as<SIMP>(A.m, rho);
     double eps[6], s[6];
     tet_strain(u, g, eps);
     iso_stress(A.m, eps, s);
@@ -200,11 +219,8 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
         double sr = 0.0;
 #pragma unroll
         for (int q = 0; q < 6; ++q) sr += s[q] * eps[q];
-        const double dw = penalty_dw(A.m, rho);
-        const double gz = A.scale * (0.5 * vol * sr * dw * 0.25);
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-          if (ln[a] < nr) lds_add(&res[ln[a]], gz);
+        const double dw = penalty_dw_as<SIMP>(A.m, rho);
+        add_element(k - l0, ln, A.scale * (0.5 * vol * sr * dw * 0.25));
       }
     }
     if constexpr (kPnV || kPnG || kPnX) {
@@ -219,11 +235,11 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
 #pragma unroll
         for (int q = 0; q < 6; ++q) t[q] = w * s[q];  // d|sigma_w|/du = w B^T C0 sigma_w / m
         cu = mval > 0.0 ? w / mval : 0.0;
-        cz = penalty_dw(A.m, rho) / w;
+        cz = penalty_dw_as<SIMP>(A.m, rho) / w;
       } else {
         const double d01 = s[0] - s[1], d12 = s[1] - s[2], d20 = s[2] - s[0];
         const double j2 = 0.5 * (d01 * d01 + d12 * d12 + d20 * d20) + 3.0 * (s[3] * s[3] + s[4] * s[4] + s[5] * s[5]);
-        const double vm0 = sqrt(j2), rq = pow(rho, A.q);
+        const double vm0 = sqrt(j2), rq = SIMP ? sqrt(rho) : pow(rho, A.q);
         mval = rq * vm0;
         t[0] = 2.0 * s[0] - s[1] - s[2];
         t[1] = 2.0 * s[1] - s[2] - s[0];
@@ -234,7 +250,7 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
         cu = vm0 > 0.0 ? rq / (2.0 * vm0) : 0.0;  // d vm / d sigma = dJ/dsigma / (2 vm)
         cz = A.q / rho;
       }
-      const double mp = pow(mval, A.pn);
+      const double mp = SIMP ? powi(mval, (int)A.pn) : pow(mval, A.pn);
       if constexpr (kPnV) {
         if (ln[0] < nr) energy += mp * vol;
       } else if constexpr (kPnX) {
@@ -298,11 +314,8 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
       double dot = 0.0;
 #pragma unroll
       for (int q = 0; q < 6; ++q) dot += el[q] * s[q];
-      const double dw = penalty_dw(A.m, rho);
-      const double v = 0.25 * dw * vol * dot;
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-        if (ln[a] < nr) lds_add(&res[ln[a]], v);
+      const double dw = penalty_dw_as<SIMP>(A.m, rho);
+      add_element(k - l0, ln, 0.25 * dw * vol * dot);
     }
     if constexpr (kRes) {
       double sw[6];
@@ -337,7 +350,7 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
         cw[2] = t.z;
         cw[3] = t.w;
       }
-      const double dw = penalty_dw(A.m, rho) * 0.25;
+      const double dw = penalty_dw_as<SIMP>(A.m, rho) * 0.25;
       double rb[4][3];
 #pragma unroll
       for (int b = 0; b < 4; ++b) tet_divergence(s, g[b], vol, rb[b]);
@@ -357,7 +370,7 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
     if constexpr (kVol) {
       // Geometric volume V = sum_e vol_e w(rho_e) with the criterion's own penalty (in
       // A.m): dV/dz_a = vol w'(rho) / 4, dV/dX_a = w vol g_a (dvol/dX_a = vol g_a)
-      const double dw = penalty_dw(A.m, rho);
+      const double dw = penalty_dw_as<SIMP>(A.m, rho);
       if (ln[0] < nr) energy += vol * w;
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
@@ -481,7 +494,19 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
     double* dst = A.out_vals + (size_t)b0 * kBlkW;
     for (int k = threadIdx.x; k < nb * kBlkW; k += NT) dst[k] = seg[k];
   }
+  if (gather) {  // four lanes a row, in list order
+    const int lane = threadIdx.x & 3;
+    for (int lr = threadIdx.x >> 2; lr < nr; lr += NT / 4) {
+      const int i1 = A.inc_offs[r0 + lr + 1];
+      double v = 0.0;
+      for (int i = A.inc_offs[r0 + lr] + lane; i < i1; i += 4) v += elem[A.inc[i] >> 2];
+      v += dpp_f64<kDppXor1>(v);
+      v += dpp_f64<kDppXor2>(v);
+      if (lane == 0) A.out_vec[r0 + lr] = v;
+    }
+  }
   if constexpr (kRowW > 0) {
+    if (gather) return;
     double* dst = A.out_vec + (size_t)r0 * kRowW;
     for (int k = threadIdx.x; k < nr * kRowW; k += NT) dst[k] = res[k];
   }
@@ -579,7 +604,7 @@ __device__ __forceinline__ void jac_stage(const ChunkArgs& A, const JacChunk& J,
 }
 
 // Phase 2 (after the staging barrier): the chunk's traction loads, then the elements.
-template <int BITS, int NT, bool WITH_R>
+template <int BITS, int NT, bool WITH_R, bool SIMP>
 __device__ __forceinline__ void jac_elements(const ChunkArgs& A, const JacChunk& J, double* seg,
                                              const double4* nodes, const int* roff, double* fl) {
   const int c = J.c, nr = J.nr;
@@ -622,7 +647,7 @@ __device__ __forceinline__ void jac_elements(const ChunkArgs& A, const JacChunk&
     }
     tet_gradients(x, g, vol);
     rho = rho / 4.0;
-    const double w = penalty_w(A.m, rho);
+    const double w = penalty_w_as<SIMP>(A.m, rho);
     const double vl = vol * w * A.m.c01, vm = vol * w * A.m.c33;
     bool own[4];
     int ro[4];
@@ -753,7 +778,7 @@ __device__ __forceinline__ void jac_stream(const ChunkArgs& A, int b0, int nb, c
   if (((n - head) & 1) && threadIdx.x == 0) __builtin_nontemporal_store(seg[n - 1], dst + n - 1);
 }
 
-template <int BITS, bool WITH_R, int NT>
+template <int BITS, bool WITH_R, int NT, bool SIMP>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 512 ? 4 : 1)))
 void k_jac_chunk(ChunkArgs A) {
   extern __shared__ double lds[];
@@ -767,7 +792,7 @@ void k_jac_chunk(ChunkArgs A) {
   const JacChunk J = jac_chunk_info(A, xcd_chunk(blockIdx.x, A.nchunks));
   jac_stage<NT, WITH_R>(A, J, seg, nodes, roff, col, fl);
   __syncthreads();
-  jac_elements<BITS, NT, WITH_R>(A, J, seg, nodes, roff, fl);
+  jac_elements<BITS, NT, WITH_R, SIMP>(A, J, seg, nodes, roff, fl);
   __syncthreads();
   jac_fixed_to_double<NT>(seg, 9 * J.nb, fixed_scale(A, J.c));
   __syncthreads();
@@ -796,24 +821,29 @@ size_t chunk_lds_bytes(int mode, int max_rows, int max_blocks, int max_nodes) {
 constexpr int kNtJac = 512;
 constexpr int kNtVec = 256;
 
-template <int BITS>
-static hipError_t launch_chunk_b(int mode, const ChunkArgs& a, hipStream_t s) {
-  const size_t lds = chunk_lds_bytes(mode, a.max_rows, a.max_blocks, a.max_nodes);
+template <int BITS, bool SIMP>
+static hipError_t launch_chunk_b(int mode, ChunkArgs a, hipStream_t s) {
+  size_t lds = chunk_lds_bytes(mode, a.max_rows, a.max_blocks, a.max_nodes);
+  if (mode == kModeEnergyGradZ || mode == kModeAdjZ) {  // a value per entry instead of per row, if it fits
+    const size_t more = sizeof(double) * (size_t)std::max(0, a.max_list - a.max_rows);
+    if (lds + more <= 64 * 1024) lds += more;
+    else a.inc = nullptr;
+  }
   dim3 grid(a.nchunks);
   switch (mode) {
-    case kModeJacobian: k_jac_chunk<BITS, false, kNtJac><<<grid, kNtJac, lds, s>>>(a); break;
-    case kModeJacobianResidual: k_jac_chunk<BITS, true, kNtJac><<<grid, kNtJac, lds, s>>>(a); break;
-    case kModeResidual: k_chunk<BITS, kModeResidual, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModeGradZT: k_chunk<BITS, kModeGradZT, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModeEnergy: k_chunk<BITS, kModeEnergy, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModeEnergyGradZ: k_chunk<BITS, kModeEnergyGradZ, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModePNorm: k_chunk<BITS, kModePNorm, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModePNormGrad: k_chunk<BITS, kModePNormGrad, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModeAdjZ: k_chunk<BITS, kModeAdjZ, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModeGradX: k_chunk<BITS, kModeGradX, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModeEnergyGradX: k_chunk<BITS, kModeEnergyGradX, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModeVolume: k_chunk<BITS, kModeVolume, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
-    case kModePNormGradX: k_chunk<BITS, kModePNormGradX, kNtVec><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeJacobian: k_jac_chunk<BITS, false, kNtJac, SIMP><<<grid, kNtJac, lds, s>>>(a); break;
+    case kModeJacobianResidual: k_jac_chunk<BITS, true, kNtJac, SIMP><<<grid, kNtJac, lds, s>>>(a); break;
+    case kModeResidual: k_chunk<BITS, kModeResidual, kNtVec, SIMP><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeGradZT: k_chunk<BITS, kModeGradZT, kNtVec, SIMP><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeEnergy: k_chunk<BITS, kModeEnergy, kNtVec, SIMP><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeEnergyGradZ: k_chunk<BITS, kModeEnergyGradZ, kNtVec, SIMP><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModePNorm: k_chunk<BITS, kModePNorm, kNtVec, SIMP><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModePNormGrad: k_chunk<BITS, kModePNormGrad, kNtVec, SIMP><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeAdjZ: k_chunk<BITS, kModeAdjZ, kNtVec, SIMP><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeGradX: k_chunk<BITS, kModeGradX, kNtVec, false><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeEnergyGradX: k_chunk<BITS, kModeEnergyGradX, kNtVec, false><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModeVolume: k_chunk<BITS, kModeVolume, kNtVec, false><<<grid, kNtVec, lds, s>>>(a); break;
+    case kModePNormGradX: k_chunk<BITS, kModePNormGradX, kNtVec, false><<<grid, kNtVec, lds, s>>>(a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -824,22 +854,30 @@ static void allow_lds(K kernel) {
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                             160 * 1024);
 }
+template <int BITS, bool SIMP>
+static void allow_lds_all() {
+  allow_lds(&k_jac_chunk<BITS, false, kNtJac, SIMP>);
+  allow_lds(&k_jac_chunk<BITS, true, kNtJac, SIMP>);
+  allow_lds(&k_chunk<BITS, kModeGradZT, kNtVec, SIMP>);
+  if (!SIMP) allow_lds(&k_chunk<BITS, kModeGradX, kNtVec, false>);
+}
 
 hipError_t launch_chunk(int bits, int mode, const ChunkArgs& a, hipStream_t s) {
   static bool once = false;
   if (!once) {
     once = true;
-    allow_lds(&k_jac_chunk<4, false, kNtJac>);
-    allow_lds(&k_jac_chunk<4, true, kNtJac>);
-    allow_lds(&k_jac_chunk<8, false, kNtJac>);
-    allow_lds(&k_jac_chunk<8, true, kNtJac>);
-    allow_lds(&k_chunk<4, kModeGradZT, kNtVec>);
-    allow_lds(&k_chunk<8, kModeGradZT, kNtVec>);
-    allow_lds(&k_chunk<4, kModeGradX, kNtVec>);
-    allow_lds(&k_chunk<8, kModeGradX, kNtVec>);
+    allow_lds_all<4, false>();
+    allow_lds_all<4, true>();
+    allow_lds_all<8, false>();
+    allow_lds_all<8, true>();
   }
   if (a.nchunks == 0) return hipSuccess;
-  return bits == 4 ? launch_chunk_b<4>(mode, a, s) : launch_chunk_b<8>(mode, a, s);
+  bool simp = a.m.model == kPenaltySimp && a.m.pint > 0;
+  // the p-norms in that form: an integer p and, for the relaxed von Mises measure, q = 1/2
+  if (mode == kModePNorm || mode == kModePNormGrad)
+    simp = simp && a.pn >= 1.0 && a.pn <= 16.0 && a.pn == std::floor(a.pn) && (a.measure == 0 || a.q == 0.5);
+  if (bits == 4) return simp ? launch_chunk_b<4, true>(mode, a, s) : launch_chunk_b<4, false>(mode, a, s);
+  return simp ? launch_chunk_b<8, true>(mode, a, s) : launch_chunk_b<8, false>(mode, a, s);
 }
 
 }  // namespace pa

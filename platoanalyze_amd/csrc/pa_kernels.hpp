@@ -42,6 +42,14 @@ __device__ __forceinline__ double simp_pow(double rho, double p, int pint) {
   return pow(rho, p);
 }
 
+// rho^n by multiplication, n >= 0
+__device__ __forceinline__ double simp_powi(double rho, int n) {
+  if (n < 1) return 1.0;
+  double r = rho;
+  for (int k = 1; k < n; ++k) r *= rho;
+  return r;
+}
+
 // w(rho) and dw/drho of the material's penalty model
 __device__ __forceinline__ double penalty_w(const Material& m, double rho) {
   switch (m.model) {
@@ -95,6 +103,34 @@ __device__ __forceinline__ double penalty_dw(const Material& m, double rho) {
   }
 }
 
+// The same where SIMP says that the model is SIMP with an integer exponent (Material::pint
+// > 0), without the other models' code: their powers and sines take an element kernel from
+// 60-90 registers to 144-170, that is from five or six waves a SIMD to three.
+template <bool SIMP>
+__device__ __forceinline__ double penalty_w_as(const Material& m, double rho) {
+  if constexpr (SIMP) return m.rmin + (1.0 - m.rmin) * simp_powi(rho, m.pint);
+  else return penalty_w(m, rho);
+}
+template <bool SIMP>
+__device__ __forceinline__ double penalty_dw_as(const Material& m, double rho) {
+  if constexpr (SIMP) return (1.0 - m.rmin) * m.p * simp_powi(rho, m.pint - 1);
+  else return penalty_dw(m, rho);
+}
+
+__device__ __forceinline__ double powi(double x, int n) {  // n >= 1
+  double r = 1.0;
+  for (; n > 0; n >>= 1, x *= x)
+    if (n & 1) r *= x;
+  return r;
+}
+
+// x^p: integer exponents to 16 by multiplication, 1/2 by the square root
+__device__ __forceinline__ double pow_of(double x, double p, int pint) {
+  if (pint > 0) return powi(x, pint);
+  if (p == 0.5) return sqrt(x);
+  return pow(x, p);
+}
+
 // Arguments of the chunked element kernels (one work-group per row chunk).
 struct ChunkArgs {
   const int4* conn;
@@ -113,6 +149,10 @@ struct ChunkArgs {
   const uint16_t* ent_ln;     // 4 local node indices per entry
   const uint32_t* ent_code;   // slot codes per entry
   const uint16_t* tslot;      // per graph block: chunk-local slot of the transposed block
+  // per row its (entry, vertex) pairs within the chunk's list, 4 entry + vertex (null: none)
+  const int32_t* inc_offs;
+  const uint16_t* inc;
+  int max_list;               // entries of a chunk at most
   double* out_vals;   // Jacobian values (9/block) or dR/dz (3/block)
   double* out_vec;    // residual (3/row) or nodal gradient (1/row)
   double* out_vec2;   // p-norm dF/dz partial (1/row)

@@ -1,7 +1,8 @@
 """FP32 matrix-free operator of general meshes by row sums of element forces kept in LDS,
 through the mixed-precision solves that use it: chunks smaller than a work-group, several
 chunks, shuffled node numbers (full node tables), and a fan of tets around an axis whose
-chunk has too many elements for LDS and takes the atomic sums."""
+chunk has too many elements for LDS and takes the atomic sums; and the FP64 element kernels
+of general meshes with long element lists."""
 import numpy as np
 import pytest
 import torch
@@ -63,3 +64,34 @@ def test_gpu_mf_gather_solutions(mesh):
     z = torch.as_tensor(np.random.default_rng(1).uniform(0.3, 1.0, m.num_nodes), device="cuda")
     u = {p: Problem(model, tolerance=1e-10, precision=p).solution(z) for p in ("fp64", "mixed")}
     assert float((u["mixed"] - u["fp64"]).norm() / u["fp64"].norm()) < 1e-6
+
+
+@pytest.mark.parametrize("times", [3, 12])
+@pytest.mark.parametrize("penalty", [("SIMP", 3.0), ("SIMP", 1.0), ("RAMP", 3.0)])
+def test_gpu_element_kernels_long_lists(times, penalty):
+    """A mesh whose elements are listed several times is several meshes: the density
+    gradients gather from LDS (3 times: up to 2400 entries a chunk) or add with atomics (12
+    times).  Both sides are FP64 sums of at most a few hundred terms a node."""
+    from platoanalyze_amd.criteria import StressPNorm, dRdz_T_apply
+    from platoanalyze_amd.elliptic import ElasticModel, EssentialBC, PhysicsScalarFunction, VectorFunction
+    from platoanalyze_amd.mesh import TetMesh, nodes_on_plane
+
+    print(f"case: long element lists x{times} {penalty}", flush=True)
+    m = _graded((9, 8, 7), False)
+    many = TetMesh(m.coords, np.ascontiguousarray(np.repeat(m.conn, times, axis=0)))
+    one, more = (ElasticModel(x, 1.0, 0.3, essential_bcs=[EssentialBC(nodes_on_plane(x, 2, 0.0), 0, 0.0)],
+                              penalty_model=penalty[0], penalty_exponent=penalty[1]) for x in (m, many))
+    rng = np.random.default_rng(6)
+    u, lam = (torch.as_tensor(rng.normal(size=one.num_dofs), device="cuda") for _ in range(2))
+    z = torch.as_tensor(rng.uniform(0.2, 0.9, one.num_nodes), device="cuda")
+
+    def close(a, b):
+        assert float((a - times * b).abs().max() / (times * b).abs().max()) < 1e-12
+
+    close(PhysicsScalarFunction(more).gradient_z(u, z), PhysicsScalarFunction(one).gradient_z(u, z))
+    close(dRdz_T_apply(more, u, lam, z), dRdz_T_apply(one, u, lam, z))
+    close(VectorFunction(more).value(u, z), VectorFunction(one).value(u, z))
+    close(VectorFunction(more).gradient_u(u, z).entries, VectorFunction(one).gradient_u(u, z).entries)
+    a, b = StressPNorm(more, 1.0, "von_mises", 0.5), StressPNorm(one, 1.0, "von_mises", 0.5)
+    close(a.gradient_u(u, z), b.gradient_u(u, z))
+    close(a.gradient_z(u, z), b.gradient_z(u, z))
