@@ -11,9 +11,14 @@
 // gradient's columns are the three edge differences over the spacings.
 //
 // What bounds it: FP64 arithmetic and the latency of the two dependent gathers (map, then
-// u and z) at ten to twelve waves a CU.
+// u and z) at twelve waves a CU: registers, as LDS holds the corner contributions of half the
+// corners at a time.  128x64x64 hexes, one thread per row with lattice copies and a weight
+// array -> bricks with all corners and every penalty model's code -> this: residual 62 -> 48.5
+// -> 39 us a call, energy and gradient (chunk kernel) 149 -> 60 -> 51; p-norm adjoint
+// gradient, 64x32x32, 182 -> 124 -> 109.  Four waves a SIMD spill (residual 51 us, gradient 109).
 #include "pa_boxtile.hpp"
 
+#include <cmath>
 #include <type_traits>
 
 #include "pa_box.hpp"
@@ -28,17 +33,28 @@ constexpr int kOwn = kTileNodes, kHex = kOwn + 1, kPts = kOwn + 2;
 constexpr int kHexes = kHex * kHex * kHex, kPoints = kPts * kPts * kPts;
 static_assert(kHexes <= kT, "a thread per hex");
 
+// Value i (of three) of a staged vector at corner c of a hex, at compile-time offsets from
+// its lower corner's address.  The points stay in LDS, so that the compiler may read a value
+// again instead of holding all corners' 24 a vector through the six tets.
+struct Corners {
+  const double* p;
+  __device__ __forceinline__ double operator()(int c, int i) const {
+    return p[i * kPoints + (c & 1) + kPts * ((c >> 1) & 1) + kPts * kPts * (c >> 2)];
+  }
+};
+
 // Voigt strain (engineering shear) of tet Q of the hex with corner displacements U
 template <int Q>
-__device__ __forceinline__ void tet_strain_of(const double U[8][3], const double ih[3], double e[6]) {
+__device__ __forceinline__ void tet_strain_of(const Corners& U, const double ih[3], double e[6]) {
   constexpr int a = kKuhnPath[Q][0], b = kKuhnPath[Q][1], c = kKuhnPath[Q][2];
   constexpr int v1 = 1 << a, v2 = (1 << a) | (1 << b);
   double G[3][3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    G[i][a] = (U[v1][i] - U[0][i]) * ih[a];
-    G[i][b] = (U[v2][i] - U[v1][i]) * ih[b];
-    G[i][c] = (U[7][i] - U[v2][i]) * ih[c];
+    const double u1 = U(v1, i), u2 = U(v2, i);
+    G[i][a] = (u1 - U(0, i)) * ih[a];
+    G[i][b] = (u2 - u1) * ih[b];
+    G[i][c] = (U(7, i) - u2) * ih[c];
   }
   e[0] = G[0][0];
   e[1] = G[1][1];
@@ -105,23 +121,18 @@ __device__ __forceinline__ double von_mises2(const double s[6]) {
   return 0.5 * (d01 * d01 + d12 * d12 + d20 * d20) + 3.0 * (s[3] * s[3] + s[4] * s[4] + s[5] * s[5]);
 }
 
-template <int MODE>
-__global__ __launch_bounds__(kT) void k_box_tile(BoxTileArgs A) {
+template <int MODE, bool SIMP>  // SIMP: powers by multiplication only (see launch_box_tile)
+__global__ __launch_bounds__(kT, 3) void k_box_tile(BoxTileArgs A) {
   constexpr bool kRes = MODE == kTileResidual, kGradZ = MODE == kTileEnergyGradZ, kPnG = MODE == kTilePNormGrad;
   constexpr bool kAdj = MODE == kTileAdjZ, kPn = MODE == kTilePNorm || kPnG;
   constexpr bool kVec = kRes || kPnG, kScal = kGradZ || kPnG || kAdj;  // corner vectors, corner scalars
   constexpr bool kSum = MODE == kTileEnergy || kGradZ || MODE == kTilePNorm;
   constexpr int kOut = (kVec ? 3 : 0) + (kScal ? 1 : 0);
-  constexpr int kStage = kPoints * (kAdj ? 7 : 4), kCorner = 8 * kOut * kT;
-  // the staged points and the corner contributions share one region (a barrier between)
-  __shared__ double sm[kStage > kCorner ? kStage : kCorner];
-  // per hex and tet: density and strain measure, then coefficients (the residual needs no
-  // strain measure: its densities start in cl)
-  __shared__ double cl[6][kT], rl_[kRes ? 1 : 6][kT];
-  auto& rl = [&]() -> auto& {
-    if constexpr (kRes) return cl;
-    else return rl_;
-  }();
+  // the points' u and z (and u2), and the contributions of four of a hex's corners at a time
+  __shared__ double sm[kPoints * (kAdj ? 7 : 4)], sc[kOut > 0 ? 4 * kOut * kT : 1];
+  // per hex and tet, where the penalty model's code shall exist once (a rolled loop): density
+  // and strain measure, then coefficients
+  __shared__ double cl[SIMP ? 1 : 6][SIMP ? 1 : kT], rl[SIMP ? 1 : 6][SIMP ? 1 : kT];
   __shared__ int ids[kPoints];
   __shared__ double sh[kT / 64];
 
@@ -151,20 +162,12 @@ __global__ __launch_bounds__(kT) void k_box_tile(BoxTileArgs A) {
   const int gi = i0 - 1 + hx, gj = j0 - 1 + hy, gk = k0 - 1 + hz;
   const bool hex = t < kHexes && gi >= 0 && gj >= 0 && gk >= 0 && gi < A.nx - 1 && gj < A.ny - 1 && gk < A.nz - 1;
   const int at = hx + kPts * (hy + kPts * hz);
-  double U[8][3], L[8][3], Z[8];
+  const Corners U{sm + at}, L{sm + 4 * kPoints + at};
+  double Z[8];
   if (hex) {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int p = at + (c & 1) + kPts * ((c >> 1) & 1) + kPts * kPts * (c >> 2);
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        U[c][i] = sm[i * kPoints + p];
-        if constexpr (kAdj) L[c][i] = sm[(4 + i) * kPoints + p];
-      }
-      Z[c] = sm[3 * kPoints + p];
-    }
+    for (int c = 0; c < 8; ++c) Z[c] = U(c, 3);
   }
-  __syncthreads();  // sm becomes the corner contributions
   double sum = 0.0, F[8][3], S[8];
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
@@ -174,12 +177,12 @@ __global__ __launch_bounds__(kT) void k_box_tile(BoxTileArgs A) {
   }
   if (hex) {
     const double ih[3] = {A.ih[0], A.ih[1], A.ih[2]};
-    // per tet: its density and the strain measure its coefficient needs
-    each_tet<0>([&](auto q) {
+    const int pni = SIMP ? (int)A.pn : (A.pn <= 16.0 && A.pn == floor(A.pn)) ? (int)A.pn : 0;
+    // strain measure of a tet that its coefficients need
+    auto measure = [&](auto q) {
       constexpr int Q = decltype(q)::value;
-      rl[Q][t] = tet_rho<Q>(Z);
+      double e[6], s[6], v = 0.0;
       if constexpr (!kRes) {
-        double e[6], s[6], v = 0.0;
         tet_strain_of<Q>(U, ih, e);
         stress_of(A.m, e, s);
         if constexpr (kPn) {
@@ -198,103 +201,139 @@ __global__ __launch_bounds__(kT) void k_box_tile(BoxTileArgs A) {
 #pragma unroll
           for (int k = 0; k < 6; ++k) v += s[k] * e[k];
         }
-        cl[Q][t] = v;
       }
-    });
-    // coefficients; a rolled loop, so the penalty models' and powers' code exists once
-    const int pni = (A.pn <= 16.0 && A.pn == floor(A.pn)) ? (int)A.pn : 0;
-#pragma unroll 1
-    for (int q = 0; q < 6; ++q) {
-      const double rho = rl[q][t];
+      return v;
+    };
+    // its coefficients: cf of the corner vectors, cs of the corner scalars
+    auto coefficients = [&](double rho, double v, double& cf, double& cs) {
+      cf = cs = 0.0;
       if constexpr (kRes) {
-        cl[q][t] = A.vol * penalty_w(A.m, rho);
+        cf = A.vol * penalty_w_as<SIMP>(A.m, rho);
       } else if constexpr (kAdj) {
-        cl[q][t] *= 0.25 * penalty_dw(A.m, rho) * A.vol;
+        cs = v * (0.25 * penalty_dw_as<SIMP>(A.m, rho) * A.vol);
       } else if constexpr (!kPn) {
-        const double v = cl[q][t];
-        sum += 0.5 * A.vol * penalty_w(A.m, rho) * v;
-        if constexpr (kGradZ) cl[q][t] = A.scale * (0.125 * A.vol * v * penalty_dw(A.m, rho));
+        sum += 0.5 * A.vol * penalty_w_as<SIMP>(A.m, rho) * v;
+        if constexpr (kGradZ) cs = A.scale * (0.125 * A.vol * v * penalty_dw_as<SIMP>(A.m, rho));
       } else {
         // m, with dm/du = c_u B^T C0 t and dm/drho = c_z m (t: see the forces below)
         double mval, cu, cz;
         if (A.measure == 0) {
-          const double w = penalty_w(A.m, rho);
-          mval = fabs(w) * sqrt(cl[q][t]);
+          const double w = penalty_w_as<SIMP>(A.m, rho);
+          mval = fabs(w) * sqrt(v);
           cu = mval > 0.0 ? w * w / mval : 0.0;
-          cz = kPnG ? penalty_dw(A.m, rho) / w : 0.0;
+          cz = kPnG ? penalty_dw_as<SIMP>(A.m, rho) / w : 0.0;
         } else {
-          const double vm0 = sqrt(cl[q][t]), rq = pow_of(rho, A.q, 0);
+          const double vm0 = sqrt(v), rq = SIMP ? sqrt(rho) : pow_of(rho, A.q, 0);
           mval = rq * vm0;
           cu = vm0 > 0.0 ? rq / (2.0 * vm0) : 0.0;
           cz = kPnG ? A.q / rho : 0.0;
         }
-        const double mp = pow_of(mval, A.pn, pni);
+        const double mp = SIMP ? powi(mval, pni) : pow_of(mval, A.pn, pni);
         sum += mp * A.vol;
         if constexpr (kPnG) {
           const double k = A.pscale * A.vol * A.pn;
-          cl[q][t] = k * (mval > 0.0 ? mp / mval : 0.0) * cu;
-          rl[q][t] = 0.25 * k * mp * cz;
+          cf = k * (mval > 0.0 ? mp / mval : 0.0) * cu;
+          cs = 0.25 * k * mp * cz;
         }
       }
-    }
-    if constexpr (kOut > 0) {
+    };
+    auto forces = [&](auto q, double cf, double cs) {
+      constexpr int Q = decltype(q)::value;
+      if constexpr (kVec) {
+        double e[6], s[6];
+        tet_strain_of<Q>(U, ih, e);
+        stress_of(A.m, e, s);
+        if constexpr (kPnG) {
+          if (A.measure != 0) {  // t = dJ/dsigma; measure 0: t = sigma
+            const double tr = s[0] + s[1] + s[2];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) s[k] = 3.0 * s[k] - tr;
+#pragma unroll
+            for (int k = 3; k < 6; ++k) s[k] *= 6.0;
+          }
+          double tau[6];
+          stress_of(A.m, s, tau);
+          tet_force<Q>(tau, cf, ih, F);
+        } else {
+          tet_force<Q>(s, cf, ih, F);
+        }
+      }
+      if constexpr (kScal) tet_scalar<Q>(cs, S);
+    };
+    if constexpr (SIMP) {
+      each_tet<0>([&](auto q) {
+        double cf, cs;
+        coefficients(tet_rho<decltype(q)::value>(Z), measure(q), cf, cs);
+        forces(q, cf, cs);
+      });
+    } else {
       each_tet<0>([&](auto q) {
         constexpr int Q = decltype(q)::value;
-        if constexpr (kVec) {
-          double e[6], s[6];
-          tet_strain_of<Q>(U, ih, e);
-          stress_of(A.m, e, s);
-          if constexpr (kPnG) {
-            if (A.measure != 0) {  // t = dJ/dsigma; measure 0: t = sigma
-              const double tr = s[0] + s[1] + s[2];
-#pragma unroll
-              for (int k = 0; k < 3; ++k) s[k] = 3.0 * s[k] - tr;
-#pragma unroll
-              for (int k = 3; k < 6; ++k) s[k] *= 6.0;
-            }
-            double tau[6];
-            stress_of(A.m, s, tau);
-            tet_force<Q>(tau, cl[Q][t], ih, F);
-          } else {
-            tet_force<Q>(s, cl[Q][t], ih, F);
-          }
-        }
-        if constexpr (kScal) tet_scalar<Q>(kPnG ? rl[Q][t] : cl[Q][t], S);
+        rl[Q][t] = tet_rho<Q>(Z);
+        cl[Q][t] = measure(q);
       });
+#pragma unroll 1
+      for (int q = 0; q < 6; ++q) {
+        double cf, cs;
+        coefficients(rl[q][t], cl[q][t], cf, cs);
+        cl[q][t] = cf;
+        rl[q][t] = cs;
+      }
+      if constexpr (kOut > 0)
+        each_tet<0>([&](auto q) {
+          constexpr int Q = decltype(q)::value;
+          forces(q, cl[Q][t], rl[Q][t]);
+        });
     }
   }
   if constexpr (kOut > 0) {
-    if (t < kHexes) {
+    constexpr int kNodes = kOwn * kOwn * kOwn, kItems = (kOut * kNodes + kT - 1) / kT;
+    double v[kItems];
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        if constexpr (kVec) {
+    for (int i = 0; i < kItems; ++i) v[i] = 0.0;
 #pragma unroll
-          for (int i = 0; i < 3; ++i) sm[(kOut * c + i) * kT + t] = F[c][i];
+    for (int h = 0; h < 2; ++h) {  // the hexes' lower, then upper corners
+      if (h) __syncthreads();      // the lower ones have been read
+      if (t < kHexes) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if constexpr (kVec) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) sc[(kOut * c + i) * kT + t] = F[4 * h + c][i];
+          }
+          if constexpr (kScal) sc[(kOut * c + kOut - 1) * kT + t] = S[4 * h + c];
         }
-        if constexpr (kScal) sm[(kOut * c + kOut - 1) * kT + t] = S[c];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < kItems; ++i) {
+        const int w = t + i * kT;
+        if (w >= kOut * kNodes) break;
+        const int n = w / kOut, o = w - kOut * n;
+        const int a = n % kOwn, b = n / kOwn % kOwn, c = n / (kOwn * kOwn);
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {  // the node is corner cc + 4 h of hex (a + 1 - bits)
+          const int hh = (a + 1 - (cc & 1)) + kHex * ((b + 1 - (cc >> 1)) + kHex * (c + 1 - h));
+          v[i] += sc[(kOut * cc + o) * kT + hh];
+        }
       }
     }
-    __syncthreads();
-    constexpr int kNodes = kOwn * kOwn * kOwn;
-    for (int w = t; w < kOut * kNodes; w += kT) {
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const int w = t + i * kT;
+      if (w >= kOut * kNodes) break;
       const int n = w / kOut, o = w - kOut * n;
       const int a = n % kOwn, b = n / kOwn % kOwn, c = n / (kOwn * kOwn);
       const int id = ids[(a + 1) + kPts * ((b + 1) + kPts * (c + 1))];
       if (id < 0) continue;
-      double v = 0.0;
-#pragma unroll
-      for (int cc = 0; cc < 8; ++cc) {  // the node is corner cc of hex (a + 1 - bits of cc)
-        const int hh = (a + 1 - (cc & 1)) + kHex * ((b + 1 - ((cc >> 1) & 1)) + kHex * (c + 1 - (cc >> 2)));
-        v += sm[(kOut * cc + o) * kT + hh];
-      }
       if constexpr (kRes) {
         const int k = A.lidx ? A.lidx[id] : -1;
-        A.out[3 * (size_t)id + o] = v - (k >= 0 ? A.load_f[3 * (size_t)k + o] : 0.0);
+        A.out[3 * (size_t)id + o] = v[i] - (k >= 0 ? A.load_f[3 * (size_t)k + o] : 0.0);
       } else if constexpr (kPnG) {
-        if (o < 3) A.out[3 * (size_t)id + o] = v;
-        else A.out2[id] = v;
+        if (o < 3) A.out[3 * (size_t)id + o] = v[i];
+        else A.out2[id] = v[i];
       } else {
-        A.out[id] = v;
+        A.out[id] = v[i];
       }
     }
   }
@@ -307,15 +346,26 @@ __global__ __launch_bounds__(kT) void k_box_tile(BoxTileArgs A) {
 
 }  // namespace
 
-hipError_t launch_box_tile(int mode, const BoxTileArgs& a, hipStream_t s) {
+template <int MODE>
+static void launch(bool simp, const BoxTileArgs& a, hipStream_t s) {
   const int grid = a.bx * a.by * a.bz;
+  if (simp) k_box_tile<MODE, true><<<grid, kT, 0, s>>>(a);
+  else k_box_tile<MODE, false><<<grid, kT, 0, s>>>(a);
+}
+
+hipError_t launch_box_tile(int mode, const BoxTileArgs& a, hipStream_t s) {
+  // integer SIMP exponents; in the p-norms also an integer p and, for the relaxed von Mises
+  // measure, q = 1/2
+  bool simp = a.m.model == kPenaltySimp && a.m.pint > 0;
+  if (mode == kTilePNorm || mode == kTilePNormGrad)
+    simp = simp && a.pn >= 1.0 && a.pn <= 16.0 && a.pn == std::floor(a.pn) && (a.measure == 0 || a.q == 0.5);
   switch (mode) {
-    case kTileResidual: k_box_tile<kTileResidual><<<grid, kT, 0, s>>>(a); break;
-    case kTileEnergy: k_box_tile<kTileEnergy><<<grid, kT, 0, s>>>(a); break;
-    case kTileEnergyGradZ: k_box_tile<kTileEnergyGradZ><<<grid, kT, 0, s>>>(a); break;
-    case kTilePNorm: k_box_tile<kTilePNorm><<<grid, kT, 0, s>>>(a); break;
-    case kTilePNormGrad: k_box_tile<kTilePNormGrad><<<grid, kT, 0, s>>>(a); break;
-    case kTileAdjZ: k_box_tile<kTileAdjZ><<<grid, kT, 0, s>>>(a); break;
+    case kTileResidual: launch<kTileResidual>(simp, a, s); break;
+    case kTileEnergy: launch<kTileEnergy>(simp, a, s); break;
+    case kTileEnergyGradZ: launch<kTileEnergyGradZ>(simp, a, s); break;
+    case kTilePNorm: launch<kTilePNorm>(simp, a, s); break;
+    case kTilePNormGrad: launch<kTilePNormGrad>(simp, a, s); break;
+    case kTileAdjZ: launch<kTileAdjZ>(simp, a, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
