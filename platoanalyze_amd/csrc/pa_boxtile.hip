@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kT, 3) void k_box_tile(BoxTileArgs A) {
         const double mp = SIMP ? powi(mval, pni) : pow_of(mval, A.pn, pni);
         sum += mp * A.vol;
         if constexpr (kPnG) {
-          const double k = A.pscale * A.vol * A.pn;
+          const double k = *A.pscale * A.vol * A.pn;
           cf = k * (mval > 0.0 ? mp / mval : 0.0) * cu;
           cs = 0.25 * k * mp * cz;
         }

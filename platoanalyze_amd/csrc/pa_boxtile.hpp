@@ -22,7 +22,8 @@ struct BoxTileArgs {
   const double* load_f;
   double scale;         // factor of the energy gradient (1, or -1 for the total derivative)
   int measure;          // p-norm: 0 Voigt norm of the weighted stress, 1 relaxed von Mises
-  double pn, q, pscale;
+  double pn, q;
+  const double* pscale;  // factor of the p-norm gradients, on the device
   Material m;
 };
 

@@ -235,6 +235,10 @@ struct pa_problem {
   bool box_res = true;  // lattice FP64 residual (k_box_res); PA_BOX_RES=0 keeps the chunk kernel
   int box_grid_res = 1024;
   double* host_scal = nullptr;
+  // work that a call left queued (see settle)
+  bool queued = false;
+  hipEvent_t queued_event = nullptr;
+  hipStream_t queued_stream = nullptr;
 
   pa::Material material() const {
     const double c = E / ((1.0 + nu) * (1.0 - 2.0 * nu));
@@ -283,6 +287,7 @@ struct pa_problem {
   }
   ~pa_problem() {
     if (host_scal) (void)hipHostFree(host_scal);
+    if (queued_event) (void)hipEventDestroy(queued_event);
   }
 };
 
@@ -301,10 +306,34 @@ static int grid_for(size_t n, int per_block = 256, int cap = 4096) {
   return (int)std::max<size_t>(1, std::min<size_t>(g, (size_t)cap));
 }
 
+// A call may return with work queued that uses the handle's partial sums and scalars.  On the
+// same stream the next call queues behind it; on another stream it waits for that work first
+// (by its event: the old stream may be gone).
+static int settle(pa_handle h) {
+  if (!h->queued || h->stream == h->queued_stream) return PA_OK;
+  h->queued = false;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // the new stream may be capturing
+  PA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  const hipError_t e = hipEventSynchronize(h->queued_event);
+  PA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  PA_HIP(e);
+  return PA_OK;
+}
+static int mark_queued(pa_handle h) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  PA_HIP(hipStreamIsCapturing(h->stream, &st));
+  if (st != hipStreamCaptureStatusNone) return PA_OK;  // queued when the graph is launched
+  if (!h->queued_event) PA_HIP(hipEventCreateWithFlags(&h->queued_event, hipEventDisableTiming));
+  PA_HIP(hipEventRecord(h->queued_event, h->stream));
+  h->queued = true;
+  h->queued_stream = h->stream;
+  return PA_OK;
+}
+
 static int ready(pa_handle h) {
   if (!h) return fail(PA_ERR_ARG, "null handle");
   if (!h->finalized) return fail(PA_ERR_STATE, "pa_finalize has not been called");
-  return PA_OK;
+  return settle(h);
 }
 
 extern "C" {
@@ -2578,23 +2607,36 @@ int pa_solution_deflated(pa_handle h, const double* z, double* u, double* vals, 
 }
 
 // ---------------------------------------------------------------- stress p-norm + adjoint
-static int pnorm_value(pa_handle h, const double* u, const double* z, int measure, double pn, double q, double* S) {
-  if (box_tiles(h)) {
+// The p-norm's sum S (read: into host_scal, valid after a wait) and the factor of its gradients
+// into scal[kPScale]: the gradients need no wait for the value.
+static int pnorm_sum(pa_handle h, const double* u, const double* z, int measure, double pn, double q, bool read) {
+  const bool tiles = box_tiles(h);
+  if (tiles) {
     pa::BoxTileArgs a = tile_args(h, u, z);
     a.measure = measure;
     a.pn = pn;
     a.q = q;
     PA_HIP(pa::launch_box_tile(pa::kTilePNorm, a, h->stream));
-    return energy_value(h, S, true);
+  } else {
+    pa::ChunkArgs a = h->chunk_args();
+    a.u = u;
+    a.z = z;
+    a.measure = measure;
+    a.pn = pn;
+    a.q = q;
+    PA_HIP(pa::launch_chunk(h->code_bits, pa::kModePNorm, a, h->stream));
   }
-  pa::ChunkArgs a = h->chunk_args();
-  a.u = u;
-  a.z = z;
-  a.measure = measure;
-  a.pn = pn;
-  a.q = q;
-  PA_HIP(pa::launch_chunk(h->code_bits, pa::kModePNorm, a, h->stream));
-  return energy_value(h, S);
+  pa::k_sum_pnorm<<<1, pa::kSumThreads, 0, h->stream>>>(tiles ? h->box_tile_part.p : h->chunk_partials.p,
+                                                        tiles ? (int)h->box_tile_part.n : h->chunks.count, h->scal.p,
+                                                        read ? h->host_scal : nullptr, pn);
+  PA_HIP(hipGetLastError());
+  return PA_OK;
+}
+// the p-norm itself, after the stream's work
+static int pnorm_read(pa_handle h, double pn, double* value) {
+  PA_HIP(hipStreamSynchronize(h->stream));
+  *value = std::pow(h->host_scal[pa::kEnergy], 1.0 / pn);
+  return PA_OK;
 }
 
 static int check_pnorm_args(int measure, double& pn, double q) {
@@ -2610,36 +2652,34 @@ int pa_stress_pnorm(pa_handle h, const double* u, const double* z, int measure, 
   if (int rc = ready(h)) return rc;
   if (!u || !z) return fail(PA_ERR_ARG, "pa_stress_pnorm: null pointer");
   if (int rc = check_pnorm_args(measure, pn, q)) return rc;
-  double S = 0.0;
-  if (int rc = pnorm_value(h, u, z, measure, pn, q, &S)) return rc;
-  if (value) *value = std::pow(S, 1.0 / pn);
-  if (!dfdu && !dfdz) return PA_OK;
-  if (int rc = ensure_solver_ws(h)) return rc;
+  const bool grad = dfdu || dfdz;
+  if (grad)
+    if (int rc = ensure_solver_ws(h)) return rc;
+  if (int rc = pnorm_sum(h, u, z, measure, pn, q, value)) return rc;
   double* gu = dfdu ? dfdu : h->w_r.p;
   double* gz = dfdz ? dfdz : h->w_z.p;  // w_z holds >= num_nodes doubles
-  const double pscale = S > 0.0 ? std::pow(S, (1.0 - pn) / pn) / pn : 0.0;
-  if (box_tiles(h)) {
+  if (grad && box_tiles(h)) {
     pa::BoxTileArgs a = tile_args(h, u, z);
     a.measure = measure;
     a.pn = pn;
     a.q = q;
-    a.pscale = pscale;
+    a.pscale = h->scal.p + pa::kPScale;
     a.out = gu;
     a.out2 = gz;
     PA_HIP(pa::launch_box_tile(pa::kTilePNormGrad, a, h->stream));
-    return PA_OK;
+  } else if (grad) {
+    pa::ChunkArgs a = h->chunk_args();
+    a.u = u;
+    a.z = z;
+    a.measure = measure;
+    a.pn = pn;
+    a.q = q;
+    a.pscale = h->scal.p + pa::kPScale;
+    a.out_vec = gu;
+    a.out_vec2 = gz;
+    PA_HIP(pa::launch_chunk(h->code_bits, pa::kModePNormGrad, a, h->stream));
   }
-  pa::ChunkArgs a = h->chunk_args();
-  a.u = u;
-  a.z = z;
-  a.measure = measure;
-  a.pn = pn;
-  a.q = q;
-  a.pscale = pscale;
-  a.out_vec = gu;
-  a.out_vec2 = gz;
-  PA_HIP(pa::launch_chunk(h->code_bits, pa::kModePNormGrad, a, h->stream));
-  return PA_OK;
+  return value ? pnorm_read(h, pn, value) : mark_queued(h);
 }
 
 int pa_stress_pnorm_gradient_x(pa_handle h, const double* u, const double* z, int measure, double pn, double q,
@@ -2647,19 +2687,17 @@ int pa_stress_pnorm_gradient_x(pa_handle h, const double* u, const double* z, in
   if (int rc = ready(h)) return rc;
   if (!u || !z || !dfdx) return fail(PA_ERR_ARG, "pa_stress_pnorm_gradient_x: null pointer");
   if (int rc = check_pnorm_args(measure, pn, q)) return rc;
-  double S = 0.0;
-  if (int rc = pnorm_value(h, u, z, measure, pn, q, &S)) return rc;
-  if (value) *value = std::pow(S, 1.0 / pn);
+  if (int rc = pnorm_sum(h, u, z, measure, pn, q, value)) return rc;
   pa::ChunkArgs a = h->chunk_args();
   a.u = u;
   a.z = z;
   a.measure = measure;
   a.pn = pn;
   a.q = q;
-  a.pscale = S > 0.0 ? std::pow(S, (1.0 - pn) / pn) / pn : 0.0;
+  a.pscale = h->scal.p + pa::kPScale;
   a.out_vec = dfdx;
   PA_HIP(pa::launch_chunk(h->code_bits, pa::kModePNormGradX, a, h->stream));
-  return PA_OK;
+  return value ? pnorm_read(h, pn, value) : mark_queued(h);
 }
 
 int pa_dRdz_T_apply(pa_handle h, const double* u, const double* lambda, const double* z, double* out) {

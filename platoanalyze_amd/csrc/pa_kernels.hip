@@ -267,8 +267,8 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
         double tau[6];
         iso_stress(A.m, t, tau);
         const double mpm1 = mval > 0.0 ? mp / mval : 0.0;
-        const double fv = A.pscale * vol * mp;
-        const double fs = A.pscale * vol * A.pn * mpm1 * cu;
+        const double fv = *A.pscale * vol * mp;
+        const double fs = *A.pscale * vol * A.pn * mpm1 * cu;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           if (ln[b] >= nr) continue;
@@ -285,8 +285,8 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
       } else {
         // dS/du_a = vol p m^(p-1) c_u B_a^T C0 t ; dS/dz_a = vol p m^p c_z / 4
         const double mpm1 = mval > 0.0 ? mp / mval : 0.0;
-        const double fu = A.pscale * vol * A.pn * mpm1 * cu;
-        const double fz = A.pscale * vol * A.pn * mp * cz * 0.25;
+        const double fu = *A.pscale * vol * A.pn * mpm1 * cu;
+        const double fz = *A.pscale * vol * A.pn * mp * cz * 0.25;
         double tau[6];
         iso_stress(A.m, t, tau);
 #pragma unroll

@@ -170,10 +170,11 @@ struct ChunkArgs {
   int max_blocks;
   int max_nodes;
   // stress p-norm F = (sum vol m^p)^(1/p): measure 0 = Voigt norm of sigma_w (the
-  // reference StressPNorm), 1 = relaxed von Mises rho^q vm(sigma0); pscale multiplies
+  // reference StressPNorm), 1 = relaxed von Mises rho^q vm(sigma0); pscale (device) multiplies
   // the gradients (pow(S,(1-p)/p)/p, known after the value pass)
   int measure;
-  double pn, q, pscale;
+  double pn, q;
+  const double* pscale;
   double scale;       // factor of the energy gradient (1; -1 for the total derivative)
   Material m;
 };

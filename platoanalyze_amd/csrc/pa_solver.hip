@@ -292,6 +292,16 @@ __global__ __launch_bounds__(kSumThreads) void k_sum(const double* partials, int
   }
 }
 
+__global__ __launch_bounds__(kSumThreads) void k_sum_pnorm(const double* partials, int n, double* scal, double* host, double pn) {
+  __shared__ double sh[kSumThreads / 64];
+  const double S = sum_partials_wide<kSumThreads>(partials, n, sh);
+  if (threadIdx.x == 0) {
+    scal[kEnergy] = S;
+    scal[kPScale] = S > 0.0 ? pow(S, (1.0 - pn) / pn) / pn : 0.0;
+    if (host) host[kEnergy] = S;
+  }
+}
+
 // 3x3 block-diagonal inverse (cofactors)
 __global__ __launch_bounds__(kT) void k_diag_inv(const double* vals, const int* diag_slot, double* dinv,
                                                  int nnodes) {

@@ -6,7 +6,7 @@ namespace pa {
 
 // slots of the device scalar array used by the PCG kernels
 enum ScalarSlot { kRZ = 0, kPQ = 1, kAlpha = 2, kBeta = 3, kRR = 4, kBB = 5, kDot0 = 6, kDot1 = 7,
-                  kEnergy = 8, kNumScal = 16 };
+                  kEnergy = 8, kPScale = 9, kNumScal = 16 };
 
 // partial arrays of the solver (kRedBlocks doubles each) in one device buffer
 enum PartialSlot { kPPQ = 0, kPRZ0 = 1, kPRZ1 = 2, kPRR = 3, kPBB = 4, kPDot = 5, kNumPartialSlots = 6 };
@@ -31,6 +31,9 @@ __global__ void k_pcg_init(const double* r, double* z, double* p, const double* 
 __global__ void k_dot(const double* a, const double* b, size_t n, double* P);
 constexpr int kSumThreads = 1024;
 __global__ void k_sum(const double* partials, int n, double* scal, int slot, double* host);
+// k_sum of the p-norm sum S into scal[kEnergy], and the factor of its gradient,
+// d(S^(1/p))/dS = S^((1-p)/p) / p (0 for S = 0), into scal[kPScale].
+__global__ void k_sum_pnorm(const double* partials, int n, double* scal, double* host, double pn);
 __global__ void k_diag_inv(const double* vals, const int* diag_slot, double* dinv, int nnodes);
 __global__ void k_add_load(double* y, const int* nodes, const double* f, int n, double s);
 __global__ void k_fill(double* y, size_t n, double v);
