@@ -497,7 +497,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * SPLIT : kT) void k_conv_tile(ConvArgs 
 //
 // Before, each (tap, 16 input channels) had work-groups of its own that gathered X and dY
 // from global memory 2 and 4 bytes a lane and added with atomics: 65x33x33, batch 4, base
-// 16: 3300 us for the 15 layers and 515 us for the bias sums; now 378 us and 113 us for the slab sums.
+// 16: 3300 us for the 15 layers and 515 us for the bias sums; now 378 us and 85 us for the slab sums.
 // LDS reads (one operand per two MFMAs) and the staging loads bound it.
 constexpr int kWgradBlocks = 512;   // work-groups of one layer: two per CU
 constexpr int kWgradLds = 64 * 1024;  // staged tiles, so that two work-groups share a CU
@@ -654,7 +654,9 @@ __global__ __launch_bounds__(kT, 2) void k_wgrad(WgradArgs A, WgradTile T) {
 }
 
 // dst[e] = sum of the slabs' e-th values: 16 lanes of four values, 16 runs of slabs added in
-// parallel, then in order.
+// parallel, then in order.  A run's loads are issued eight at a time: one by one, 512 slabs of
+// a small layer were a chain of 32 memory latencies (65x33x33, batch 4, base 16, the 15
+// layers: 113 us, now 85).
 __global__ __launch_bounds__(kT) void k_slab_sum(const float* __restrict__ part, int slabs, size_t n,
                                                  float* __restrict__ dst) {
   __shared__ float4 sh[16][16];
@@ -664,12 +666,18 @@ __global__ __launch_bounds__(kT) void k_slab_sum(const float* __restrict__ part,
     const size_t e = e0 + 4 * l;  // n is a multiple of 8 (channels), and so are the offsets
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (e < n)
-      for (int b = b0; b < b1; ++b) {
-        const float4 p = *reinterpret_cast<const float4*>(part + (size_t)b * n + e);
-        v.x += p.x;
-        v.y += p.y;
-        v.z += p.z;
-        v.w += p.w;
+      for (int b = b0; b < b1; b += 8) {
+        float4 p[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          p[k] = b + k < b1 ? *reinterpret_cast<const float4*>(part + (size_t)(b + k) * n + e) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          v.x += p[k].x;
+          v.y += p[k].y;
+          v.z += p[k].z;
+          v.w += p[k].w;
+        }
       }
     sh[r][l] = v;
     __syncthreads();
@@ -1012,10 +1020,12 @@ struct pa_unet_s {
   Dev<double> partials;
   Dev<float> split;  // split-reduction slices of the small convolutions
   double* host_partials = nullptr;
+  hipEvent_t loss_event = nullptr;  // the loss has arrived
   int step = 0;
   hipStream_t stream = nullptr;
   std::string err;
   ~pa_unet_s() {
+    if (loss_event) (void)hipEventDestroy(loss_event);
     if (host_partials) (void)hipHostFree(host_partials);
   }
 };
@@ -1148,8 +1158,13 @@ pa::unet::ConvArgs fwd_args(pa_unet h, const Layer& l) {
   return a;
 }
 
-int forward(pa_unet h) {
-  for (const Layer& l : h->L) PA_UHIP(h, pa::unet::launch_conv(fwd_args(h, l), h->stream));
+// y: where the output goes, if not to h->out
+int forward(pa_unet h, float* y = nullptr) {
+  for (const Layer& l : h->L) {
+    pa::unet::ConvArgs a = fwd_args(h, l);
+    if (y && a.Yf) a.Yf = y;
+    PA_UHIP(h, pa::unet::launch_conv(a, h->stream));
+  }
   return PA_OK;
 }
 
@@ -1228,11 +1243,16 @@ int loss_and_grad(pa_unet h, const float* target, double* loss) {
   PA_UHIP(h, pa::unet::launch_mse(h->out.p, target, n, h->dout.p, h->partials.p, grid, h->stream));
   PA_UHIP(h, hipMemcpyAsync(h->host_partials, h->partials.p, grid * sizeof(double), hipMemcpyDeviceToHost,
                             h->stream));
-  PA_UHIP(h, hipStreamSynchronize(h->stream));
+  if (!h->loss_event) PA_UHIP(h, hipEventCreateWithFlags(&h->loss_event, hipEventDisableTiming));
+  PA_UHIP(h, hipEventRecord(h->loss_event, h->stream));
+  // the backward pass is queued before the host waits for the loss, so the GPU does not wait
+  // for the host
+  const int rc = backward(h);
+  PA_UHIP(h, hipEventSynchronize(h->loss_event));
   double s = 0.0;
   for (int i = 0; i < grid; ++i) s += h->host_partials[i];
   if (loss) *loss = s;
-  return PA_OK;
+  return rc;
 }
 
 }  // namespace
@@ -1316,9 +1336,12 @@ int pa_unet_params(pa_unet h, float* dst, const float* src) {
 int pa_unet_forward(pa_unet h, const float* x, int batch, float* y) {
   if (!h || !x || !y || batch < 1) return ufail(h, PA_ERR_ARG, "pa_unet_forward: bad argument");
   if (int rc = load_input(h, x, batch)) return rc;
-  if (int rc = forward(h)) return rc;
-  PA_UHIP(h, hipMemcpyAsync(y, h->out.p, (size_t)batch * h->g[0].count() * kOutCh * sizeof(float),
-                            hipMemcpyDeviceToDevice, h->stream));
+  // the last layer stores 16 bytes a lane, so its output goes straight to a y aligned to that
+  const bool direct = reinterpret_cast<size_t>(y) % 16 == 0;
+  if (int rc = forward(h, direct ? y : nullptr)) return rc;
+  if (!direct)
+    PA_UHIP(h, hipMemcpyAsync(y, h->out.p, (size_t)batch * h->g[0].count() * kOutCh * sizeof(float),
+                              hipMemcpyDeviceToDevice, h->stream));
   return PA_OK;
 }
 
@@ -1327,7 +1350,6 @@ int pa_unet_gradient(pa_unet h, const float* x, const float* target, int batch, 
   if (int rc = load_input(h, x, batch)) return rc;
   if (int rc = forward(h)) return rc;
   if (int rc = loss_and_grad(h, target, loss)) return rc;
-  if (int rc = backward(h)) return rc;
   if (grad) PA_UHIP(h, hipMemcpyAsync(grad, h->G.p, h->nparams * sizeof(float), hipMemcpyDeviceToDevice, h->stream));
   return PA_OK;
 }
