@@ -648,7 +648,15 @@ __device__ __forceinline__ void jac_elements(const ChunkArgs& A, const JacChunk&
     tet_gradients(x, g, vol);
     rho = rho / 4.0;
     const double w = penalty_w_as<SIMP>(A.m, rho);
-    const double vl = vol * w * A.m.c01, vm = vol * w * A.m.c33;
+    // scaled to the fixed-point unit S, a power of two: the same bits as scaling every entry
+    const double vl = S * (vol * w * A.m.c01), vm = S * (vol * w * A.m.c33);
+    // an element whose entries are not finite adds nothing (as the conversion of a NaN did)
+    double all = vl + vm;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) all += g[a][d];
+    if (!(fabs(all) < INFINITY)) continue;
     bool own[4];
     int ro[4];
 #pragma unroll
@@ -675,7 +683,7 @@ __device__ __forceinline__ void jac_elements(const ChunkArgs& A, const JacChunk&
 #pragma unroll
       for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) lds_add_fixed64(dst + 3 * i + j, rowb ? kv[j][i] : kv[i][j], S);
+        for (int j = 0; j < 3; ++j) lds_add_rounded64(dst + 3 * i + j, rowb ? kv[j][i] : kv[i][j]);
     }
   }
 }
