@@ -889,8 +889,11 @@ __global__ __launch_bounds__(256, 6) void k_boxmf_apply(BoxMfArgs A) {
 // of a hex from slot q of its record; each tet's force is formed in FP32 from FP32 p and
 // weights, summed in FP32 over the four tets of each path and in FP64 over the paths, in
 // a fixed order.
+// Registers bound the waves in flight (124 to 132, three or four a SIMD).  A floor of four
+// waves made the compiler spill and schedule worse: 256x128x128 hexes, product 208 us with it
+// and 187 without, Jacobi step 369 and 298; 128x64x64 24.0 and 20.6, 37.4 and 32.7.
 template <int OUT>
-__global__ __launch_bounds__(256, 4) void k_boxmf_apply_kuhn(BoxMfArgs A) {
+__global__ __launch_bounds__(256) void k_boxmf_apply_kuhn(BoxMfArgs A) {
   __shared__ double sh[4];
   const int px = A.nx + 2, pxy = (A.nx + 2) * (A.ny + 2);
   const float ih[3] = {A.ih[0], A.ih[1], A.ih[2]};

@@ -14,8 +14,8 @@
 // u and z) at twelve waves a CU: registers, as LDS holds the corner contributions of half the
 // corners at a time.  128x64x64 hexes, one thread per row with lattice copies and a weight
 // array -> bricks with all corners and every penalty model's code -> this: residual 62 -> 48.5
-// -> 39 us a call, energy and gradient (chunk kernel) 149 -> 60 -> 51; p-norm adjoint
-// gradient, 64x32x32, 182 -> 124 -> 109.  Four waves a SIMD spill (residual 51 us, gradient 109).
+// -> 36 us a call, energy and gradient (chunk kernel) 149 -> 60 -> 49; p-norm adjoint
+// gradient, 64x32x32, 182 -> 124 -> 104 (93 since its factor is summed on the device).  Four waves a SIMD spill (residual 51 us, gradient 109).
 #include "pa_boxtile.hpp"
 
 #include <cmath>
