@@ -15,7 +15,8 @@
 // corners at a time.  128x64x64 hexes, one thread per row with lattice copies and a weight
 // array -> bricks with all corners and every penalty model's code -> this: residual 62 -> 48.5
 // -> 36 us a call, energy and gradient (chunk kernel) 149 -> 60 -> 49; p-norm adjoint
-// gradient, 64x32x32, 182 -> 124 -> 104 (93 since its factor is summed on the device).  Four waves a SIMD spill (residual 51 us, gradient 109).
+// gradient, 64x32x32, 182 -> 124 -> 104 (93 since its factor is summed on the device).
+// Four waves a SIMD spill (residual 51 us, gradient 109).
 #include "pa_boxtile.hpp"
 
 #include <cmath>
