@@ -238,7 +238,6 @@ struct pa_problem {
   // work that a call left queued (see settle)
   bool queued = false;
   hipEvent_t queued_event = nullptr;
-  hipStream_t queued_stream = nullptr;
 
   pa::Material material() const {
     const double c = E / ((1.0 + nu) * (1.0 - 2.0 * nu));
@@ -306,15 +305,29 @@ static int grid_for(size_t n, int per_block = 256, int cap = 4096) {
   return (int)std::max<size_t>(1, std::min<size_t>(g, (size_t)cap));
 }
 
-// A call may return with work queued that uses the handle's partial sums and scalars.  On the
-// same stream the next call queues behind it; on another stream it waits for that work first
-// (by its event: the old stream may be gone).
+// A call may return with work queued that uses the handle's partial sums and scalars.  The
+// stream of the next call waits for that work's event.  Events and not handles tell streams
+// apart: a new stream may have the handle of a destroyed one.  On the event's own stream the
+// wait costs nothing; a stream under capture cannot wait for work outside its graph, so there
+// the host does.
 static int settle(pa_handle h) {
-  if (!h->queued || h->stream == h->queued_stream) return PA_OK;
-  h->queued = false;
+  if (!h->queued) return PA_OK;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // the new stream may be capturing
   PA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-  const hipError_t e = hipEventSynchronize(h->queued_event);
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  hipError_t e = hipEventQuery(h->queued_event);
+  if (e == hipSuccess) {
+    h->queued = false;
+  } else if (e == hipErrorNotReady) {
+    (void)hipGetLastError();  // not an error of the next launch
+    e = hipStreamIsCapturing(h->stream, &st);
+    if (e == hipSuccess && st == hipStreamCaptureStatusNone) {
+      e = hipStreamWaitEvent(h->stream, h->queued_event, 0);
+    } else if (e == hipSuccess) {
+      e = hipEventSynchronize(h->queued_event);
+      h->queued = e != hipSuccess;
+    }
+  }
   PA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
   PA_HIP(e);
   return PA_OK;
@@ -326,7 +339,6 @@ static int mark_queued(pa_handle h) {
   if (!h->queued_event) PA_HIP(hipEventCreateWithFlags(&h->queued_event, hipEventDisableTiming));
   PA_HIP(hipEventRecord(h->queued_event, h->stream));
   h->queued = true;
-  h->queued_stream = h->stream;
   return PA_OK;
 }
 
