@@ -110,7 +110,11 @@ int pa_set_graph(pa_handle h, const int32_t* rowmap, const int32_t* colidx);
  * once after the set-up calls and before any compute call. */
 int pa_finalize(pa_handle h);
 
-/* HIP stream for all later launches (hipStream_t passed as void*; NULL = default). */
+/* HIP stream for all later launches (hipStream_t passed as void*; NULL = default).  Calls
+ * share the handle's work arrays: one on another stream first waits for what earlier calls
+ * left queued there.  Calls captured into a graph use the arrays when the graph is launched,
+ * which the library does not see: the caller orders graph launches with each other and with
+ * other calls on the handle. */
 int pa_set_stream(pa_handle h, void* hip_stream);
 
 int pa_graph_size(pa_handle h, int* num_rows, int* nnz_blocks);

@@ -305,11 +305,11 @@ static int grid_for(size_t n, int per_block = 256, int cap = 4096) {
   return (int)std::max<size_t>(1, std::min<size_t>(g, (size_t)cap));
 }
 
-// A call may return with work queued that uses the handle's partial sums and scalars.  The
-// stream of the next call waits for that work's event.  Events and not handles tell streams
-// apart: a new stream may have the handle of a destroyed one.  On the event's own stream the
-// wait costs nothing; a stream under capture cannot wait for work outside its graph, so there
-// the host does.
+// A call may return with work queued that uses the handle's own arrays (partial sums, scalars,
+// lattice copies, solver vectors); it then ends with mark_queued.  The stream of the next call
+// waits for that work's event.  Events and not handles tell streams apart: a new stream may
+// have the handle of a destroyed one.  On the event's own stream the wait costs nothing; a
+// stream under capture cannot wait for work outside its graph, so there the host does.
 static int settle(pa_handle h) {
   if (!h->queued) return PA_OK;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // the new stream may be capturing
@@ -688,6 +688,9 @@ static int residual(pa_handle h, const double* u, const double* z, double* R, bo
   return run_chunk(h, pa::kModeResidual, u, z, nullptr, R, sub);
 }
 
+// whether it goes through the handle's lattice copies and weights
+static bool residual_scratch(pa_handle h) { return h->box_fast && h->box_res && !box_tiles(h); }
+
 static int sub_load(pa_handle h, double* R, double s) {
   if (h->nload == 0) return PA_OK;
   pa::k_add_load<<<grid_for(h->nload), 256, 0, h->stream>>>(R, h->load_nodes.p, h->load_f.p, h->nload, s);
@@ -698,13 +701,15 @@ static int sub_load(pa_handle h, double* R, double s) {
 int pa_vf_value(pa_handle h, const double* u, const double* z, double* R) {
   if (int rc = ready(h)) return rc;
   if (!u || !z || !R) return fail(PA_ERR_ARG, "pa_vf_value: null pointer");
-  return residual(h, u, z, R, true);
+  if (int rc = residual(h, u, z, R, true)) return rc;
+  return residual_scratch(h) ? mark_queued(h) : PA_OK;
 }
 
 int pa_vf_gradient_u(pa_handle h, const double* u, const double* z, double* vals, double* R) {
   if (int rc = ready(h)) return rc;
   if (!z || !vals || (R && !u)) return fail(PA_ERR_ARG, "pa_vf_gradient_u: null pointer");
-  return assemble_jacobian(h, u, z, vals, R);
+  if (int rc = assemble_jacobian(h, u, z, vals, R)) return rc;
+  return h->box_fast && !h->box_jac.n ? mark_queued(h) : PA_OK;  // the lattice copies and weights
 }
 
 int pa_vf_gradient_z(pa_handle h, const double* u, const double* z, double* vals_t) {
@@ -820,8 +825,7 @@ int pa_volume(pa_handle h, const double* z, int model, double exponent, double m
   a.out_vec = dvdx ? dvdx : h->w_p.p;   // w_p holds 3N doubles
   a.out_vec2 = dvdz ? dvdz : h->w_z.p;  // w_z holds >= N doubles
   PA_HIP(pa::launch_chunk(h->code_bits, pa::kModeVolume, a, h->stream));
-  if (value) return energy_value(h, value);
-  return PA_OK;
+  return value ? energy_value(h, value) : mark_queued(h);
 }
 
 // --------------------------------------------------------------- scalar function
@@ -848,7 +852,8 @@ int pa_sf_value(pa_handle h, const double* u, const double* z, double* value) {
 int pa_sf_gradient_u(pa_handle h, const double* u, const double* z, double* g) {
   if (int rc = ready(h)) return rc;
   if (!u || !z || !g) return fail(PA_ERR_ARG, "pa_sf_gradient_u: null pointer");
-  return residual(h, u, z, g, false);
+  if (int rc = residual(h, u, z, g, false)) return rc;
+  return residual_scratch(h) ? mark_queued(h) : PA_OK;
 }
 
 // g = scale times the partial dC/dz, and C
@@ -867,7 +872,7 @@ static int energy_gradient(pa_handle h, const double* u, const double* z, double
     a.scale = scale;
     PA_HIP(pa::launch_chunk(h->code_bits, pa::kModeEnergyGradZ, a, h->stream));
   }
-  return value ? energy_value(h, value, tiles) : PA_OK;
+  return value ? energy_value(h, value, tiles) : mark_queued(h);  // its partials
 }
 
 int pa_sf_gradient_z(pa_handle h, const double* u, const double* z, double* g, double* value) {
@@ -2477,7 +2482,7 @@ int pa_smooth(pa_handle h, const double* z, double* u, int steps, double omega) 
     if (int rc = residual(h, u, z, h->m_R.p, false)) return rc;  // K u
     PA_HIP(pa::launch_jacobi_step(u, h->m_R.p, h->m_dinv.p, h->bcmask.p, h->nn, omega, h->stream));
   }
-  return PA_OK;
+  return mark_queued(h);
 }
 
 int pa_solution(pa_handle h, const double* z, double* u, double* vals, const pa_solver_opts* o,
@@ -2780,7 +2785,7 @@ int pa_stress_pnorm_gradient(pa_handle h, const double* u, const double* z, int 
   if (int rc = pa_dRdz_T_apply(h, u, lambda, z, h->w_adjz.p)) return rc;
   pa::k_axpy<<<grid_for((size_t)h->nn), 256, 0, h->stream>>>(dfdz, h->w_adjz.p, (size_t)h->nn, -1.0);
   PA_HIP(hipGetLastError());
-  return PA_OK;
+  return mark_queued(h);
 }
 
 int pa_compliance_gradient(pa_handle h, const double* u, const double* z, double* dcdz, double* value) {

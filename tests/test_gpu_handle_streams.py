@@ -57,3 +57,47 @@ def test_gpu_stream_created_after_a_destroyed_one():
     torch.cuda.synchronize()
     for g in got:
         assert float((g - want[0]).abs().max()) <= 1e-12 * float(want[0].abs().max())
+
+
+def _volume_gradient(m, z):
+    """Volume's dV/dz without the value, which leaves partial sums queued."""
+    from platoanalyze_amd import _capi
+
+    g = torch.empty_like(z)
+    m._stream()
+    _capi.call("pa_volume", m.handle, C.c_void_p(z.data_ptr()), 0, 3.0, 1e-3, 1.0, None, C.c_void_p(g.data_ptr()), None)
+    return g
+
+
+@pytest.mark.parametrize("path", ["bricks", "lattice", "chunks"])
+def test_gpu_gradients_then_values_on_another_stream(monkeypatch, path):
+    from platoanalyze_amd.elliptic import PhysicsScalarFunction, VectorFunction, Volume
+
+    print(f"case: queued gradients, then values on another stream, {path}", flush=True)
+    if path == "lattice":
+        monkeypatch.setenv("PA_BOX_RES_KUHN", "0")
+        monkeypatch.setenv("PA_BOX_JAC_KUHN", "0")
+    m, u, z = _model(path != "chunks")
+    f, vf, vol = PhysicsScalarFunction(m), VectorFunction(m), Volume(m, "SIMP", 3.0, 1e-3)
+    v, w = 2.0 * u, 0.5 * z
+    want = [f.gradient_z(v, z), f.value(u, z), _volume_gradient(m, w), vol.value(z), vf.value(v, z), vf.value(u, w)]
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(6):
+        with torch.cuda.stream(a):
+            gz = f.gradient_z(v, z)
+        with torch.cuda.stream(b):
+            energy = f.value(u, z)
+        with torch.cuda.stream(a):
+            gv = _volume_gradient(m, w)
+        with torch.cuda.stream(b):
+            volume = vol.value(z)
+        with torch.cuda.stream(a):
+            r0 = vf.value(v, z)
+        with torch.cuda.stream(b):
+            r1 = vf.value(u, w)
+        torch.cuda.synchronize()
+        assert energy == want[1] and volume == want[3]
+        # the chunk kernels' gradient sums may differ in their order from run to run
+        for got, ref in ((gz, want[0]), (gv, want[2]), (r0, want[4]), (r1, want[5])):
+            assert float((got - ref).abs().max()) <= 1e-12 * float(ref.abs().max())
