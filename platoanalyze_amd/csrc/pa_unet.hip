@@ -378,8 +378,12 @@ __global__ __launch_bounds__(SPLIT ? 64 * SPLIT : kT) void k_conv_tile(ConvArgs 
     f32x4 acc[kConvM][NT], tot[SPLIT ? 1 : kConvM][NT];
     // steps [i, iend) of the step list into acc; the next kConvAhead steps' weights load
     // from L2 while this run is multiplied.  The number of tiles N is a template argument and
-    // not a branch around the products: this compiler does not keep the wait states between
-    // an MFMA and a read of its result when a taken branch shortens the way between them.
+    // not a branch around the products: where a block between an MFMA and a read of its result
+    // rewrites only some of the accumulators, this compiler misses the shortest way round it
+    // and leaves fewer than the 8 wait states that the read needs (built so: down to 1).  The
+    // tail's branches below are sound: each block rewrites all N NT accumulators, so every
+    // way to a read starts in the last block passed.  tests/test_mfma_waits.py checks the
+    // built code's shortest ways (now 10).
     auto run = [&](int i, int iend, auto N) {
 #pragma unroll
       for (int j = 0; j < kConvM; ++j)
