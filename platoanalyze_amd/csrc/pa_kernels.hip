@@ -114,8 +114,11 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
   constexpr bool kAdj = MODE == kModeAdjZ;
   constexpr bool kGx = MODE == kModeGradX, kEGx = MODE == kModeEnergyGradX, kVol = MODE == kModeVolume;
   // one value per element, the same for its four vertices: kept in LDS and gathered by the
-  // rows, or added with atomics where the chunks' lists are too long (no incidences)
-  constexpr bool kGather = kGradZ || kAdj;
+  // rows, or added with atomics where the chunks' lists are too long (no incidences) and in
+  // the instances with every penalty model's code: their three waves a SIMD hide the atomics
+  // but not the rows' phase after them (97x51x45 hexes of five tets, RAMP: energy gradient
+  // 94 us a call with atomics, 108 gathered; adjoint product 56 and 65)
+  constexpr bool kGather = SIMP && (kGradZ || kAdj);
   constexpr bool kReduce = MODE == kModeEnergy || kGradZ || kPnV || kVol;
   constexpr int kBlkW = kGzT ? 3 : (kGx ? 9 : 0);                      // doubles per block in LDS
   constexpr int kRowW = (kRes || kPnG || kEGx || kVol || kPnX) ? 3 : ((kGradZ || kAdj) ? 1 : 0);  // doubles per row
@@ -832,7 +835,7 @@ constexpr int kNtVec = 256;
 template <int BITS, bool SIMP>
 static hipError_t launch_chunk_b(int mode, ChunkArgs a, hipStream_t s) {
   size_t lds = chunk_lds_bytes(mode, a.max_rows, a.max_blocks, a.max_nodes);
-  if (mode == kModeEnergyGradZ || mode == kModeAdjZ) {  // a value per entry instead of per row, if it fits
+  if (SIMP && (mode == kModeEnergyGradZ || mode == kModeAdjZ)) {  // a value per entry instead of per row, if it fits
     const size_t more = sizeof(double) * (size_t)std::max(0, a.max_list - a.max_rows);
     if (lds + more <= 64 * 1024) lds += more;
     else a.inc = nullptr;
