@@ -1306,6 +1306,10 @@ static int solve_mixed(pa_handle h, const double* z, double* u, const double* b,
   // the apply (or the lattice scatter) takes beta from both and the update alpha from the
   // p.q partials, so an iteration has no one-group summing kernels of its own
   if (!conv) PA_HIP(pa::launch_pcgm_init(h->m_r.p, h->m_z.p, h->m_dinv.p, nn, PS(pa::kPRZ0), G, s));
+  // Where k_mf_apply has several rounds of work-groups, each summing both partials of beta
+  // before its loads costs more than one launch that sums them (97x51x45 hexes, RAMP, us an
+  // iteration: graded 70 -> 64, five tets 92 -> 82).
+  const bool sum_rz = !(h->box_fast && h->box_mf) && ma.nchunks > pa::kRedBlocks && !pa::mf_gathers(ma);
   int it = 0;
   bool restart = true;  // the next apply starts the direction from p = z
   while (!conv) {
@@ -1317,6 +1321,12 @@ static int solve_mixed(pa_handle h, const double* z, double* u, const double* b,
     ma.P_rz_new = PS(pa::kPRZ0 + cur);
     ma.P_rz_old = PS(pa::kPRZ0 + (cur ^ 1));
     ma.np_rz = G;
+    if (sum_rz) {
+      pa::k_sum<<<1, pa::kSumThreads, 0, s>>>(ma.P_rz_new, G, h->scal.p, pa::kRZ0 + cur, nullptr);
+      ma.P_rz_new = h->scal.p + pa::kRZ0 + cur;
+      ma.P_rz_old = h->scal.p + pa::kRZ0 + (cur ^ 1);
+      ma.np_rz = 1;
+    }
     const double* Pq = nullptr;
     int npq = 0;
     if (int rc = mf_apply(h, ma, &Pq, &npq)) return rc;

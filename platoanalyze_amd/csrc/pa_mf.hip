@@ -121,8 +121,8 @@ __global__ __launch_bounds__(NT) void k_mf_apply(MfArgs A) {
 
   double beta = 0.0;
   if (!A.first) {
-    double a, b;
-    sum_partials_two<NT>(A.P_rz_new, A.np_rz, A.P_rz_old, A.np_rz, sh, a, b);
+    double a = A.P_rz_new[0], b = A.P_rz_old[0];
+    if (A.np_rz > 1) sum_partials_two<NT>(A.P_rz_new, A.np_rz, A.P_rz_old, A.np_rz, sh, a, b);
     beta = a / b;
   }
   const int c = xcd_map(blockIdx.x, A.nchunks);
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(NT) void k_mf_apply(MfArgs A) {
 // a chunk's 500 to 800 elements.  Graded hexes, against k_mf_apply: 35x19x17 (67830 tets)
 // 9.0 -> 7.0 us an apply, 97x51x45 (1.34 million) 66 -> 55 us an iteration; 256 threads
 // 7.6 us and 58 us.
-template <int NT, bool SIMP_INT>
+template <int NT>
 __global__ __launch_bounds__(NT, 4) void k_mf_gather(MfArgs A) {
   extern __shared__ double smem_d[];
   double* pown = smem_d;  // own-row p (FP64), node table, p at its nodes, forces [entry][4][3]
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(NT, 4) void k_mf_gather(MfArgs A) {
     const int ln[4] = {(int)(ent.x & 0xFFFFu), (int)(ent.x >> 16), (int)(ent.y & 0xFFFFu), (int)(ent.y >> 16)};
     if (k + NT < l1) ent = ents[k + NT];
     float F[4][3];
-    mf_element<SIMP_INT>(A.m, c00, c01, c33, rmin, pp, nd4, xl, ln, F);
+    mf_element<true>(A.m, c00, c01, c33, rmin, pp, nd4, xl, ln, F);
     float4* f = fl + 3 * (k - l0);
     f[0] = make_float4(F[0][0], F[0][1], F[0][2], F[1][0]);
     f[1] = make_float4(F[1][1], F[1][2], F[2][0], F[2][1]);
@@ -454,19 +454,26 @@ int grid_of(size_t n, int cap = 1024) {
 
 }  // namespace
 
+static size_t mf_gather_lds(const MfArgs& a) {
+  return sizeof(double) * 3 * ((a.max_rows + 1) & ~1) + sizeof(float4) * (a.max_nodes + 3 * (size_t)a.max_list) +
+         sizeof(float) * 3 * a.max_nodes;
+}
+// Forces in LDS where two work-groups still share a CU (Kuhn meshes: 750 entries, 44 KB);
+// denser chunks add with atomics.  So do all penalty models but SIMP with an integer exponent:
+// with every model's code k_mf_gather spills at its register limit, and from 51x27x25 hexes on
+// it is the slower one (us an iteration, RAMP, 97x51x45: graded hexes 81 against 64 with
+// k_mf_apply, five tets 119 and 82; below, within 7 % either way).
+bool mf_gathers(const MfArgs& a) {
+  return a.inc && mf_gather_lds(a) <= 64 * 1024 && a.m.model == kPenaltySimp && a.m.pint > 0;
+}
+
 hipError_t launch_mf_apply(const MfArgs& a, hipStream_t s) {
-  const size_t lds = sizeof(double) * 6 * ((a.max_rows + 1) & ~1) + sizeof(float4) * a.max_nodes +
-                     sizeof(float) * 3 * a.max_nodes;
-  // forces in LDS where two work-groups still share a CU (Kuhn meshes: 750 entries, 44 KB);
-  // denser chunks add with atomics
-  const size_t gather = sizeof(double) * 3 * ((a.max_rows + 1) & ~1) + sizeof(float4) * (a.max_nodes + 3 * (size_t)a.max_list) +
-                        sizeof(float) * 3 * a.max_nodes;
-  if (a.inc && gather <= 64 * 1024) {
-    const bool ip = a.m.model == kPenaltySimp && a.m.pint > 0;
-    if (ip) k_mf_gather<512, true><<<a.nchunks, 512, gather, s>>>(a);
-    else k_mf_gather<512, false><<<a.nchunks, 512, gather, s>>>(a);
+  if (mf_gathers(a)) {
+    k_mf_gather<512><<<a.nchunks, 512, mf_gather_lds(a), s>>>(a);
     return hipGetLastError();
   }
+  const size_t lds = sizeof(double) * 6 * ((a.max_rows + 1) & ~1) + sizeof(float4) * a.max_nodes +
+                     sizeof(float) * 3 * a.max_nodes;
   k_mf_apply<256><<<a.nchunks, 256, lds, s>>>(a);
   return hipGetLastError();
 }

@@ -39,6 +39,8 @@ struct MfArgs {
   int max_list;         // entries of a chunk at most
 };
 hipError_t launch_mf_apply(const MfArgs& a, hipStream_t s);
+// whether it takes k_mf_gather, else k_mf_apply (atomics)
+bool mf_gathers(const MfArgs& a);
 
 // FP64 3x3 diagonal blocks of K(z) per node, inverted (constrained dofs -> identity).
 struct DiagArgs {

@@ -6,7 +6,7 @@ namespace pa {
 
 // slots of the device scalar array used by the PCG kernels
 enum ScalarSlot { kRZ = 0, kPQ = 1, kAlpha = 2, kBeta = 3, kRR = 4, kBB = 5, kDot0 = 6, kDot1 = 7,
-                  kEnergy = 8, kPScale = 9, kNumScal = 16 };
+                  kEnergy = 8, kPScale = 9, kRZ0 = 10, kRZ1 = 11, kNumScal = 16 };
 
 // partial arrays of the solver (kRedBlocks doubles each) in one device buffer
 enum PartialSlot { kPPQ = 0, kPRZ0 = 1, kPRZ1 = 2, kPRR = 3, kPBB = 4, kPDot = 5, kNumPartialSlots = 6 };
