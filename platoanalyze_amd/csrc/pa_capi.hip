@@ -336,7 +336,10 @@ static int mark_queued(pa_handle h) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   PA_HIP(hipStreamIsCapturing(h->stream, &st));
   if (st != hipStreamCaptureStatusNone) return PA_OK;  // queued when the graph is launched
-  if (!h->queued_event) PA_HIP(hipEventCreateWithFlags(&h->queued_event, hipEventDisableTiming));
+  // ordered on one device only, so without the system-scope fence, which took 3 us of the
+  // stream at each record (20x10x10 hexes, general lattice residual: 17 -> 21 us, now 17)
+  if (!h->queued_event)
+    PA_HIP(hipEventCreateWithFlags(&h->queued_event, hipEventDisableTiming | hipEventDisableSystemFence));
   PA_HIP(hipEventRecord(h->queued_event, h->stream));
   h->queued = true;
   return PA_OK;
