@@ -646,8 +646,31 @@ static int run_chunk(pa_handle h, int mode, const double* u, const double* z, do
 // kernels of the energy, p-norm and adjoint functions and a scatter, a weight and a row
 // pass of the residual.  128x64x64: residual 62.7 -> 36.4 us, compliance and gradient
 // 150 -> 49 us; 64x32x32: p-norm, its partials and the adjoint product 182 -> 93 us.
-// Taken at every size (20x10x10 is launch-bound either way).
 static bool box_tiles(pa_handle h) { return h->box_fast && h->box_res_kuhn; }
+
+// A power or a sine per tet (SIMP with a non-integer exponent, Heaviside; p-norms with a
+// non-integer p or, relaxed von Mises, q other than 1/2) sets the pace: a thread of a brick
+// evaluates six in turn and a tet's 1.95 times, a thread of a chunk one.  Small boxes, whose
+// few bricks leave the chip idle, therefore keep the chunk kernels.  Microseconds a call,
+// chunks / bricks, at 20x10x10, 48x24x24, 64x32x32 and 96x48x48 hexes:
+//   SIMP 2.5, C and dC/dz                 29/33, 33/36, 46/42, 94/76
+//   Heaviside, adjoint product            11/12, 12/15, 22/24, 58/54
+//   von Mises p = 6.5, q = 0.3, dF/du     24/37, 31/40, 54/67, 138/133
+static bool penalty_powers(const pa::Material& m) {
+  return m.model == pa::kPenaltyHeaviside || (m.model == pa::kPenaltySimp && m.pint == 0);
+}
+static bool pnorm_powers(const pa::Material& m, int measure, double pn, double q) {
+  return pn > 16.0 || pn != std::floor(pn) || (measure == 0 ? penalty_powers(m) : q != 0.5);
+}
+constexpr int kPowerTileNodes = 100000, kPowerEnergyTileNodes = 50000;
+static bool box_tiles_for(pa_handle h, bool powers, int nodes) { return box_tiles(h) && !(powers && h->nn <= nodes); }
+static bool energy_tiles(pa_handle h) {
+  return box_tiles_for(h, penalty_powers(h->material()), kPowerEnergyTileNodes);
+}
+static bool pnorm_tiles(pa_handle h, int measure, double pn, double q) {
+  return box_tiles_for(h, pnorm_powers(h->material(), measure, pn, q), kPowerTileNodes);
+}
+static bool adjoint_tiles(pa_handle h) { return box_tiles_for(h, penalty_powers(h->material()), kPowerTileNodes); }
 static pa::BoxTileArgs tile_args(pa_handle h, const double* u, const double* z) {
   pa::BoxTileArgs a{};
   a.node_of = h->box_node_of.p;
@@ -844,7 +867,7 @@ static int energy_value(pa_handle h, double* value, bool tiles) {
 int pa_sf_value(pa_handle h, const double* u, const double* z, double* value) {
   if (int rc = ready(h)) return rc;
   if (!u || !z || !value) return fail(PA_ERR_ARG, "pa_sf_value: null pointer");
-  if (box_tiles(h)) {
+  if (energy_tiles(h)) {
     PA_HIP(pa::launch_box_tile(pa::kTileEnergy, tile_args(h, u, z), h->stream));
     return energy_value(h, value, true);
   }
@@ -861,7 +884,7 @@ int pa_sf_gradient_u(pa_handle h, const double* u, const double* z, double* g) {
 
 // g = scale times the partial dC/dz, and C
 static int energy_gradient(pa_handle h, const double* u, const double* z, double* g, double* value, double scale) {
-  const bool tiles = box_tiles(h);
+  const bool tiles = energy_tiles(h);
   if (tiles) {
     pa::BoxTileArgs a = tile_args(h, u, z);
     a.out = g;
@@ -2640,7 +2663,7 @@ int pa_solution_deflated(pa_handle h, const double* z, double* u, double* vals, 
 // The p-norm's sum S (read: into host_scal, valid after a wait) and the factor of its gradients
 // into scal[kPScale]: the gradients need no wait for the value.
 static int pnorm_sum(pa_handle h, const double* u, const double* z, int measure, double pn, double q, bool read) {
-  const bool tiles = box_tiles(h);
+  const bool tiles = pnorm_tiles(h, measure, pn, q);
   if (tiles) {
     pa::BoxTileArgs a = tile_args(h, u, z);
     a.measure = measure;
@@ -2688,7 +2711,7 @@ int pa_stress_pnorm(pa_handle h, const double* u, const double* z, int measure, 
   if (int rc = pnorm_sum(h, u, z, measure, pn, q, value)) return rc;
   double* gu = dfdu ? dfdu : h->w_r.p;
   double* gz = dfdz ? dfdz : h->w_z.p;  // w_z holds >= num_nodes doubles
-  if (grad && box_tiles(h)) {
+  if (grad && pnorm_tiles(h, measure, pn, q)) {
     pa::BoxTileArgs a = tile_args(h, u, z);
     a.measure = measure;
     a.pn = pn;
@@ -2733,7 +2756,7 @@ int pa_stress_pnorm_gradient_x(pa_handle h, const double* u, const double* z, in
 int pa_dRdz_T_apply(pa_handle h, const double* u, const double* lambda, const double* z, double* out) {
   if (int rc = ready(h)) return rc;
   if (!u || !lambda || !z || !out) return fail(PA_ERR_ARG, "pa_dRdz_T_apply: null pointer");
-  if (box_tiles(h)) {
+  if (adjoint_tiles(h)) {
     pa::BoxTileArgs a = tile_args(h, u, z);
     a.u2 = lambda;
     a.out = out;
