@@ -17,6 +17,8 @@
 // -> 36 us a call, energy and gradient (chunk kernel) 149 -> 60 -> 49; p-norm adjoint
 // gradient, 64x32x32, 182 -> 124 -> 104 (93 since its factor is summed on the device).
 // Four waves a SIMD spill (residual 51 us, gradient 109).
+// kTileResidualW reads the tets' weights instead, where a power or a sine each would be
+// evaluated 1.95 times (128x64x64, Heaviside: 93 us with the pass that makes them, 119 without).
 #include "pa_boxtile.hpp"
 
 #include <cmath>
@@ -124,7 +126,8 @@ __device__ __forceinline__ double von_mises2(const double s[6]) {
 
 template <int MODE, bool SIMP>  // SIMP: powers by multiplication only (see launch_box_tile)
 __global__ __launch_bounds__(kT, 3) void k_box_tile(BoxTileArgs A) {
-  constexpr bool kRes = MODE == kTileResidual, kGradZ = MODE == kTileEnergyGradZ, kPnG = MODE == kTilePNormGrad;
+  constexpr bool kWgt = MODE == kTileResidualW;  // the tets' weights are given
+  constexpr bool kRes = MODE == kTileResidual || kWgt, kGradZ = MODE == kTileEnergyGradZ, kPnG = MODE == kTilePNormGrad;
   constexpr bool kAdj = MODE == kTileAdjZ, kPn = MODE == kTilePNorm || kPnG;
   constexpr bool kVec = kRes || kPnG, kScal = kGradZ || kPnG || kAdj;  // corner vectors, corner scalars
   constexpr bool kSum = MODE == kTileEnergy || kGradZ || MODE == kTilePNorm;
@@ -205,10 +208,12 @@ __global__ __launch_bounds__(kT, 3) void k_box_tile(BoxTileArgs A) {
       }
       return v;
     };
-    // its coefficients: cf of the corner vectors, cs of the corner scalars
+    // its coefficients: cf of the corner vectors, cs of the corner scalars (kWgt: rho is the weight)
     auto coefficients = [&](double rho, double v, double& cf, double& cs) {
       cf = cs = 0.0;
-      if constexpr (kRes) {
+      if constexpr (kWgt) {
+        cf = A.vol * rho;
+      } else if constexpr (kRes) {
         cf = A.vol * penalty_w_as<SIMP>(A.m, rho);
       } else if constexpr (kAdj) {
         cs = v * (0.25 * penalty_dw_as<SIMP>(A.m, rho) * A.vol);
@@ -262,9 +267,13 @@ __global__ __launch_bounds__(kT, 3) void k_box_tile(BoxTileArgs A) {
       if constexpr (kScal) tet_scalar<Q>(cs, S);
     };
     if constexpr (SIMP) {
+      const double* W = kWgt ? A.W + 6 * (gi + 1 + (A.nx + 1) * (gj + 1 + (size_t)(A.ny + 1) * (gk + 1))) : nullptr;
       each_tet<0>([&](auto q) {
-        double cf, cs;
-        coefficients(tet_rho<decltype(q)::value>(Z), measure(q), cf, cs);
+        constexpr int Q = decltype(q)::value;
+        double cf, cs, rho;
+        if constexpr (kWgt) rho = W[A.tperm[Q]];
+        else rho = tet_rho<Q>(Z);
+        coefficients(rho, measure(q), cf, cs);
         forces(q, cf, cs);
       });
     } else {
@@ -362,6 +371,7 @@ hipError_t launch_box_tile(int mode, const BoxTileArgs& a, hipStream_t s) {
     simp = simp && a.pn >= 1.0 && a.pn <= 16.0 && a.pn == std::floor(a.pn) && (a.measure == 0 || a.q == 0.5);
   switch (mode) {
     case kTileResidual: launch<kTileResidual>(simp, a, s); break;
+    case kTileResidualW: k_box_tile<kTileResidualW, true><<<a.bx * a.by * a.bz, kT, 0, s>>>(a); break;
     case kTileEnergy: launch<kTileEnergy>(simp, a, s); break;
     case kTileEnergyGradZ: launch<kTileEnergyGradZ>(simp, a, s); break;
     case kTilePNorm: launch<kTilePNorm>(simp, a, s); break;

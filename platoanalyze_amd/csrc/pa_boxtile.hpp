@@ -20,6 +20,8 @@ struct BoxTileArgs {
   double* partials;     // one per brick: energy or p-norm sum
   const int* lidx;      // per node: its entry in load_f, or -1 (kTileResidual; null: no load)
   const double* load_f;
+  const double* W;      // kTileResidualW: weights of the padded hexes, six a hex, path q's at tperm[q]
+  int tperm[6];
   double scale;         // factor of the energy gradient (1, or -1 for the total derivative)
   int measure;          // p-norm: 0 Voigt norm of the weighted stress, 1 relaxed von Mises
   double pn, q;
@@ -28,7 +30,7 @@ struct BoxTileArgs {
 };
 
 enum TileMode { kTileResidual = 0, kTileEnergy = 1, kTileEnergyGradZ = 2, kTilePNorm = 3, kTilePNormGrad = 4,
-                kTileAdjZ = 5 };
+                kTileAdjZ = 5, kTileResidualW = 6 };
 
 constexpr int kTileNodes = 4;  // a brick owns kTileNodes^3 lattice points
 inline int tile_bricks(int nodes) { return (nodes + kTileNodes - 1) / kTileNodes; }

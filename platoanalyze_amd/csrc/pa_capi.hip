@@ -671,6 +671,10 @@ static bool pnorm_tiles(pa_handle h, int measure, double pn, double q) {
   return box_tiles_for(h, pnorm_powers(h->material(), measure, pn, q), kPowerTileNodes);
 }
 static bool adjoint_tiles(pa_handle h) { return box_tiles_for(h, penalty_powers(h->material()), kPowerTileNodes); }
+// A residual's weights from a pass of their own, each evaluated once: Heaviside, 128x64x64,
+// 93 us against 119 with bricks that evaluate them (64x32x32, where launches count: 26).
+static bool residual_weights(pa_handle h) { return penalty_powers(h->material()) && h->nn > kPowerTileNodes; }
+
 static pa::BoxTileArgs tile_args(pa_handle h, const double* u, const double* z) {
   pa::BoxTileArgs a{};
   a.node_of = h->box_node_of.p;
@@ -700,7 +704,13 @@ static int residual(pa_handle h, const double* u, const double* z, double* R, bo
       a.out = R;
       a.lidx = sub ? h->box_lidx.p : nullptr;
       a.load_f = h->load_f.p;
-      PA_HIP(pa::launch_box_tile(pa::kTileResidual, a, h->stream));
+      if (residual_weights(h)) {
+        const pa::BoxArgs b = box_args(h, nullptr, z, nullptr, nullptr);
+        box_weights(h, b, b.W);
+        a.W = b.W;
+        std::copy(h->box_tperm, h->box_tperm + 6, a.tperm);
+      }
+      PA_HIP(pa::launch_box_tile(a.W ? pa::kTileResidualW : pa::kTileResidual, a, h->stream));
       return PA_OK;
     }
     const pa::BoxArgs a = box_args(h, u, z, nullptr, R);
@@ -715,7 +725,7 @@ static int residual(pa_handle h, const double* u, const double* z, double* R, bo
 }
 
 // whether it goes through the handle's lattice copies and weights
-static bool residual_scratch(pa_handle h) { return h->box_fast && h->box_res && !box_tiles(h); }
+static bool residual_scratch(pa_handle h) { return h->box_fast && h->box_res && (!box_tiles(h) || residual_weights(h)); }
 
 static int sub_load(pa_handle h, double* R, double s) {
   if (h->nload == 0) return PA_OK;

@@ -62,3 +62,13 @@ def test_gpu_box_powers_functions(monkeypatch, dims, penalty):
         assert abs(pa.value(u, z) - pb.value(u, z)) <= RTOL * pb.value(u, z)
         _close(pa.gradient_u(u, z), pb.gradient_u(u, z), f"{measure} dF/du")
         _close(pa.gradient_z(u, z), pb.gradient_z(u, z), f"{measure} dF/dz")
+
+
+@pytest.mark.parametrize("dims", SIZES[2:])
+@pytest.mark.parametrize("penalty", PENALTIES)
+def test_gpu_box_powers_residual(monkeypatch, dims, penalty):
+    from platoanalyze_amd.elliptic import PhysicsScalarFunction, VectorFunction
+
+    a, b, u, _, z = _models(monkeypatch, dims, penalty)
+    _close(VectorFunction(a).value(u, z), VectorFunction(b).value(u, z), "residual")
+    _close(PhysicsScalarFunction(a).gradient_u(u, z), PhysicsScalarFunction(b).gradient_u(u, z), "K u")
