@@ -674,6 +674,13 @@ static bool adjoint_tiles(pa_handle h) { return box_tiles_for(h, penalty_powers(
 // A residual's weights from a pass of their own, each evaluated once: Heaviside, 128x64x64,
 // 93 us against 119 with bricks that evaluate them (64x32x32, where launches count: 26).
 static bool residual_weights(pa_handle h) { return penalty_powers(h->material()) && h->nn > kPowerTileNodes; }
+// The Jacobian's row tiles evaluate up to 2.6 weights a tet.  Between launch-bound boxes and
+// those whose lattice arrays leave the last-level cache the general kernels, which evaluate
+// each once, are faster (Heaviside, us, row tiles / general: 64x32x32 36/41, 128x64x64 226/192,
+// 192x96x96 653/571, 256x128x128 1763/1842; SIMP 2.5 30/38, 193/180, 570/532, 1588/1768).
+static bool jac_tiles(pa_handle h) {
+  return h->box_jac.n && !(penalty_powers(h->material()) && h->nn > kPowerTileNodes && !h->box_ahead);
+}
 
 static pa::BoxTileArgs tile_args(pa_handle h, const double* u, const double* z) {
   pa::BoxTileArgs a{};
@@ -745,7 +752,7 @@ int pa_vf_gradient_u(pa_handle h, const double* u, const double* z, double* vals
   if (int rc = ready(h)) return rc;
   if (!z || !vals || (R && !u)) return fail(PA_ERR_ARG, "pa_vf_gradient_u: null pointer");
   if (int rc = assemble_jacobian(h, u, z, vals, R)) return rc;
-  return h->box_fast && !h->box_jac.n ? mark_queued(h) : PA_OK;  // the lattice copies and weights
+  return h->box_fast && !jac_tiles(h) ? mark_queued(h) : PA_OK;  // the lattice copies and weights
 }
 
 int pa_vf_gradient_z(pa_handle h, const double* u, const double* z, double* vals_t) {
@@ -1810,7 +1817,7 @@ static void box_weights(pa_handle h, const pa::BoxArgs& a, T* W) {
 
 // K (and R = K u - f) on the lattice: element weights, then the rows.
 static int box_jacobian(pa_handle h, const double* u, const double* z, double* vals, double* R) {
-  if (h->box_jac.n) {
+  if (jac_tiles(h)) {
     pa::BoxJacArgs j{};
     j.tiles = h->box_jac.p;
     j.ntiles = (int)h->box_jac.n;

@@ -72,3 +72,15 @@ def test_gpu_box_powers_residual(monkeypatch, dims, penalty):
     a, b, u, _, z = _models(monkeypatch, dims, penalty)
     _close(VectorFunction(a).value(u, z), VectorFunction(b).value(u, z), "residual")
     _close(PhysicsScalarFunction(a).gradient_u(u, z), PhysicsScalarFunction(b).gradient_u(u, z), "K u")
+
+
+@pytest.mark.parametrize("dims", SIZES[2:])
+@pytest.mark.parametrize("penalty", PENALTIES)
+def test_gpu_box_powers_jacobian(monkeypatch, dims, penalty):
+    from platoanalyze_amd.elliptic import VectorFunction
+
+    a, b, u, _, z = _models(monkeypatch, dims, penalty)
+    Ra, Rb = torch.full_like(u, np.nan), torch.empty_like(u)
+    _close(VectorFunction(a).gradient_u(u, z, residual_out=Ra).entries,
+           VectorFunction(b).gradient_u(u, z, residual_out=Rb).entries, "K")
+    _close(Ra, Rb, "R")
