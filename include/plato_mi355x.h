@@ -187,10 +187,10 @@ int pa_solve(pa_handle h, const double* values, double* x, const double* b,
 /* No counterpart in the reference.  pa_solve for callers that cannot allocate device
  * memory during the call (code under stream capture, tight serving loops, harnesses that
  * forbid hipMalloc): the same block-Jacobi PCG, same arguments and results, with its
- * workspace (five node vectors, the block-diagonal inverse, reduction partials and
+ * workspace (four or five node vectors, the block-diagonal inverse, reduction partials and
  * scalars) in a fixed device array of the library instead of handle memory allocated on
  * first use.  Meshes of at most PA_NOALLOC_MAX_NODES nodes (more: PA_ERR_UNSUPPORTED);
- * the array (24 * PA_NOALLOC_MAX_NODES doubles plus 6160, about 25 MB) is held on every
+ * the array (21 * PA_NOALLOC_MAX_NODES doubles plus 6160, about 22 MB) is held on every
  * GPU the library runs on until the process ends.  Every call on one GPU shares that
  * GPU's array: calls that overlap on one GPU (other streams, other threads, other
  * handles) race and must be serialised by the caller. */

@@ -944,7 +944,6 @@ static int ensure_solver_ws(pa_handle h) {
     PA_HIP(h->w_r.alloc(ndof));
     PA_HIP(h->w_z.alloc(ndof));
     PA_HIP(h->w_p.alloc(ndof));
-    PA_HIP(h->w_p2.alloc(ndof));
     PA_HIP(h->w_q.alloc(ndof));
     PA_HIP(h->w_dinv.alloc(9 * (size_t)h->nn));
   }
@@ -957,9 +956,9 @@ static int read_scal(pa_handle h) {
   return PA_OK;
 }
 
-// Device workspace of the block-Jacobi PCG: five node vectors (3N doubles each), the 3x3
-// block-diagonal inverse (9N), kNumPartialSlots x kRedBlocks reduction partials and
-// kNumScal scalars.  Every entry is written before it is read.
+// Device workspace of the block-Jacobi PCG: four node vectors (3N doubles each) and, up to
+// kFusedDirNodes nodes, a fifth (p2), the 3x3 block-diagonal inverse (9N), kNumPartialSlots x
+// kRedBlocks reduction partials and kNumScal scalars.  Every entry is written before it is read.
 struct PcgWork {
   double *r, *z, *p, *p2, *q, *dinv, *partials, *scal;
 };
@@ -1002,6 +1001,15 @@ static int deflate_apply(pa_handle h, const Deflation& D, const double* X, const
 // gathered vector costs more than the launch (40.1 us against 38.9), at 545025 198 us
 // against 180.
 constexpr int kFusedDirNodes = 100000;
+
+// handle memory of pcg_block_jacobi (p2: the second direction of k_pcg_dir_spmv)
+static int pcg_workspace(pa_handle h, PcgWork& W) {
+  if (int rc = ensure_solver_ws(h)) return rc;
+  const size_t ndof = 3 * (size_t)h->nn;
+  if (h->nn <= kFusedDirNodes && h->w_p2.n != ndof) PA_HIP(h->w_p2.alloc(ndof));
+  W = PcgWork{h->w_r.p, h->w_z.p, h->w_p.p, h->w_p2.p, h->w_q.p, h->w_dinv.p, h->partials.p, h->scal.p};
+  return PA_OK;
+}
 
 // Jacobi(3x3 block)-PCG in FP64 on the handle's graph, on the workspace W; with a
 // deflation space D, deflated PCG (the start corrected by V E^-1 V^T r, every direction
@@ -1091,9 +1099,9 @@ int pa_solve(pa_handle h, const double* vals, double* x, const double* b, const 
   if (!vals || !x || !b) return fail(PA_ERR_ARG, "pa_solve: null pointer");
   pa_solver_opts opts;
   if (int rc = solve_opts(o, opts, "pa_solve")) return rc;
-  if (int rc = ensure_solver_ws(h)) return rc;
-  return pcg_block_jacobi(h, vals, x, b, opts, st,
-                          PcgWork{h->w_r.p, h->w_z.p, h->w_p.p, h->w_p2.p, h->w_q.p, h->w_dinv.p, h->partials.p, h->scal.p});
+  PcgWork work;
+  if (int rc = pcg_workspace(h, work)) return rc;
+  return pcg_block_jacobi(h, vals, x, b, opts, st, work);
 }
 
 // ------------------------------------------------------------ solve without allocation
@@ -1103,7 +1111,8 @@ int pa_solve(pa_handle h, const double* vals, double* x, const double* b, const 
 // each GPU's copy comes from hipGetSymbolAddress, taken once per device with that device
 // current, and only that address is handed to kernels.
 constexpr size_t kNoAllocPartials = (size_t)pa::kNumPartialSlots * pa::kRedBlocks;
-constexpr size_t kNoAllocDoubles = 24 * (size_t)PA_NOALLOC_MAX_NODES + kNoAllocPartials + pa::kNumScal;
+constexpr size_t kNoAllocDoubles = 21 * (size_t)PA_NOALLOC_MAX_NODES + kNoAllocPartials + pa::kNumScal;
+static_assert(24 * kFusedDirNodes <= 21 * PA_NOALLOC_MAX_NODES, "a second direction fits where it is used");
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
 constexpr int kNoAllocMaxDevices = 64;
@@ -1137,8 +1146,9 @@ int pa_solve_noalloc(pa_handle h, const double* vals, double* x, const double* b
   double* ws = nullptr;
   if (int rc = noalloc_scratch(&ws)) return rc;
   const size_t nd = 3 * (size_t)h->nn;
-  PcgWork W{ws, ws + nd, ws + 2 * nd, ws + 3 * nd, ws + 4 * nd, ws + 5 * nd, ws + 5 * nd + 9 * (size_t)h->nn, nullptr};
+  PcgWork W{ws, ws + nd, ws + 2 * nd, nullptr, ws + 3 * nd, ws + 4 * nd, ws + 4 * nd + 9 * (size_t)h->nn, nullptr};
   W.scal = W.partials + kNoAllocPartials;
+  W.p2 = W.scal + pa::kNumScal;  // up to kFusedDirNodes nodes
   return pcg_block_jacobi(h, vals, x, b, opts, st, W);
 }
 
@@ -1980,7 +1990,7 @@ static int mg_build(pa_handle h) {
   if (h->mg.size() < 2) return fail(PA_ERR_UNSUPPORTED, "multigrid: the box has no coarser level");
   const size_t nc = 3 * (size_t)h->mg.back()->nn;
   PA_HIP(h->mg_Ainv.alloc(nc * nc));
-  PA_HIP(h->mg_T.alloc(nc * nc));
+  PA_HIP(h->mg_T.alloc(pa::mg_dense_scratch(h->mg.back()->nn)));
   PA_HIP(h->mg_lz.alloc((h->mg.size() - 1) * (3 * (size_t)pa::kLzBlocks + 2 * pa::kLzSteps) + 1));
   return PA_OK;
 }
@@ -2592,7 +2602,8 @@ int pa_solution_deflated(pa_handle h, const double* z, double* u, double* vals, 
   if (int rc = pa_apply_constraints(h, vals, rhs, 1.0)) return rc;
   const int nbc = (int)h->bc_dofs.size();
   if (opts.use_x0 && nbc) pa::k_bc_set<<<grid_for(nbc), 256, 0, s>>>(u, h->bc_d.p, h->bc_v.p, nbc, 1.0);
-  PcgWork work{h->w_r.p, h->w_z.p, h->w_p.p, h->w_p2.p, h->w_q.p, h->w_dinv.p, h->partials.p, h->scal.p};
+  PcgWork work;
+  if (int rc = pcg_workspace(h, work)) return rc;
   if (k == 0) return pcg_block_jacobi(h, vals, u, rhs, opts, st, work);
   // V = W with the constrained dofs zeroed, A V, E = V^T A V
   const size_t kn = (size_t)k * ndof;

@@ -609,6 +609,10 @@ hipError_t launch_lz_dir(const LzArgs& a, int step, hipStream_t s) {
   k_lz_dir<<<a.blocks, kT, 0, s>>>(a, step);
   return hipGetLastError();
 }
+size_t mg_dense_scratch(int nn) {
+  const size_t n = 3 * (size_t)nn;
+  return n <= 32 * kGjTile ? 0 : n * n;
+}
 hipError_t launch_mg_dense_inverse(const double* vals, const int32_t* rowmap, const int32_t* col, int nn, double* A,
                                    double* T, double* flag, hipStream_t s) {
   const int n = 3 * nn;

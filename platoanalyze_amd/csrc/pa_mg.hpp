@@ -115,8 +115,10 @@ hipError_t launch_lz_update(const LzArgs& a, int step, hipStream_t s);
 hipError_t launch_lz_dir(const LzArgs& a, int step, hipStream_t s);
 
 // Inverse of the coarsest level's matrix (symmetric positive definite, 3 nn square) into A,
-// by Gauss-Jordan elimination on the device; T is scratch of the same size.  *flag (device)
-// becomes 1 when a pivot is not positive, else 0.
+// by Gauss-Jordan elimination on the device; T is scratch of mg_dense_scratch(nn) doubles (none
+// where one work-group holds the matrix in registers).  *flag (device) becomes 1 when a pivot
+// is not positive, else 0.
+size_t mg_dense_scratch(int nn);
 hipError_t launch_mg_dense_inverse(const double* vals, const int32_t* rowmap, const int32_t* col, int nn, double* A,
                                    double* T, double* flag, hipStream_t s);
 
