@@ -369,8 +369,9 @@ __global__ __launch_bounds__(kT) void k_bc_lift(const double* vals, const int* r
 // applyBlockConstraints first loop, matrix part: BC row -> unit diagonal, zero
 // elsewhere; the symmetric (col,row) entries zeroed too.  16 lanes per BC dof, a lane per
 // block of its row, the partner row searched once for all components (its column loads are
-// independent; a caller's graph may repeat a column, so every match is cleared): a thread per dof walked ~15 blocks x 3 components x ~15 dependent loads
-// and took 68-96 us whatever the size (20x10x10: 84 us).
+// independent; a caller's graph may repeat a column, so every match is cleared): a thread
+// per dof walked ~15 blocks x 3 components x ~15 dependent loads and took 68-96 us whatever
+// the size (20x10x10: 84 us).
 __global__ __launch_bounds__(kT) void k_bc_zero(double* vals, const int* rowmap, const int* col,
                                                 const int* dofs, int nbc) {
   const int lane = threadIdx.x % kLanesPerRow;
