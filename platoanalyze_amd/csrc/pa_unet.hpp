@@ -45,10 +45,11 @@ struct ConvArgs {
   int accumulate;     // Yf += result instead of =
   const bf16_t* gate; // multiply the result by (gate > 0) (ReLU derivative), same shape as Yf
   int ldg, gcol;
-  // Split reduction for grids too small to fill the GPU: work-group slice z sums its range
-  // of the 27*cin reduction into part[z][M][cout] (FP32, M = batch x output voxels) and a
-  // second kernel adds the slices in slice order and applies the epilogue.  part null:
-  // one pass.  part_cap: floats available at part.
+  // Split reduction for grids too small to fill the GPU: the 27*cin reduction is cut into
+  // slices, summed apart and added in slice order.  k_conv_tile's waves exchange them in LDS;
+  // where no tile fits there, work-group slice z of k_conv writes part[z][M][cout] (FP32, M =
+  // batch x output voxels) and a second kernel adds them and applies the epilogue.  part null:
+  // one pass.  part_cap: floats available at part (it bounds the slices of both).
   float* part;
   size_t part_cap;
 };
