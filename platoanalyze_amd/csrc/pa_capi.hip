@@ -2117,8 +2117,9 @@ static int mg_vcycle_lattice(pa_handle h, const double* r, double* x, const doub
 // full-weighting restriction, trilinear prolongation, dense solve on the last level.
 // `started`: the caller has already set x = d = D^-1 r / theta (fused into its
 // restriction).  Where the level has an assembled operator the smoothing steps are
-// fused with the operator product (6 launches per level); level 0 of the mixed solve
-// applies the FP32 matrix-free operator and runs the steps as separate kernels.
+// fused with the operator product (6 launches per level).  Level 0 of the mixed solve applies
+// the FP32 matrix-free operator: mg_vcycle_lattice on Kuhn lattices with one smoothing step a
+// side, else the steps as separate kernels.
 static int mg_vcycle(pa_handle h, size_t l, const double* r, double* x, const double* vals0, bool mixed,
                      bool started) {
   hipStream_t s = h->stream;
