@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kT, 3) void k_box_tile(BoxTileArgs A) {
   if constexpr (kSum) {  // every hex is summed by the brick that owns its lower corner
     const double own = hex && hx > 0 && hy > 0 && hz > 0 ? sum : 0.0;
     const double r = block_reduce_all<kT>(own, sh);
-    if (t == 0) A.partials[brick] = r;
+    if (t == 0 && A.partials) A.partials[brick] = r;
   }
 }
 

@@ -17,7 +17,7 @@ struct BoxTileArgs {
   const double* z;
   double* out;          // 3 per node (residual, p-norm dF/du) or 1 (energy gradient, adjoint)
   double* out2;         // 1 per node (p-norm dF/dz)
-  double* partials;     // one per brick: energy or p-norm sum
+  double* partials;     // one per brick: energy or p-norm sum (null: none)
   const int* lidx;      // per node: its entry in load_f, or -1 (kTileResidual; null: no load)
   const double* load_f;
   const double* W;      // kTileResidualW: weights of the padded hexes, six a hex, path q's at tperm[q]

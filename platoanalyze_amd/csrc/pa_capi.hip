@@ -899,13 +899,15 @@ int pa_sf_gradient_u(pa_handle h, const double* u, const double* z, double* g) {
   return residual_scratch(h) ? mark_queued(h) : PA_OK;
 }
 
-// g = scale times the partial dC/dz, and C
+// g = scale times the partial dC/dz, and C (without it nothing of the handle's is written, so
+// that no later call has to wait)
 static int energy_gradient(pa_handle h, const double* u, const double* z, double* g, double* value, double scale) {
   const bool tiles = energy_tiles(h);
   if (tiles) {
     pa::BoxTileArgs a = tile_args(h, u, z);
     a.out = g;
     a.scale = scale;
+    if (!value) a.partials = nullptr;
     PA_HIP(pa::launch_box_tile(pa::kTileEnergyGradZ, a, h->stream));
   } else {
     pa::ChunkArgs a = h->chunk_args();
@@ -913,9 +915,10 @@ static int energy_gradient(pa_handle h, const double* u, const double* z, double
     a.z = z;
     a.out_vec = g;
     a.scale = scale;
+    if (!value) a.partials = nullptr;
     PA_HIP(pa::launch_chunk(h->code_bits, pa::kModeEnergyGradZ, a, h->stream));
   }
-  return value ? energy_value(h, value, tiles) : mark_queued(h);  // its partials
+  return value ? energy_value(h, value, tiles) : PA_OK;
 }
 
 int pa_sf_gradient_z(pa_handle h, const double* u, const double* z, double* g, double* value) {

@@ -472,7 +472,7 @@ __global__ __launch_bounds__(NT) void k_chunk(ChunkArgs A) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && A.partials) {
       double t = 0.0;
       for (int q = 0; q < NT / 64; ++q) t += wsum[q];
       A.partials[c] = t;

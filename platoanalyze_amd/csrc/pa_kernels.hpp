@@ -156,7 +156,7 @@ struct ChunkArgs {
   double* out_vals;   // Jacobian values (9/block) or dR/dz (3/block)
   double* out_vec;    // residual (3/row) or nodal gradient (1/row)
   double* out_vec2;   // p-norm dF/dz partial (1/row)
-  double* partials;   // per-chunk partial sums (energy)
+  double* partials;   // per-chunk partial sums (energy; null: none)
   // traction load of the chunk's rows, subtracted from the residual (R = K u - f)
   const int32_t* load_offs;  // [nchunks+1]
   const int32_t* load_row;   // row index relative to the chunk's first row
