@@ -15,7 +15,7 @@
 // corners at a time.  128x64x64 hexes, one thread per row with lattice copies and a weight
 // array -> bricks with all corners and every penalty model's code -> this: residual 62 -> 48.5
 // -> 36 us a call, energy and gradient (chunk kernel) 149 -> 60 -> 49; p-norm adjoint
-// gradient, 64x32x32, 182 -> 124 -> 104 (89 since its factor is summed on the device).
+// gradient, 64x32x32, 182 -> 124 -> 104 (89 to 92 since its factor is summed on the device).
 // Four waves a SIMD spill (residual 51 us, gradient 109).
 // kTileResidualW reads the tets' weights instead, where a power or a sine each would be
 // evaluated 1.95 times (128x64x64, Heaviside: 93 us with the pass that makes them, 119 without).

@@ -645,7 +645,7 @@ static int run_chunk(pa_handle h, int mode, const double* u, const double* z, do
 // Brick kernels (pa_boxtile.hip).  They replace, on Kuhn-split uniform boxes, the chunk
 // kernels of the energy, p-norm and adjoint functions and a scatter, a weight and a row
 // pass of the residual.  128x64x64: residual 62.7 -> 36.4 us, compliance and gradient
-// 150 -> 49 us; 64x32x32: p-norm, its partials and the adjoint product 182 -> 89 us.
+// 150 -> 49 us; 64x32x32: p-norm, its partials and the adjoint product 182 -> 89 to 92 us.
 static bool box_tiles(pa_handle h) { return h->box_fast && h->box_res_kuhn; }
 
 // A power or a sine per tet (SIMP with a non-integer exponent, Heaviside; p-norms with a
